@@ -88,6 +88,20 @@ def test_elementwise_ops(res):
         assert np.array_equal(do.numpy(), want)
 
 
+@pytest.mark.parametrize("w,h", [(1, 1), (3, 65), (15, 4), (511, 5), (512, 4), (513, 7), (1100, 3), (2, 1030),
+                                 (1, 2049)])
+def test_dot_compat_chunk_edges(res, w, h):
+    """The strided dot around its chunk of 512 products a part, 16 at a time,
+    and its stage of 1024 parts: bit-identical to the sequential sum."""
+    print("case dot compat", w, h, flush=True)
+    rng = np.random.default_rng(w * 10007 + h)
+    a = rng.standard_normal((h, w)).astype(np.float32)
+    b = rng.standard_normal((h, w)).astype(np.float32)
+    da, db, r = _dev(a), _dev(b), C.c_float()
+    uir.check(uir.load().uir_op_dot_compat(da.ptr, db.ptr, w, h, C.byref(r), None))
+    assert r.value == O.dot_compat(a, b)
+
+
 def test_reductions_and_stencils(res):
     rng = np.random.default_rng(1)
     a = rng.standard_normal((40, 48)).astype(np.float32)
