@@ -59,6 +59,27 @@ def test_bp_matches_oracle(res, n, d, a, step):
     assert err <= TOL, (err, np.abs(got - ref).max())
 
 
+@pytest.mark.parametrize("n,d,a,axis", [
+    (1, 1, 1, -1.0), (3, 5, 2, -1.0),
+    (63, 90, 7, -1.0), (65, 65, 9, -1.0),       # no clamp; detector as wide as the image: clamped corners
+    (511, 723, 17, -1.0), (513, 726, 15, -1.0),  # one and two pixels a thread, odd last rows, angles not in eights
+    (512, 725, 8, 355.25),                       # off-centre axis: the clamp window shrinks
+    (64, 91, 24, 0.2), (64, 91, 24, 95.0),       # no active detector: the clamp's two edges cross
+])
+def test_bp_bit_exact(res, n, d, a, axis):
+    """The BP runs the reference's operations in its order
+    (projector-parallel-joseph.cl:196-216): equal to the oracle bit for bit."""
+    print("case bp bit-exact", n, d, a, axis, flush=True)
+    step = np.float32(np.pi / a)
+    g = O.Geometry(n, d, a, step, axis=axis)
+    sino = np.random.default_rng(n + a).standard_normal((a, d)).astype(np.float32)
+    p = _projector(n, d, a, step, False, axis_position=axis).setup(res)
+    ds, out = uir.DeviceArray.from_numpy(sino), uir.DeviceArray((n, n))
+    assert p.requisition(ds) == (n, n)
+    p.process(ds, out)
+    assert np.array_equal(out.numpy(), O.bp(g, sino))
+
+
 def test_luts_and_runs_match_oracle(res):
     a, step = 720, np.float32(np.pi / 720)
     g = O.Geometry(1448, 1448, a, step)

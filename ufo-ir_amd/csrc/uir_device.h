@@ -54,11 +54,6 @@ int uirk_fp_ref_split(const float *vol, const float *r_sino, float *w_sino, cons
                       const float *sin_lut, const float *cos_lut, int n, int n_dets, float axis,
                       float corr, int ang0, int n_ang, int dir, void *stream);
 
-/* Reference-compatible BP (projector-parallel-joseph.cl:158-218) over a list of
- * subsets (runs), one per-run accumulation each: w = r + relax * sum_run.
- * pix_w == NULL: accumulate mode (r_vol may equal w_vol).
- * pix_w != NULL: SIRT mode, tmp = sum_runs(relax * S_run) (from 0), then
- * w = tmp * pix_w + r (ufo-ir-sirt-task.c:208-212); posc clamps the result. */
 /* The coordinate at the start of every 64-sample block of every ray of
  * angles [0, n_angles) ([angle][detector][block], ceil(n / 64) blocks), taken
  * by the reference's sequential float walk; inactive rays get 0. */
@@ -75,6 +70,11 @@ int uirk_fp_ref_seg(const float *vol, const float *r_sino, float *w_sino, const 
 int uirk_bp_ref_angle(const float *r_vol, float *w_vol, const float *sino, const float *sin_lut,
                       const float *cos_lut, int n, int n_dets, float axis, float relax, int ang, void *stream);
 
+/* Reference-compatible BP (projector-parallel-joseph.cl:158-218) over a list of
+ * subsets (runs), one per-run accumulation each: w = r + relax * sum_run.
+ * pix_w == NULL: accumulate mode (r_vol may equal w_vol).
+ * pix_w != NULL: SIRT mode, tmp = sum_runs(relax * S_run) (from 0), then
+ * w = tmp * pix_w + r (ufo-ir-sirt-task.c:208-212); posc clamps the result. */
 int uirk_bp_ref(const float *r_vol, float *w_vol, const float *sino, int n_angles,
                 const float *sin_lut, const float *cos_lut, int n, int n_dets, float axis,
                 float relax, const uirk_runs *runs, const float *pix_w, int posc, void *stream);
@@ -155,7 +155,7 @@ typedef struct {
     const void *b;       /* FP input sinogram (r_sinogram / measured data) */
     void *r;             /* FP output sinogram (may equal b) */
     const float *ray_w;  /* FP: multiply the result by ray_w (NULL: none) */
-    const float *pix_w;  /* ref BP: SIRT pixel weights (NULL: accumulate form) */
+    const float *pix_w;  /* line BP: pixel weights (NULL: none) */
     const float *trig;   /* per angle (sin, cos) interleaved, FP32 */
     int32_t n, n_dets, n_angles, posc;
     float axis, corr, relax, pix_scale;
@@ -224,7 +224,7 @@ typedef struct {
 /* Footprint width limit of a tile's FP. */
 #define UIRK_TILE_FP_WMAX(t) ((t).fp_single ? UIRK_FP_WMAX_SINGLE : UIRK_FP_WMAX)
 
-/* mode: 0 = reference-compatible FP32 arithmetic, 1 = fast path (FP32 math on
+/* mode: 0 = reference-compatible FP32 arithmetic (FP only), 1 = fast path (FP32 math on
  * FP32 / FP16 / BF16 storage), 3 = (BP only) the fast path over slice pairs
  * (items with pair set cover slices slice and slice + 1 of one geometry, with
  * the same results as mode 1; d_slices required), 4 = (BP only) mode 2 over

@@ -1,18 +1,19 @@
 // uir_fast.hip -- table-driven, LDS-staged Joseph projector pair for gfx950.
 //
-// One kernel family serves two paths:
-//   REF  = true : the reference's FP32 arithmetic operation for operation
-//                 (exact incremental float ray stepping from the double start
-//                 coordinate, 64-sample blocked sums, per-run BP sums, clamped
-//                 detector coordinate), bit-identical to the one-thread-per-ray
-//                 restatement of projector-parallel-joseph.cl.
-//   REF  = false: the batched fast path.  FP32 interpolation and accumulation
-//                 on FP32 / FP16 / BF16 storage, exact (double-anchored) ray
-//                 coordinates, fused SIRT epilogues.  Its FP is k_fp_pairs
-//                 (staged (e, d) pairs, one floor-convert and one FMA per
-//                 sample) or, for geometries whose angle blocks need windows
-//                 wider than the pairs' (sparse angles on large images),
-//                 k_fp_tab<..., false, ...> (single staged values, fract).
+// Two paths:
+//   reference-compatible FP (k_fp_tab with REF): the reference's FP32
+//                 arithmetic operation for operation (exact incremental float
+//                 ray stepping from the double start coordinate, 64-sample
+//                 blocked sums), bit-identical to the one-thread-per-ray
+//                 restatement of projector-parallel-joseph.cl.  Its BP is
+//                 k_bp_gather in uir_kernels.hip.
+//   fast path:    FP32 interpolation and accumulation on FP32 / FP16 / BF16
+//                 storage, exact (double-anchored) ray coordinates, fused SIRT
+//                 epilogues.  Its FP is k_fp_pairs (staged (e, d) pairs, one
+//                 float add for the index and one FMA per sample) or, for
+//                 geometries whose angle blocks need windows wider than the
+//                 pairs' (sparse angles on large images), k_fp_tab without REF
+//                 (single staged values, fract); its BP is k_bp_tab.
 // Work is described by tables (uirk_fp_item / uirk_bp_item) over any number
 // of slices of any geometry; the kernels stride over the table (launched with
 // one workgroup per item, so that the hardware's dispatch balances the items'
@@ -901,38 +902,37 @@ __global__ __launch_bounds__(256, APT == 8 ? 4 : 6) void k_fp_pairs(const uirk_s
 // Backprojection
 // ------------------------------------------------------------------------
 // A workgroup backprojects a tile of 64 x 4 ROWS pixels (one column per lane,
-// rows wave + 4 q), NA angles at a time staged in LDS.  The window and, on the
-// fast path, the sample coordinates belong to the 64 x 64 super-tile holding
-// the tile, and each pixel sums its angles in order, so the result of a pixel
+// rows wave + 4 q), NA angles at a time staged in LDS.  The window and the
+// sample coordinates belong to the 64 x 64 super-tile holding the tile, and each
+// pixel sums its angles in order, so the result of a pixel
 // does not depend on ROWS, NA or slice pairing.
-// LINE (fast path only): the line model.  Bins outside the detector read 0
+// LINE: the line model.  Bins outside the detector read 0
 // (every ray is active, no clamp), bins are staged as single values (a
 // sample reads two adjacent words in one instruction), and a sample weighs
 // them by the chord lengths of the pixel on the two rays,
 // w0 = clamp(bp_b0 - bp_k (f - 1/2), 0, 1/M), w1 = clamp(bp_b1 + bp_k (f - 1/2),
 // 0, 1/M), f the fraction of the detector coordinate; pix_w, when given,
 // multiplies the update (the model's pixel weights are not uniform).
-// PAIR (fast path only): an item with item.pair set also backprojects slice
+// PAIR: an item with item.pair set also backprojects slice
 // item.slice + 1 of the same geometry; both slices' (e, d) pairs share a
 // 16-byte entry, so a pixel-angle's coordinate, address and one LDS read
 // serve both (the same operations per slice as alone).  With LINE the staged
 // bin holds both slices' values (t, t'), and the chord weights are shared.
-template <typename T, typename TI, bool REF, int NA, int ROWS, bool LINE, bool PAIR>
-__global__ __launch_bounds__(256, REF ? 1 : (LINE ? 4 : (PAIR ? (NA == 32 ? 3 : 4) : 6))) void k_bp_tab(
+template <typename T, typename TI, int NA, int ROWS, bool LINE, bool PAIR>
+__global__ __launch_bounds__(256, LINE ? 4 : (PAIR ? (NA == 32 ? 3 : 4) : 6)) void k_bp_tab(
     const uirk_slice *__restrict__ slices, uirk_slice one, const uirk_bp_item *__restrict__ items, int n_items,
     uirk_xcd_part part, int *__restrict__ err)
 {
-    static_assert(!PAIR || !REF, "slice pairs: the fast path only");
     using E = typename fp_entry<PAIR>::type;
-    // reference-compatible path and line model: plain staged bins (line pairs:
-    // both slices' values); fast path: (e, d) pairs
-    __shared__ float lds[(REF || (LINE && !PAIR)) ? NA * kBpWb : 1];
+    // line model: plain staged bins (line pairs: both slices' values); joseph:
+    // (e, d) pairs
+    __shared__ float lds[(LINE && !PAIR) ? NA * kBpWb : 1];
     __shared__ float2 ldl[(LINE && PAIR) ? NA * kBpWb : 1];
-    __shared__ E ldp[(REF || LINE) ? 1 : NA * kBpWb];
+    __shared__ E ldp[LINE ? 1 : NA * kBpWb];
     __shared__ int s_umin[NA];
     __shared__ float s_trig[2 * NA];
     __shared__ float4 s_line[LINE ? NA : 1];
-    __shared__ float s_base[REF ? 1 : NA]; // fast path: window coordinate at the super-tile's corner
+    __shared__ float s_base[NA]; // window coordinate at the super-tile's corner
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const ItemRange range = item_range(part, n_items);
@@ -946,7 +946,6 @@ __global__ __launch_bounds__(256, REF ? 1 : (LINE ? 4 : (PAIR ? (NA == 32 ? 3 : 
         const T *sino = uniform((const T *)S->b);
         const T *sino2 = PAIR ? uniform((const T *)S2->b) : sino;
         const float *trig = uniform(S->trig);
-        const float relax = S->relax;
         const int n_runs = S->n_runs;
         const int px = item.x0 + lane;
 
@@ -961,8 +960,7 @@ __global__ __launch_bounds__(256, REF ? 1 : (LINE ? 4 : (PAIR ? (NA == 32 ? 3 : 
         const float det_shift = (float)D / 2.0f;
         const float origin_shift = (float)N / 2.0f;
         const float shift = det_shift - rot;
-        const float fX = (float)px + 0.5f - origin_shift;
-        // active bins for the fast path's clamp-to-edge staging, kept inside
+        // active bins for the clamp-to-edge staging, kept inside
         // [0, D - 1]: an axis near 0 or past D leaves the active window empty
         // or outside the detector, and every staging load must stay in the row
         const int bin_lo = min(max((int)floorf(edge0 - 0.5f), 0), D - 1);
@@ -970,46 +968,33 @@ __global__ __launch_bounds__(256, REF ? 1 : (LINE ? 4 : (PAIR ? (NA == 32 ? 3 : 
         // Clamping the bins equals the reference's clamp of u (:203-210) when
         // both edges sit on bin centres (edge - 0.5 an integer: a centred axis,
         // or one shifted by a multiple of 1/2).  Otherwise an edge falls inside
-        // a bin, and the fast path clamps the coordinate itself (one more
-        // operation per sample; uniform over the slice).
+        // a bin, and the coordinate itself is clamped (one more operation per
+        // sample; uniform over the slice).
         const bool clamp_u =
-            !REF && !LINE && ((edge0 - 0.5f) != floorf(edge0 - 0.5f) || (edge1 - 0.5f) != floorf(edge1 - 0.5f));
+            !LINE && ((edge0 - 0.5f) != floorf(edge0 - 0.5f) || (edge1 - 0.5f) != floorf(edge1 - 0.5f));
         // Window corners (pixel centres): those of the 64 x 64 super-tile that
-        // holds the tile.  A tile of 32 rows stages its super-tile's window and,
-        // on the fast path, computes its super-tile's sample coordinates, so a
-        // pixel's result does not depend on the tile's rows or staged angles.
+        // holds the tile.  A tile of 32 rows stages its super-tile's window and
+        // computes its super-tile's sample coordinates, so a pixel's result does not depend on the tile's rows or staged angles.
         const int y0s = item.y0 & ~(kBpT - 1);
         const float cx0 = (float)item.x0 + 0.5f - origin_shift;
         const float cx1 = cx0 + (float)(kBpT - 1);
         const float cy0 = (float)y0s + 0.5f - origin_shift;
         const float cy1 = cy0 + (float)(kBpT - 1);
-        const float fY0 = (float)(item.y0 + wave) + 0.5f - origin_shift;
 
-        float acc[ROWS], val[ROWS], acc2[PAIR ? ROWS : 1];
+        float acc[ROWS], acc2[PAIR ? ROWS : 1];
 #pragma unroll
         for (int k = 0; k < ROWS; ++k) {
             acc[k] = 0.0f;
-            val[k] = 0.0f;
             if constexpr (PAIR)
                 acc2[k] = 0.0f;
         }
-        // fast path: minus the offset of each of this thread's rows within the
-        // super-tile, uniform over a wave (scalar registers)
-        float nys[REF ? 1 : ROWS];
-        if constexpr (!REF) {
-            const int ys0 = item.y0 - y0s + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        // minus the offset of each of this thread's rows within the super-tile,
+        // uniform over a wave (scalar registers)
+        float nys[ROWS];
+        const int ys0 = item.y0 - y0s + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 #pragma unroll
-            for (int q = 0; q < ROWS; ++q)
-                nys[q] = neg_float_of(ys0 + 4 * q);
-        }
-        if (REF && !S->pix_w) {
-            const TI *xin = uniform((const TI *)S->x);
-#pragma unroll
-            for (int k = 0; k < ROWS; ++k) {
-                const int py = item.y0 + wave + 4 * k;
-                acc[k] = (px < N && py < N) ? gload(xin, (uint32_t)py * (uint32_t)N + (uint32_t)px) : 0.0f;
-            }
-        }
+        for (int q = 0; q < ROWS; ++q)
+            nys[q] = neg_float_of(ys0 + 4 * q);
 
         for (int r = 0; r < n_runs; ++r) {
             const int roff = (int)S->run_off[r], rn = (int)S->run_n[r];
@@ -1024,7 +1009,7 @@ __global__ __launch_bounds__(256, REF ? 1 : (LINE ? 4 : (PAIR ? (NA == 32 ? 3 : 
                     const float u01 = cx0 * ct - cy1 * st, u11 = cx1 * ct - cy1 * st;
                     float umn = fminf(fminf(u00, u10), fminf(u01, u11)) + shift;
                     float umx = fmaxf(fmaxf(u00, u10), fmaxf(u01, u11)) + shift;
-                    if (REF || clamp_u) {
+                    if (clamp_u) {
                         umn = fminf(fmaxf(umn, edge0), edge1);
                         umx = fminf(fmaxf(umx, edge0), edge1);
                     }
@@ -1039,14 +1024,12 @@ __global__ __launch_bounds__(256, REF ? 1 : (LINE ? 4 : (PAIR ? (NA == 32 ? 3 : 
                         s_line[threadIdx.x] = make_float4(gload(lt, 8 * ang + 4), gload(lt, 8 * ang + 5),
                                                           gload(lt, 8 * ang + 6), gload(lt, 8 * ang + 7));
                     }
-                    if constexpr (!REF) {
-                        // u - 1/2 - umin at the super-tile's corner (joseph: less
-                        // another 1/2, as its entries are found by rounding to
-                        // nearest), rounded once; the line weights multiply
-                        // coordinate errors by 1 / (M m)
-                        s_base[threadIdx.x] = (float)((double)cx0 * (double)ct - (double)cy0 * (double)st +
-                                                      (double)shift - (LINE ? 0.5 : 1.0) - (double)umin);
-                    }
+                    // u - 1/2 - umin at the super-tile's corner (joseph: less
+                    // another 1/2, as its entries are found by rounding to
+                    // nearest), rounded once; the line weights multiply
+                    // coordinate errors by 1 / (M m)
+                    s_base[threadIdx.x] = (float)((double)cx0 * (double)ct - (double)cy0 * (double)st + (double)shift -
+                                                  (LINE ? 0.5 : 1.0) - (double)umin);
                 }
                 __syncthreads();
                 {
@@ -1062,7 +1045,7 @@ __global__ __launch_bounds__(256, REF ? 1 : (LINE ? 4 : (PAIR ? (NA == 32 ? 3 : 
                         const int i = lane + 64 * (e & 1);
                         const uint32_t rowo = (uint32_t)(abase + k) * (uint32_t)D;
                         const int bin = s_umin[k] + i;
-                        if constexpr (REF || LINE) {
+                        if constexpr (LINE) {
                             const int bc = min(max(bin, 0), D - 1);
                             const float t = gload(sino, rowo + (uint32_t)bc);
                             v0[e] = bin == bc ? t : 0.0f;
@@ -1091,7 +1074,7 @@ __global__ __launch_bounds__(256, REF ? 1 : (LINE ? 4 : (PAIR ? (NA == 32 ? 3 : 
                         if (k < na && i < kBpWb) {
                             if constexpr (LINE && PAIR) {
                                 ldl[k * kBpWb + i] = make_float2(v0[e], y0[e]);
-                            } else if constexpr (REF || LINE) {
+                            } else if constexpr (LINE) {
                                 lds[k * kBpWb + i] = v0[e];
                             } else {
                                 // (e, d) with d = t[i+1] - t[i], e = t[i] - (i - 1/2) d: the
@@ -1110,139 +1093,107 @@ __global__ __launch_bounds__(256, REF ? 1 : (LINE ? 4 : (PAIR ? (NA == 32 ? 3 : 
                 __syncthreads();
                 for (int k = 0; k < na; ++k) {
                     const float st = s_trig[2 * k], ct = s_trig[2 * k + 1];
-                    if constexpr (REF) {
-                        const float *L = lds + k * kBpWb - s_umin[k];
-                        const float fXc = fX * ct;
-#pragma unroll
-                        for (int g = 0; g < ROWS; g += 4) {
-                            float t0[4], t1[4], a[4];
-#pragma unroll
-                            for (int h = 0; h < 4; ++h) {
-                                const float fY = fY0 + (float)(4 * (g + h));
-                                float u = fXc - fY * st + shift;
-                                u = __builtin_amdgcn_fmed3f(u, edge0, edge1); // the clamp of :206-210
-                                const float w = u - 0.5f;                     // >= 0: edge0 >= 0.5
-                                const int i0 = cvt_flr(w);
-                                a[h] = fract_pos(w);
-                                t0[h] = L[i0];
-                                t1[h] = L[i0 + 1];
-                            }
-#pragma unroll
-                            for (int h = 0; h < 4; ++h) {
-                                const float oma = 1.0f - a[h];
-                                val[g + h] += oma * t0[h] + a[h] * t1[h];
-                            }
-                        }
-                    } else {
-                        // Window coordinates: row q's is fma(-ys_q, st, A), one FMA from
-                        // the thread's column term A and the row's offset ys_q in the
-                        // super-tile, whatever the tile's rows.  Joseph: less 1/2, so a
-                        // sample's entry is rne_index of it, one float add
-                        // (floor-converts and shifts issue at half the rate of float
-                        // adds), and its address one shift-add.
-                        const float A = __builtin_fmaf((float)lane, ct, s_base[k]);
-                        if constexpr (LINE) {
-                            const float4 L = s_line[k]; // (bp_k, bp_b0, bp_b1, 1/M)
-                            if constexpr (PAIR) {
-                                const float2 *B2 = ldl + k * kBpWb;
-#pragma unroll
-                                for (int g = 0; g < ROWS; g += 8) {
-                                    float2 p[8], q[8];
-                                    float fh[8];
-#pragma unroll
-                                    for (int h = 0; h < 8; ++h) {
-                                        const float w = __builtin_fmaf(nys[g + h], st, A); // >= 1: inside the window
-                                        const int i0 = cvt_flr(w);
-                                        p[h] = B2[i0];
-                                        q[h] = B2[i0 + 1];
-                                        fh[h] = fract_pos(w) - 0.5f;
-                                    }
-#pragma unroll
-                                    for (int h = 0; h < 8; ++h) {
-                                        const float w0 =
-                                            __builtin_amdgcn_fmed3f(__builtin_fmaf(fh[h], -L.x, L.y), 0.0f, L.w);
-                                        const float w1 =
-                                            __builtin_amdgcn_fmed3f(__builtin_fmaf(fh[h], L.x, L.z), 0.0f, L.w);
-                                        acc[g + h] = __builtin_fmaf(w1, q[h].x, __builtin_fmaf(w0, p[h].x, acc[g + h]));
-                                        acc2[g + h] =
-                                            __builtin_fmaf(w1, q[h].y, __builtin_fmaf(w0, p[h].y, acc2[g + h]));
-                                    }
-                                }
-                            } else {
-                                const float *B = lds + k * kBpWb;
-#pragma unroll
-                                for (int g = 0; g < ROWS; g += 8) {
-                                    float2 p[8];
-                                    float fh[8];
-#pragma unroll
-                                    for (int h = 0; h < 8; ++h) {
-                                        const float w = __builtin_fmaf(nys[g + h], st, A); // >= 1: inside the window
-                                        const int i0 = cvt_flr(w);
-                                        p[h] = make_float2(B[i0], B[i0 + 1]);
-                                        fh[h] = fract_pos(w) - 0.5f;
-                                    }
-#pragma unroll
-                                    for (int h = 0; h < 8; ++h) {
-                                        const float w0 = __builtin_amdgcn_fmed3f(__builtin_fmaf(fh[h], -L.x, L.y), 0.0f, L.w);
-                                        const float w1 = __builtin_amdgcn_fmed3f(__builtin_fmaf(fh[h], L.x, L.z), 0.0f, L.w);
-                                        acc[g + h] = __builtin_fmaf(w1, p[h].y, __builtin_fmaf(w0, p[h].x, acc[g + h]));
-                                    }
-                                }
-                            }
-                        } else if (!clamp_u) {
-                            const uint32_t P = lds_rne_base(ldp + k * kBpWb);
-                            // a copy of A per branch: the compiler would otherwise hoist
-                            // every row's coordinate above the branch, all live at once
-                            float Ab = A;
-                            asm volatile("" : "+v"(Ab));
+                    // Window coordinates: row q's is fma(-ys_q, st, A), one FMA from
+                    // the thread's column term A and the row's offset ys_q in the
+                    // super-tile, whatever the tile's rows.  Joseph: less 1/2, so a
+                    // sample's entry is rne_index of it, one float add
+                    // (floor-converts and shifts issue at half the rate of float
+                    // adds), and its address one shift-add.
+                    const float A = __builtin_fmaf((float)lane, ct, s_base[k]);
+                    if constexpr (LINE) {
+                        const float4 L = s_line[k]; // (bp_k, bp_b0, bp_b1, 1/M)
+                        if constexpr (PAIR) {
+                            const float2 *B2 = ldl + k * kBpWb;
 #pragma unroll
                             for (int g = 0; g < ROWS; g += 8) {
-                                E p[8];
-                                float w[8];
+                                float2 p[8], q[8];
+                                float fh[8];
 #pragma unroll
                                 for (int h = 0; h < 8; ++h) {
-                                    w[h] = __builtin_fmaf(nys[g + h], st, Ab);
-                                    p[h] = lds_rne_read<E>(P, w[h]);
+                                    const float w = __builtin_fmaf(nys[g + h], st, A); // >= 1: inside the window
+                                    const int i0 = cvt_flr(w);
+                                    p[h] = B2[i0];
+                                    q[h] = B2[i0 + 1];
+                                    fh[h] = fract_pos(w) - 0.5f;
                                 }
 #pragma unroll
                                 for (int h = 0; h < 8; ++h) {
-                                    acc[g + h] = __builtin_fmaf(w[h], p[h].y, acc[g + h] + p[h].x);
-                                    if constexpr (PAIR)
-                                        acc2[g + h] = __builtin_fmaf(w[h], p[h].w, acc2[g + h] + p[h].z);
+                                    const float w0 =
+                                        __builtin_amdgcn_fmed3f(__builtin_fmaf(fh[h], -L.x, L.y), 0.0f, L.w);
+                                    const float w1 =
+                                        __builtin_amdgcn_fmed3f(__builtin_fmaf(fh[h], L.x, L.z), 0.0f, L.w);
+                                    acc[g + h] = __builtin_fmaf(w1, q[h].x, __builtin_fmaf(w0, p[h].x, acc[g + h]));
+                                    acc2[g + h] =
+                                        __builtin_fmaf(w1, q[h].y, __builtin_fmaf(w0, p[h].y, acc2[g + h]));
                                 }
                             }
                         } else {
-                            // u clamped to [edge0, edge1] (:203-210), in window coordinates less 1/2
-                            const float wlo = (edge0 - 1.0f) - (float)s_umin[k];
-                            const float whi = (edge1 - 1.0f) - (float)s_umin[k];
-                            const uint32_t P = lds_rne_base(ldp + k * kBpWb);
-                            float Ab = A;
-                            asm volatile("" : "+v"(Ab));
+                            const float *B = lds + k * kBpWb;
 #pragma unroll
                             for (int g = 0; g < ROWS; g += 8) {
-                                E p[8];
-                                float w[8];
+                                float2 p[8];
+                                float fh[8];
 #pragma unroll
                                 for (int h = 0; h < 8; ++h) {
-                                    w[h] = __builtin_amdgcn_fmed3f(__builtin_fmaf(nys[g + h], st, Ab), wlo, whi);
-                                    p[h] = lds_rne_read<E>(P, w[h]);
+                                    const float w = __builtin_fmaf(nys[g + h], st, A); // >= 1: inside the window
+                                    const int i0 = cvt_flr(w);
+                                    p[h] = make_float2(B[i0], B[i0 + 1]);
+                                    fh[h] = fract_pos(w) - 0.5f;
                                 }
 #pragma unroll
                                 for (int h = 0; h < 8; ++h) {
-                                    acc[g + h] = __builtin_fmaf(w[h], p[h].y, acc[g + h] + p[h].x);
-                                    if constexpr (PAIR)
-                                        acc2[g + h] = __builtin_fmaf(w[h], p[h].w, acc2[g + h] + p[h].z);
+                                    const float w0 = __builtin_amdgcn_fmed3f(__builtin_fmaf(fh[h], -L.x, L.y), 0.0f, L.w);
+                                    const float w1 = __builtin_amdgcn_fmed3f(__builtin_fmaf(fh[h], L.x, L.z), 0.0f, L.w);
+                                    acc[g + h] = __builtin_fmaf(w1, p[h].y, __builtin_fmaf(w0, p[h].x, acc[g + h]));
                                 }
                             }
                         }
-                    }
-                }
-            }
-            if (REF) { // per-run accumulation (:216)
+                    } else if (!clamp_u) {
+                        const uint32_t P = lds_rne_base(ldp + k * kBpWb);
+                        // a copy of A per branch: the compiler would otherwise hoist
+                        // every row's coordinate above the branch, all live at once
+                        float Ab = A;
+                        asm volatile("" : "+v"(Ab));
 #pragma unroll
-                for (int q = 0; q < ROWS; ++q) {
-                    acc[q] = acc[q] + relax * val[q];
-                    val[q] = 0.0f;
+                        for (int g = 0; g < ROWS; g += 8) {
+                            E p[8];
+                            float w[8];
+#pragma unroll
+                            for (int h = 0; h < 8; ++h) {
+                                w[h] = __builtin_fmaf(nys[g + h], st, Ab);
+                                p[h] = lds_rne_read<E>(P, w[h]);
+                            }
+#pragma unroll
+                            for (int h = 0; h < 8; ++h) {
+                                acc[g + h] = __builtin_fmaf(w[h], p[h].y, acc[g + h] + p[h].x);
+                                if constexpr (PAIR)
+                                    acc2[g + h] = __builtin_fmaf(w[h], p[h].w, acc2[g + h] + p[h].z);
+                            }
+                        }
+                    } else {
+                        // u clamped to [edge0, edge1] (:203-210), in window coordinates less 1/2
+                        const float wlo = (edge0 - 1.0f) - (float)s_umin[k];
+                        const float whi = (edge1 - 1.0f) - (float)s_umin[k];
+                        const uint32_t P = lds_rne_base(ldp + k * kBpWb);
+                        float Ab = A;
+                        asm volatile("" : "+v"(Ab));
+#pragma unroll
+                        for (int g = 0; g < ROWS; g += 8) {
+                            E p[8];
+                            float w[8];
+#pragma unroll
+                            for (int h = 0; h < 8; ++h) {
+                                w[h] = __builtin_amdgcn_fmed3f(__builtin_fmaf(nys[g + h], st, Ab), wlo, whi);
+                                p[h] = lds_rne_read<E>(P, w[h]);
+                            }
+#pragma unroll
+                            for (int h = 0; h < 8; ++h) {
+                                acc[g + h] = __builtin_fmaf(w[h], p[h].y, acc[g + h] + p[h].x);
+                                if constexpr (PAIR)
+                                    acc2[g + h] = __builtin_fmaf(w[h], p[h].w, acc2[g + h] + p[h].z);
+                            }
+                        }
+                    }
                 }
             }
         }
@@ -1253,7 +1204,7 @@ __global__ __launch_bounds__(256, REF ? 1 : (LINE ? 4 : (PAIR ? (NA == 32 ? 3 : 
             const float *pix_w = uniform(Sx->pix_w);
             const int posc = Sx->posc;
             const float gain = Sx->relax * Sx->pix_scale;
-            const float *tv = REF ? nullptr : uniform(Sx->tv);
+            const float *tv = uniform(Sx->tv);
             const float tv_scale = Sx->tv_scale;
 #pragma unroll
             for (int q = 0; q < ROWS; ++q) {
@@ -1262,13 +1213,7 @@ __global__ __launch_bounds__(256, REF ? 1 : (LINE ? 4 : (PAIR ? (NA == 32 ? 3 : 
                     continue;
                 const uint32_t o = (uint32_t)py * (uint32_t)N + (uint32_t)px;
                 float out;
-                if (REF) {
-                    out = a[q];
-                    if (pix_w) { // SIRT form (ufo-ir-sirt-task.c:208-212)
-                        out = out * gload(pix_w, o);
-                        out = out + gload(xin, o);
-                    }
-                } else if (LINE && tv) {
+                if (LINE && tv) {
                     // split-Bregman sweep of the line model: P = 1 / (mu BP(1) + 8 lambda)
                     // per pixel, from C = 1 / BP(1) (0: BP(1) below the floor)
                     const float C = gload(pix_w, o), mu = Sx->pix_scale, lam = Sx->tv_scale;
@@ -1694,11 +1639,11 @@ int launch_fp_pairs(const uirk_slice *sl, const uirk_slice &one, const uirk_fp_i
     return (int)hipGetLastError();
 }
 
-template <typename T, typename TI, bool REF, int NA, int ROWS, bool LINE = false, bool PAIR = false>
+template <typename T, typename TI, int NA, int ROWS, bool LINE = false, bool PAIR = false>
 int launch_bp(const uirk_slice *sl, const uirk_slice &one, const uirk_bp_item *items, int n,
               const uirk_xcd_part &part, int grid, int *err, hipStream_t st)
 {
-    hipLaunchKernelGGL((k_bp_tab<T, TI, REF, NA, ROWS, LINE, PAIR>), dim3(grid), dim3(256), 0, st, sl, one, items, n,
+    hipLaunchKernelGGL((k_bp_tab<T, TI, NA, ROWS, LINE, PAIR>), dim3(grid), dim3(256), 0, st, sl, one, items, n,
                        part, err);
     return (int)hipGetLastError();
 }
@@ -1731,28 +1676,28 @@ int launch_bp_fast(const uirk_tile &tile, bool line, bool pair, const uirk_slice
                    const uirk_bp_item *items, int n, const uirk_xcd_part &part, int grid, int *err, hipStream_t st)
 {
     if (line && pair) // 32 staged angles; tiles of 64 or 32 rows
-        return tile.bp_rows == 32 ? launch_bp<T, TI, false, 32, 8, true, true>(sl, one, items, n, part, grid, err, st)
-                                  : launch_bp<T, TI, false, 32, 16, true, true>(sl, one, items, n, part, grid, err, st);
+        return tile.bp_rows == 32 ? launch_bp<T, TI, 32, 8, true, true>(sl, one, items, n, part, grid, err, st)
+                                  : launch_bp<T, TI, 32, 16, true, true>(sl, one, items, n, part, grid, err, st);
     if (line)
-        return tile.bp_rows == 32 ? launch_bp<T, TI, false, 32, 8, true>(sl, one, items, n, part, grid, err, st)
-                                  : launch_bp<T, TI, false, 32, 16, true>(sl, one, items, n, part, grid, err, st);
+        return tile.bp_rows == 32 ? launch_bp<T, TI, 32, 8, true>(sl, one, items, n, part, grid, err, st)
+                                  : launch_bp<T, TI, 32, 16, true>(sl, one, items, n, part, grid, err, st);
     const bool na16 = tile.bp_angles == 16, r8 = tile.bp_rows == 32;
     if (pair) {
         if (na16 && r8)
-            return launch_bp<T, TI, false, 16, 8, false, true>(sl, one, items, n, part, grid, err, st);
+            return launch_bp<T, TI, 16, 8, false, true>(sl, one, items, n, part, grid, err, st);
         if (na16)
-            return launch_bp<T, TI, false, 16, 16, false, true>(sl, one, items, n, part, grid, err, st);
+            return launch_bp<T, TI, 16, 16, false, true>(sl, one, items, n, part, grid, err, st);
         if (r8)
-            return launch_bp<T, TI, false, 32, 8, false, true>(sl, one, items, n, part, grid, err, st);
-        return launch_bp<T, TI, false, 32, 16, false, true>(sl, one, items, n, part, grid, err, st);
+            return launch_bp<T, TI, 32, 8, false, true>(sl, one, items, n, part, grid, err, st);
+        return launch_bp<T, TI, 32, 16, false, true>(sl, one, items, n, part, grid, err, st);
     }
     if (na16 && r8)
-        return launch_bp<T, TI, false, 16, 8>(sl, one, items, n, part, grid, err, st);
+        return launch_bp<T, TI, 16, 8>(sl, one, items, n, part, grid, err, st);
     if (na16)
-        return launch_bp<T, TI, false, 16, 16>(sl, one, items, n, part, grid, err, st);
+        return launch_bp<T, TI, 16, 16>(sl, one, items, n, part, grid, err, st);
     if (r8)
-        return launch_bp<T, TI, false, 32, 8>(sl, one, items, n, part, grid, err, st);
-    return launch_bp<T, TI, false, 32, 16>(sl, one, items, n, part, grid, err, st);
+        return launch_bp<T, TI, 32, 8>(sl, one, items, n, part, grid, err, st);
+    return launch_bp<T, TI, 32, 16>(sl, one, items, n, part, grid, err, st);
 }
 
 // (sinogram, image) storage pairs: both FP32, both FP16, both BF16, or
@@ -1911,11 +1856,6 @@ int uirk_bp_table(const uirk_slice *d_slices, const uirk_slice *one, const uirk_
     if (part)
         pt = *part;
     hipStream_t st = (hipStream_t)stream;
-    if (mode == 0) {
-        if (dtype != UIR_DTYPE_F32 || img_dtype != UIR_DTYPE_F32 || tl.bp_angles != 32 || tl.bp_rows != UIRK_BP_TILE)
-            return (int)hipErrorInvalidValue;
-        return launch_bp<float, float, true, 32, 16>(d_slices, single, d_items, n_items, pt, grid, d_err, st);
-    }
     if (mode < 1 || mode > 4 || (mode >= 3 && !d_slices))
         return (int)hipErrorInvalidValue;
     return launch_fast<false>(dtype, img_dtype, tl, mode == 2 || mode == 4, mode >= 3, d_slices, single, d_items,

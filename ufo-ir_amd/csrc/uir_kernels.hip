@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstring>
+#include <type_traits>
 
 #include "uir_device.h"
 
@@ -331,7 +332,7 @@ __global__ __launch_bounds__(256) void k_fp_ref_seg(FpRefArgs p, const float *__
 }
 
 // --------------------------------------------------------------------------
-// Backprojection, one thread per pixel, per-run accumulation.
+// Backprojection, R pixels per thread, per-run accumulation.
 // --------------------------------------------------------------------------
 struct BpRefArgs {
     const float *r_vol;
@@ -345,14 +346,52 @@ struct BpRefArgs {
     uirk_runs runs;
 };
 
-__global__ __launch_bounds__(256) void k_bp_ref(BpRefArgs p)
+// The taps are gathered straight from the sinogram rows: neighbouring pixels
+// read neighbouring bins, so a wave's 64 taps lie in three cache lines that the
+// workgroup's other rows read too, and nothing is staged or waited for at a
+// barrier.  A thread keeps R pixels (rows) and takes kBpU angles at a time, all
+// their taps in flight before the first is used.  What bounds it is the VALU:
+// about 13 operations a sample, three of them at half rate.  Against LDS-staged
+// 64 x 64 tiles (a wave a SIMD at 1024 x 1024, 16 workgroups at 256 x 256) it
+// took 197 us instead of 425 at 1024 / 720 / 1448 and 15 instead of 109 at
+// 256 / 180 / 367.
+constexpr int kBpU = 8;
+
+// A raw buffer load whose byte offset lies at or beyond the resource's size
+// returns zero and touches no memory (negative offsets are large unsigned
+// ones): the zero border of a row.  The offset has to be whole in the vector
+// register, as the check does not see a wrap by an immediate one (opaque).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t row_rsrc(const float *base, uint32_t elems)
 {
-    const int px = blockIdx.x * 64 + threadIdx.x;
-    const int py = blockIdx.y * 4 + threadIdx.y;
+    return __builtin_amdgcn_make_buffer_rsrc((void *)base, (short)0, (int)(elems * 4u), 0x00020000);
+}
+__device__ __forceinline__ float row_load(__amdgpu_buffer_rsrc_t r, int i)
+{
+    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, (uint32_t)i * 4u, 0, 0));
+}
+__device__ __forceinline__ int opaque(int i)
+{
+    asm("" : "+v"(i));
+    return i;
+}
+
+// floor(x) converted to int in one instruction (no memory access).
+__device__ __forceinline__ int cvt_flr(float x)
+{
+    int r;
+    asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(r) : "v"(x));
+    return r;
+}
+
+// CLAMP 2: any axis.  1: 0.5 <= edge0 <= edge1 <= n_dets - 0.5 (an axis with
+// active detectors), so that the clamp is one median and every lower tap lies
+// in the row.  0: no pixel reaches an edge either, no clamp.
+template <int R, int CLAMP> __global__ __launch_bounds__(256) void k_bp_gather(BpRefArgs p)
+{
     const int N = p.n, D = p.n_dets;
-    if (px >= N || py >= N)
-        return;
-    const size_t o = (size_t)py * N + px;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int px = blockIdx.x * 64 + lane;
+    const int py0 = (blockIdx.y * 4 + wave) * R;
 
     // projector-parallel-joseph.cl:174-190 (detector quantities use n_dets)
     const float required_width = p.axis * 2;
@@ -365,39 +404,99 @@ __global__ __launch_bounds__(256) void k_bp_ref(BpRefArgs p)
     const float origin_shift = (float)N / 2.0f;
     const float shift = det_shift - rot;
     const float fX = (float)px + 0.5f - origin_shift;
-    const float fY = (float)py + 0.5f - origin_shift;
-
-    float out = p.pix_w ? 0.0f : p.r_vol[o];
+    float fY[R], out[R];
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+        fY[q] = (float)(py0 + q) + 0.5f - origin_shift;
+        out[q] = (!p.pix_w && px < N && py0 + q < N) ? p.r_vol[(size_t)(py0 + q) * N + px] : 0.0f;
+    }
     for (int r = 0; r < p.runs.count; ++r) {
         const int off = (int)p.runs.offset[r], cnt = (int)p.runs.n[r];
-        float value = 0.0f;
-        for (int k = 0; k < cnt; ++k) { // :196-214
-            const int ang = off + k;
-            const float st = p.sin_lut[ang], ct = p.cos_lut[ang];
-            float u = fX * ct - fY * st + shift;
-            if (u > edge1)
-                u = edge1;
-            else if (u < edge0)
-                u = edge0;
-            const float w = u - 0.5f;
-            const float fw = floorf(w);
-            const int i0 = (int)fw;
-            const float a = w - fw;
-            const float oma = 1.0f - a;
-            const float *row = p.sino + (size_t)ang * D;
-            const float t0 = (i0 >= 0 && i0 < D) ? row[i0] : 0.0f;
-            const float t1 = (i0 + 1 >= 0 && i0 + 1 < D) ? row[i0 + 1] : 0.0f;
-            value += oma * t0 + a * t1;
+        float value[R];
+#pragma unroll
+        for (int q = 0; q < R; ++q)
+            value[q] = 0.0f;
+        // :196-214, kBpU angles at a time: their taps are all in flight before
+        // the first is used
+        auto angles = [&](int k, auto n_) {
+            constexpr int n = decltype(n_)::value;
+            float t0[n][R], t1[n][R], a[n][R];
+#pragma unroll
+            for (int e = 0; e < n; ++e) {
+                const int ang = off + k + e;
+                const float st = p.sin_lut[ang], ct = p.cos_lut[ang];
+                const float *row = p.sino + (size_t)ang * D;
+                const __amdgpu_buffer_rsrc_t r0 = row_rsrc(row, (uint32_t)D), r1 = row_rsrc(row + 1, (uint32_t)D - 1u);
+                const float fXc = fX * ct;
+#pragma unroll
+                for (int q = 0; q < R; ++q) {
+                    float u = fXc - fY[q] * st + shift;
+                    if (CLAMP == 1) {
+                        u = __builtin_amdgcn_fmed3f(u, edge0, edge1);
+                    } else if (CLAMP == 2) {
+                        if (u > edge1)
+                            u = edge1;
+                        else if (u < edge0)
+                            u = edge0;
+                    }
+                    const float w = u - 0.5f;
+                    const int i0 = cvt_flr(w);
+                    a[e][q] = CLAMP < 2 ? __builtin_amdgcn_fractf(w) : w - floorf(w); // the same for w >= 0
+                    t0[e][q] = row_load(r0, i0);
+                    t1[e][q] = CLAMP < 2 ? row_load(r1, i0) : row_load(r0, opaque(i0 + 1));
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < n; ++e) {
+#pragma unroll
+                for (int q = 0; q < R; ++q) {
+                    const float oma = 1.0f - a[e][q];
+                    value[q] += oma * t0[e][q] + a[e][q] * t1[e][q];
+                }
+            }
+        };
+        int k = 0;
+        for (; k + kBpU <= cnt; k += kBpU)
+            angles(k, std::integral_constant<int, kBpU>{});
+        for (; k < cnt; ++k)
+            angles(k, std::integral_constant<int, 1>{});
+#pragma unroll
+        for (int q = 0; q < R; ++q)
+            out[q] = out[q] + p.relax * value[q]; // :216
+    }
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+        if (px >= N || py0 + q >= N)
+            continue;
+        const size_t o = (size_t)(py0 + q) * N + px;
+        float v = out[q];
+        if (p.pix_w) {
+            v = v * p.pix_w[o];
+            v = v + p.r_vol[o];
+            if (p.posc)
+                v = v > 0 ? v : 0.0f;
         }
-        out = out + p.relax * value; // :216
+        p.w_vol[o] = v;
     }
-    if (p.pix_w) {
-        out = out * p.pix_w[o];
-        out = out + p.r_vol[o];
-        if (p.posc)
-            out = out > 0 ? out : 0.0f;
-    }
-    p.w_vol[o] = out;
+}
+
+template <int R> void launch_bp_gather(const BpRefArgs &a, hipStream_t st)
+{
+    const float half = (float)a.n_dets - a.axis * 2 < 0 ? (float)a.n_dets - a.axis : a.axis;
+    const float edge0 = a.axis - half + 0.5f, edge1 = a.axis + half - 0.5f;
+    const bool window = edge0 >= 0.5f && edge0 <= edge1 && edge1 <= (float)a.n_dets - 0.5f;
+    // u - shift is at most the distance of a corner pixel's centre from the
+    // image centre, plus the rounding of three float operations
+    const float rot = ((float)a.n_dets - a.axis * 2) / 2.0f, shift = (float)a.n_dets / 2.0f - rot;
+    const double reach = 0.7071067811865476 * (a.n - 1) * (1.0 + 1e-5) + 1e-3;
+    const bool inside = window && shift - reach > edge0 && shift + reach < edge1;
+    const dim3 grid((a.n + 63) / 64, (a.n + 4 * R - 1) / (4 * R));
+    if (inside)
+        hipLaunchKernelGGL((k_bp_gather<R, 0>), grid, dim3(256), 0, st, a);
+    else if (window)
+        hipLaunchKernelGGL((k_bp_gather<R, 1>), grid, dim3(256), 0, st, a);
+    else
+        hipLaunchKernelGGL((k_bp_gather<R, 2>), grid, dim3(256), 0, st, a);
 }
 
 // --------------------------------------------------------------------------
@@ -899,8 +998,14 @@ int uirk_bp_ref(const float *r_vol, float *w_vol, const float *sino, int n_angle
     a.axis = axis;
     a.relax = relax;
     a.runs = *runs;
-    dim3 block(64, 4), grid((n + 63) / 64, (n + 3) / 4);
-    hipLaunchKernelGGL(k_bp_ref, grid, block, 0, (hipStream_t)stream, a);
+    // Two pixels a thread from 512 x 512 on (2 waves a SIMD are left): the
+    // per-angle scalar work is shared.  Below, one: 15 us against 22 at 256 /
+    // 180 / 367; at 512 / 400 / 725 both take 46 - 51 us, at 1024 / 720 / 1448
+    // two take 197 us and one 269.
+    if (n < 512)
+        launch_bp_gather<1>(a, (hipStream_t)stream);
+    else
+        launch_bp_gather<2>(a, (hipStream_t)stream);
     return (int)hipGetLastError();
 }
 

@@ -42,13 +42,12 @@ struct uir_task {
     uint32_t lut_n;
     uir_subset *runs;
     uint32_t n_runs;
-    /* work tables of the table-driven kernels for the current geometry */
+    /* FP work table of the table-driven kernel for the current geometry */
     uint32_t plan_n, plan_dets, plan_angles;
     float plan_axis;
     uirk_fp_item *d_fp_items;
-    uirk_bp_item *d_bp_items;
-    int n_fp_items, n_bp_items;
-    uirk_xcd_part fp_part, bp_part;
+    int n_fp_items;
+    uirk_xcd_part fp_part;
     float *d_trig;
     int *d_err;
     /* the line model (model "line"): per-angle constants of the current
@@ -268,7 +267,6 @@ void uir_task_unref(uir_task *t)
     uir_dfree(t->d_cos);
     free(t->runs);
     uir_dfree(t->d_fp_items);
-    uir_dfree(t->d_bp_items);
     uir_dfree(t->d_trig);
     uir_dfree(t->d_err);
     free(t->h_line);
@@ -594,48 +592,46 @@ static void proj_runs_dev(const uir_task *p, const uir_subset *subs, uint32_t n,
     (void)p;
 }
 
-/* Work tables of the projector's current geometry for an n x n image. */
+static uir_status proj_limits(const uir_task *p, uint32_t n)
+{
+    if ((uint64_t)n * n * 4 >= (1ull << 32) || (uint64_t)p->lut_n * p->n_dets * 4 >= (1ull << 32))
+        return uir_set_error(UIR_ERR_INVALID_ARGUMENT, "image or sinogram of 4 GiB or more");
+    return UIR_OK;
+}
+
+/* FP work table of the projector's current geometry for an n x n image. */
 static uir_status proj_plan(uir_task *p, uint32_t n)
 {
     const float axis = proj_axis(p);
-    if ((uint64_t)n * n * 4 >= (1ull << 32) || (uint64_t)p->lut_n * p->n_dets * 4 >= (1ull << 32))
-        return uir_set_error(UIR_ERR_INVALID_ARGUMENT, "image or sinogram of 4 GiB or more");
+    TRY(proj_limits(p, n));
     if (p->d_fp_items && p->plan_n == n && p->plan_dets == p->n_dets && p->plan_angles == p->lut_n &&
         p->plan_axis == axis)
         return UIR_OK;
     uir_dfree(p->d_fp_items);
-    uir_dfree(p->d_bp_items);
     uir_dfree(p->d_trig);
     p->d_fp_items = NULL;
-    p->d_bp_items = NULL;
     p->d_trig = NULL;
     uirk_fp_vec fv = {0};
-    uirk_bp_vec bv = {0};
     float *trig = (float *)malloc(sizeof(float) * 2 * (p->lut_n ? p->lut_n : 1));
     uir_status s = UIR_OK;
     if (!trig || uirk_plan_fp(&fv, 0, (int)n, (int)p->n_dets, axis, p->h_sin, p->h_cos, p->runs, p->n_runs,
-                              UIRK_FP_ANGLES, UIRK_FP_WMAX_SINGLE) ||
-        uirk_plan_bp(&bv, 0, (int)n, UIRK_BP_TILE)) {
+                              UIRK_FP_ANGLES, UIRK_FP_WMAX_SINGLE)) {
         s = uir_set_error(UIR_ERR_OUT_OF_MEMORY, "work table");
         goto done;
     }
     uirk_plan_trig(p->h_sin, p->h_cos, p->lut_n, trig);
     if ((s = uir_dmalloc((void **)&p->d_fp_items, fv.n * sizeof(uirk_fp_item))) != UIR_OK ||
-        (s = uir_dmalloc((void **)&p->d_bp_items, bv.n * sizeof(uirk_bp_item))) != UIR_OK ||
         (s = uir_dmalloc((void **)&p->d_trig, 2 * sizeof(float) * (p->lut_n ? p->lut_n : 1))) != UIR_OK)
         goto done;
     if (!p->d_err && (s = uir_dmalloc((void **)&p->d_err, sizeof(int))) != UIR_OK)
         goto done;
     if ((s = uir_check_hip(hipMemcpy(p->d_fp_items, fv.v, fv.n * sizeof(uirk_fp_item), hipMemcpyHostToDevice),
                            "table upload")) != UIR_OK ||
-        (s = uir_check_hip(hipMemcpy(p->d_bp_items, bv.v, bv.n * sizeof(uirk_bp_item), hipMemcpyHostToDevice),
-                           "table upload")) != UIR_OK ||
         (s = uir_check_hip(hipMemcpy(p->d_trig, trig, 2 * sizeof(float) * p->lut_n, hipMemcpyHostToDevice),
                            "table upload")) != UIR_OK ||
         (s = uir_check_hip(hipMemset(p->d_err, 0, sizeof(int)), "memset")) != UIR_OK)
         goto done;
     p->n_fp_items = (int)fv.n;
-    p->n_bp_items = (int)bv.n;
     {
         double *cost = (double *)malloc(sizeof(double) * (fv.n ? fv.n : 1));
         if (!cost) {
@@ -645,7 +641,6 @@ static uir_status proj_plan(uir_task *p, uint32_t n)
         for (size_t i = 0; i < fv.n; ++i)
             cost[i] = uirk_fp_item_cost(&fv.v[i]);
         uirk_plan_xcd(cost, (int)fv.n, uirk_plan_num_xcd(), &p->fp_part);
-        uirk_plan_xcd(NULL, (int)bv.n, uirk_plan_num_xcd(), &p->bp_part);
         free(cost);
     }
     p->plan_n = n;
@@ -654,7 +649,6 @@ static uir_status proj_plan(uir_task *p, uint32_t n)
     p->plan_axis = axis;
 done:
     free(fv.v);
-    free(bv.v);
     free(trig);
     if (s != UIR_OK) {
         uir_dfree(p->d_fp_items);
@@ -886,25 +880,14 @@ static uir_status proj_bp_ex(uir_task *p, uint32_t n, const float *sino, float *
                                            p->d_err, p->res->stream),
                              "BP launch");
     }
-    TRY(proj_plan(p, n));
+    TRY(proj_limits(p, n));
     if (pix_w && p->n_runs > UIRK_MAX_RUNS)
         return uir_set_error(UIR_ERR_UNSUPPORTED, "more than %d direction runs", UIRK_MAX_RUNS);
     for (uint32_t first = 0; first < p->n_runs; first += UIRK_MAX_RUNS) {
-        uirk_slice sl;
-        proj_slice(p, n, &sl);
-        sl.b = sino;
-        sl.x = vol;
-        sl.x_out = vol;
-        sl.pix_w = pix_w;
-        sl.posc = posc;
-        uint32_t k = 0;
-        for (uint32_t i = first; i < p->n_runs && k < UIRK_MAX_RUNS; ++i, ++k) {
-            sl.run_off[k] = p->runs[i].offset;
-            sl.run_n[k] = p->runs[i].n;
-        }
-        sl.n_runs = (int32_t)k;
-        TRY(uir_check_hip(uirk_bp_table(NULL, &sl, p->d_bp_items, p->n_bp_items, &p->bp_part, 0, UIR_DTYPE_F32, UIR_DTYPE_F32, NULL,
-                                        uirk_plan_grid_xcd(&p->bp_part, p->n_bp_items), p->d_err, p->res->stream), "BP launch"));
+        uirk_runs r;
+        proj_runs_dev(p, p->runs, p->n_runs, &r, first);
+        TRY(uir_check_hip(uirk_bp_ref(vol, vol, sino, (int)p->lut_n, p->d_sin, p->d_cos, (int)n, (int)p->n_dets,
+                                      proj_axis(p), p->relaxation, &r, pix_w, posc, p->res->stream), "BP launch"));
     }
     return UIR_OK;
 }
