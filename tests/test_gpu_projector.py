@@ -60,6 +60,30 @@ def test_bp_matches_oracle(res, n, d, a, step):
 
 
 @pytest.mark.parametrize("n,d,a,axis", [
+    (1, 1, 1, -1.0), (3, 5, 2, -1.0), (64, 64, 9, -1.0),
+    (71, 101, 12, -1.0), (130, 184, 10, 85.25),   # a last block of 7 and of 2 lines; inactive detectors
+    (640, 906, 6, -1.0), (641, 907, 6, -1.0),     # both sides of the staged work table's line
+    (200, 283, 40, 260.5),
+])
+def test_fp_bit_exact(res, n, d, a, axis):
+    """The FP runs the reference's operations in its order
+    (projector-parallel-joseph.cl:51-94): equal to the oracle bit for bit,
+    adding to what the sinogram holds."""
+    print("case fp bit-exact", n, d, a, axis, flush=True)
+    step = np.float32(np.pi / a)
+    g = O.Geometry(n, d, a, step, axis=axis)
+    rng = np.random.default_rng(n + a)
+    x = rng.standard_normal((n, n)).astype(np.float32)
+    base = rng.standard_normal((a, d)).astype(np.float32)
+    p = _projector(n, d, a, step, True, axis_position=axis).setup(res)
+    dx, ds = uir.DeviceArray.from_numpy(x), uir.DeviceArray.from_numpy(base)
+    assert p.requisition(dx) == (a, d)
+    p["correction_scale"] = 0.75
+    p.forward(dx, ds)
+    assert np.array_equal(ds.numpy(), O.fp(g, x, sino=base, corr=0.75))
+
+
+@pytest.mark.parametrize("n,d,a,axis", [
     (1, 1, 1, -1.0), (3, 5, 2, -1.0),
     (63, 90, 7, -1.0), (65, 65, 9, -1.0),       # no clamp; detector as wide as the image: clamped corners
     (511, 723, 17, -1.0), (513, 726, 15, -1.0),  # one and two pixels a thread, odd last rows, angles not in eights

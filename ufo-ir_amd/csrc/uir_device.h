@@ -54,6 +54,15 @@ int uirk_fp_ref_split(const float *vol, const float *r_sino, float *w_sino, cons
                       const float *sin_lut, const float *cos_lut, int n, int n_dets, float axis,
                       float corr, int ang0, int n_ang, int dir, void *stream);
 
+/* out = in^T, n x n. */
+int uirk_transpose(const float *in, float *out, int n, void *stream);
+/* The same FP, bit-identical, over all of a projector's rays (each angle takes
+ * the direction of its LUT pair): one wave per 64-sample block of 64 rays.
+ * vol_t: the transpose of vol (may be NULL if no angle is horizontal). */
+int uirk_fp_blocks(const float *vol, const float *vol_t, const float *r_sino, float *w_sino, const float *ray_w,
+                   const float *sin_lut, const float *cos_lut, int n, int n_dets, float axis, float corr, int ang0,
+                   int n_ang, void *stream);
+
 /* The coordinate at the start of every 64-sample block of every ray of
  * angles [0, n_angles) ([angle][detector][block], ceil(n / 64) blocks), taken
  * by the reference's sequential float walk; inactive rays get 0. */

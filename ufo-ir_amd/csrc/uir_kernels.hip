@@ -18,6 +18,24 @@ namespace {
 
 constexpr int kBlockSamples = 64; // projector-parallel-joseph.cl:4
 
+// A raw buffer load whose byte offset lies at or beyond the resource's size
+// returns zero and touches no memory (negative offsets are large unsigned
+// ones): the zero border of a row.  The offset has to be whole in the vector
+// register, as the check does not see a wrap by an immediate one (opaque).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t row_rsrc(const float *base, uint32_t elems)
+{
+    return __builtin_amdgcn_make_buffer_rsrc((void *)base, (short)0, (int)(elems * 4u), 0x00020000);
+}
+__device__ __forceinline__ float row_load(__amdgpu_buffer_rsrc_t r, int i)
+{
+    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, (uint32_t)i * 4u, 0, 0));
+}
+__device__ __forceinline__ int opaque(int i)
+{
+    asm("" : "+v"(i));
+    return i;
+}
+
 // --------------------------------------------------------------------------
 // Joseph forward projection, one thread per ray (detector s, angle).
 // --------------------------------------------------------------------------
@@ -200,6 +218,108 @@ __global__ __launch_bounds__(256) void k_fp_ref_split(FpRefArgs p)
 }
 
 // --------------------------------------------------------------------------
+// The same projection with one wave per 64-sample block of 64 rays, from the
+// image and its transpose.
+// --------------------------------------------------------------------------
+// A workgroup owns 64 detectors of one angle, a wave one of the rays' blocks
+// (waves past 16 blocks take further ones): it replays the reference's float
+// additions to the block's start, and its samples walk the lines of the image
+// (FP_vert) or of the transposed image (FP_hor), so that the 64 rays' taps are
+// neighbours on one line and the line's ends read as zero.  The block sums
+// meet in LDS and are added in block order.  For images whose LDS-staged work
+// table (k_fp_tab) would leave most of the chip idle.
+constexpr int kBlkWaves = 16;
+
+// kFpBatch samples (or n of them) of a block from line l on, added in order.
+template <int n> __device__ __forceinline__ float fp_lines(const float *img, int N, int l, float &pos, float step, float inner)
+{
+    float w[n], va[n], vb[n];
+#pragma unroll
+    for (int k = 0; k < n; ++k) {
+        const float v = pos - 0.5f;
+        const float fv = floorf(v);
+        const int c0 = (int)fv;
+        w[k] = v - fv;
+        const __amdgpu_buffer_rsrc_t r = row_rsrc(img + (size_t)(l + k) * N, (uint32_t)N);
+        va[k] = row_load(r, c0);
+        vb[k] = row_load(r, opaque(c0 + 1));
+        pos += step;
+    }
+#pragma unroll
+    for (int k = 0; k < n; ++k) {
+        const float omw = 1.0f - w[k];
+        inner += omw * va[k] + w[k] * vb[k];
+    }
+    return inner;
+}
+
+__global__ __launch_bounds__(64 * kBlkWaves) void k_fp_blocks(FpRefArgs p, const float *__restrict__ vol_t)
+{
+    __shared__ float sums[kBlkWaves][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n_waves = blockDim.x >> 6;
+    const int s = blockIdx.x * 64 + lane, ang = p.ang0 + blockIdx.y;
+    const int N = p.n, n_blocks = (N + kBlockSamples - 1) / kBlockSamples;
+    const size_t o = (size_t)ang * p.n_dets + s;
+    float pos = 0.0f, step = 0.0f;
+    int dir = 0;
+    const bool live = s < p.n_dets &&
+                      fp_ray_setup(s, ang, N, p.n_dets, p.axis, p.sin_lut, p.cos_lut, p.dir, pos, step, dir);
+    const bool vertical = p.dir >= 0 ? p.dir != 0 : fabsf(p.sin_lut[ang]) <= fabsf(p.cos_lut[ang]); // uniform
+    const float *img = vertical ? p.vol : vol_t;
+    float acc = 0.0f;
+    int at = 0; // blocks already stepped over
+    for (int j0 = 0; j0 < n_blocks; j0 += n_waves) {
+        const int j = j0 + wave;
+        if (j < n_blocks) {
+            for (; at < j; ++at) {
+#pragma unroll
+                for (int k = 0; k < kBlockSamples; ++k)
+                    pos += step;
+            }
+            const int bend = min(N, (j + 1) * kBlockSamples);
+            float inner = 0.0f;
+            int l = j * kBlockSamples;
+            for (; l + kFpBatch <= bend; l += kFpBatch)
+                inner = fp_lines<kFpBatch>(img, N, l, pos, step, inner);
+            for (; l < bend; ++l)
+                inner = fp_lines<1>(img, N, l, pos, step, inner);
+            at = j + 1;
+            sums[wave][lane] = inner;
+        }
+        __syncthreads();
+        if (wave == 0)
+            for (int k = 0; k < n_waves && j0 + k < n_blocks; ++k) // :89
+                acc += sums[k][lane];
+        __syncthreads();
+    }
+    if (wave != 0 || s >= p.n_dets)
+        return;
+    if (live)
+        fp_epilogue(p, o, acc);
+    else
+        fp_inactive(p, o);
+}
+
+// out = in^T of an n x n image, 64 x 64 tiles through LDS.
+__global__ __launch_bounds__(256) void k_transpose(const float *__restrict__ in, float *__restrict__ out, int n)
+{
+    __shared__ float t[64][65];
+    const int lx = threadIdx.x & 63, ly = threadIdx.x >> 6;
+    const int x = blockIdx.x * 64 + lx, y0 = blockIdx.y * 64;
+#pragma unroll
+    for (int k = 0; k < 64; k += 4)
+        if (x < n && y0 + ly + k < n)
+            t[ly + k][lx] = in[(size_t)(y0 + ly + k) * n + x];
+    __syncthreads();
+    const int xo = y0 + lx, yo = blockIdx.x * 64;
+#pragma unroll
+    for (int k = 0; k < 64; k += 4)
+        if (xo < n && yo + ly + k < n)
+            out[(size_t)(yo + ly + k) * n + xo] = t[lx][ly + k];
+}
+
+// --------------------------------------------------------------------------
 // The same projection with one wave per ray and the block starts from a table.
 // --------------------------------------------------------------------------
 // A ray's coordinate before sample i is the reference's sequential float walk
@@ -356,24 +476,6 @@ struct BpRefArgs {
 // took 197 us instead of 425 at 1024 / 720 / 1448 and 15 instead of 109 at
 // 256 / 180 / 367.
 constexpr int kBpU = 8;
-
-// A raw buffer load whose byte offset lies at or beyond the resource's size
-// returns zero and touches no memory (negative offsets are large unsigned
-// ones): the zero border of a row.  The offset has to be whole in the vector
-// register, as the check does not see a wrap by an immediate one (opaque).
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t row_rsrc(const float *base, uint32_t elems)
-{
-    return __builtin_amdgcn_make_buffer_rsrc((void *)base, (short)0, (int)(elems * 4u), 0x00020000);
-}
-__device__ __forceinline__ float row_load(__amdgpu_buffer_rsrc_t r, int i)
-{
-    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, (uint32_t)i * 4u, 0, 0));
-}
-__device__ __forceinline__ int opaque(int i)
-{
-    asm("" : "+v"(i));
-    return i;
-}
 
 // floor(x) converted to int in one instruction (no memory access).
 __device__ __forceinline__ int cvt_flr(float x)
@@ -927,6 +1029,31 @@ int uirk_fp_ref_split(const float *vol, const float *r_sino, float *w_sino, cons
     FpRefArgs a{vol, r_sino, w_sino, ray_w, sin_lut, cos_lut, n, n_dets, ang0, n_ang, dir, axis, corr};
     dim3 grid((n_dets + kSplitRays - 1) / kSplitRays, n_ang);
     hipLaunchKernelGGL(k_fp_ref_split, grid, dim3(256), 0, (hipStream_t)stream, a);
+    return (int)hipGetLastError();
+}
+
+int uirk_transpose(const float *in, float *out, int n, void *stream)
+{
+    if (n <= 0)
+        return 0;
+    const unsigned t = (n + 63) / 64;
+    hipLaunchKernelGGL(k_transpose, dim3(t, t), dim3(256), 0, (hipStream_t)stream, in, out, n);
+    return (int)hipGetLastError();
+}
+
+int uirk_fp_blocks(const float *vol, const float *vol_t, const float *r_sino, float *w_sino, const float *ray_w,
+                   const float *sin_lut, const float *cos_lut, int n, int n_dets, float axis, float corr, int ang0,
+                   int n_ang, void *stream)
+{
+    if (n_ang <= 0 || n_dets <= 0)
+        return 0;
+    if (n_ang > 65535)
+        return (int)hipErrorInvalidValue;
+    FpRefArgs a{vol, r_sino, w_sino, ray_w, sin_lut, cos_lut, n, n_dets, ang0, n_ang, -1, axis, corr};
+    const int n_blocks = (n + kBlockSamples - 1) / kBlockSamples;
+    const unsigned waves = n_blocks < 1 ? 1 : (n_blocks < kBlkWaves ? n_blocks : kBlkWaves);
+    hipLaunchKernelGGL(k_fp_blocks, dim3((n_dets + 63) / 64, n_ang), dim3(64 * waves), 0, (hipStream_t)stream, a,
+                       vol_t);
     return (int)hipGetLastError();
 }
 
