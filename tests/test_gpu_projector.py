@@ -104,6 +104,22 @@ def test_bp_bit_exact(res, n, d, a, axis):
     assert np.array_equal(out.numpy(), O.bp(g, sino))
 
 
+@pytest.mark.parametrize("n", [96, 700])
+def test_forward_again_and_with_another_step(res, n):
+    """A forward projector keeps its tables between calls and takes a changed
+    step property at the next one, on both sides of the work table's line."""
+    print("case forward, changed step", n, flush=True)
+    d, a = n, 20
+    x = ellipse_phantom(n, seed=n)
+    steps = [np.float32(np.pi / a), np.float32(np.pi / a), np.float32(0.1)]
+    p = _projector(n, d, a, steps[0], True).setup(res)
+    dx, ds = uir.DeviceArray.from_numpy(x), uir.DeviceArray((a, d))
+    for step in steps:
+        p["step"] = float(step)
+        p.process(dx, ds)
+        assert np.array_equal(ds.numpy(), O.fp(O.Geometry(n, d, a, step), x))
+
+
 def test_luts_and_runs_match_oracle(res):
     a, step = 720, np.float32(np.pi / 720)
     g = O.Geometry(1448, 1448, a, step)

@@ -40,10 +40,11 @@ struct uir_task {
     uint32_t n_dets;
     float *h_sin, *h_cos, *d_sin, *d_cos;
     uint32_t lut_n;
+    float lut_step; /* the step the LUT was built with */
     uir_subset *runs;
     uint32_t n_runs;
     /* FP work table of the table-driven kernel for the current geometry */
-    uint32_t plan_n, plan_dets, plan_angles;
+    uint32_t plan_gen, plan_n, plan_dets, plan_angles;
     float plan_axis;
     uirk_fp_item *d_fp_items;
     int n_fp_items;
@@ -509,6 +510,7 @@ uir_status uir_task_setup(uir_task *t, uir_resources *res)
 
 static uir_status proj_build_luts(uir_task *p, uint32_t n_angles)
 {
+    p->lut_n = 0; /* a build that fails is taken again by the next call */
     free(p->h_sin);
     free(p->h_cos);
     free(p->runs);
@@ -531,6 +533,7 @@ static uir_status proj_build_luts(uir_task *p, uint32_t n_angles)
         HIPTRY(hipStreamSynchronize(st), "LUT upload sync");
     }
     p->lut_n = n_angles;
+    p->lut_step = p->step;
     p->lut_gen++;
     return UIR_OK;
 }
@@ -541,7 +544,9 @@ static uir_status proj_requisition(uir_task *p, const uir_buffer *in, uir_requis
         return uir_set_error(UIR_ERR_INVALID_ARGUMENT, "empty input buffer");
     if (p->angles_num == 0)
         p->angles_num = in->dims[1];
-    if (p->first_run || p->angles_num != in->dims[1] || p->lut_n != p->angles_num) {
+    /* a forward projector's input is the image, whose height is not the angle
+     * count: its LUT is rebuilt only for another count or step */
+    if (p->first_run || p->lut_n != p->angles_num || (p->angles_num != in->dims[1] && p->lut_step != p->step)) {
         p->first_run = 0;
         TRY(proj_build_luts(p, p->angles_num));
     }
@@ -604,8 +609,8 @@ static uir_status proj_plan(uir_task *p, uint32_t n)
 {
     const float axis = proj_axis(p);
     TRY(proj_limits(p, n));
-    if (p->d_fp_items && p->plan_n == n && p->plan_dets == p->n_dets && p->plan_angles == p->lut_n &&
-        p->plan_axis == axis)
+    if (p->d_fp_items && p->plan_gen == p->lut_gen && p->plan_n == n && p->plan_dets == p->n_dets &&
+        p->plan_angles == p->lut_n && p->plan_axis == axis)
         return UIR_OK;
     uir_dfree(p->d_fp_items);
     uir_dfree(p->d_trig);
@@ -643,6 +648,7 @@ static uir_status proj_plan(uir_task *p, uint32_t n)
         uirk_plan_xcd(cost, (int)fv.n, uirk_plan_num_xcd(), &p->fp_part);
         free(cost);
     }
+    p->plan_gen = p->lut_gen;
     p->plan_n = n;
     p->plan_dets = p->n_dets;
     p->plan_angles = p->lut_n;
