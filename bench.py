@@ -200,8 +200,8 @@ def sart_c2(args, uir):
     iterations (30), relaxation 0.5 (the reference-compatible SART task, FP32).
     Beside the time: accuracy against the oracle's FP32 SART (the reference's
     arithmetic) and its FP64 evaluation, the roofline of the per-angle
-    projection kernels (single-angle launches through the kernel-level ABI,
-    the kernels the sweep runs), and the oracle's SART on the host cores."""
+    projection kernels (the sweep's step kernel with its FP and BP apart), and
+    the oracle's SART on the host cores."""
     import oracle as O
     res = uir.Resources(0)
     n, a, d = 1024, 720, 1448
@@ -237,15 +237,17 @@ def sart_c2(args, uir):
     # writes the row; BP reads the row and the image and writes the image
     fp_bytes = n * n * 4 + 2 * d * 4
     bp_bytes = 2 * n * n * 4 + d * 4
-    k = ("k_fp_ref_seg", fp_us, fp_bytes) if fp_us >= bp_us else ("k_bp_ref_angle", bp_us, bp_bytes)
+    k = ("k_sart_ref_step (FP alone)", fp_us, fp_bytes) if fp_us >= bp_us else \
+        ("k_sart_ref_step (BP alone)", bp_us, bp_bytes)
     gbs = k[2] / (k[1] * 1e-6) / 1e9
     roof = {"bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(gbs / HBM_PEAK_GBS, 4), "traffic": None, "kernel": k[0],
             "launch_us": {"fp": round(fp_us, 2), "bp": round(bp_us, 2)},
             "bytes_per_launch": {"fp": fp_bytes, "bp": bp_bytes},
-            "what": "one angle per launch (the sweep's structure, ufo-ir-sart-task.c:208-220): the FP streams "
-                    "the image once, the BP reads and writes it; every launch of one sweep bracketed by "
-                    "events (uir_task_time_kernels), so the figures include each launch's start-up"}
+            "what": "one angle per launch, its FP and BP apart (the sweep joins one angle's BP and the next one's "
+                    "FP in a launch): the FP streams the image once, the BP reads and writes it; every launch of "
+                    "one sweep bracketed by events (uir_task_time_kernels), so the figures include each launch's "
+                    "start-up"}
     print("c2: FP %.2f us, BP %.2f us per angle" % (fp_us, bp_us), file=sys.stderr, flush=True)
 
     # accuracy (full iteration count) and the CPU baseline

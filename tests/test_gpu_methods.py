@@ -76,6 +76,29 @@ def test_sart_bit_exact(res, n, d, a, axis, iters):
     assert np.array_equal(got, ref)
 
 
+@pytest.mark.parametrize("n,d,a,step,axis", [
+    (1, 1, 1, 0.4, -1.0), (2, 3, 2, 1.6, -1.0),
+    (200, 283, 7, 1.3, -1.0),    # one angle far from the next, the direction changing at almost every one
+    (129, 183, 5, 0.79, -1.0),   # a last block of one line
+    (130, 140, 6, 0.9, 61.25),   # pixels beyond the detector, inactive detectors
+    (320, 320, 9, 0.35, -1.0),
+    (64, 91, 6, 0.5, 0.2),       # no active detector
+])
+def test_sart_steps_bit_exact(res, n, d, a, step, axis):
+    """The fused SART step where its regions can go wrong: a BP and an FP at
+    unrelated angles, partial blocks and tiles, clamped and inactive bins, a
+    single angle; two sweeps so that the captured one runs again."""
+    print("case sart steps", n, d, a, step, axis, flush=True)
+    step = np.float32(step)
+    g = O.Geometry(n, d, a, step, axis)
+    b = np.random.default_rng(n * 7 + a).random((a, d)).astype(np.float32)
+    proj = uir.Task("parallel-projector", step=float(step), is_forward=False, image_size=n, axis_position=axis)
+    for iters in (1, 2):
+        m = uir.Task("sart", projector=proj, num_iterations=iters, relaxation_factor=0.5).setup(res)
+        got, _ = _run(m, b, n)
+        assert np.array_equal(got, O.sart(g, b, iters, 0.5), equal_nan=True), iters
+
+
 @pytest.mark.parametrize("df", ["sart", "sirt"])
 def test_asdpocs(res, df):
     n = d = 96

@@ -64,20 +64,25 @@ int uirk_fp_blocks(const float *vol, const float *vol_t, const float *r_sino, fl
                    int n_ang, void *stream);
 
 /* The coordinate at the start of every 64-sample block of every ray of
- * angles [0, n_angles) ([angle][detector][block], ceil(n / 64) blocks), taken
+ * angles [0, n_angles) ([angle][block][detector], ceil(n / 64) blocks), taken
  * by the reference's sequential float walk; inactive rays get 0. */
 int uirk_fp_block_starts(const float *sin_lut, const float *cos_lut, int n, int n_dets, float axis, int n_angles,
                          int dir, float *starts, void *stream);
-/* The same FP as uirk_fp_ref, bit-identical, one wave per ray, from the
- * block-start table of uirk_fp_block_starts (built for the same geometry,
- * direction rule and LUTs). */
-int uirk_fp_ref_seg(const float *vol, const float *r_sino, float *w_sino, const float *ray_w,
-                    const float *sin_lut, const float *cos_lut, int n, int n_dets, float axis,
-                    float corr, int ang0, int n_ang, int dir, const float *starts, void *stream);
-/* BP of one angle in accumulate mode (w = r + relax * BP_ang), bit-identical
- * to uirk_bp_ref with a one-angle run. */
-int uirk_bp_ref_angle(const float *r_vol, float *w_vol, const float *sino, const float *sin_lut,
-                      const float *cos_lut, int n, int n_dets, float axis, float relax, int ang, void *stream);
+/* One step of a SART sweep: x_out = x_in + relax A_bp^T r with r = (b + corr
+ * sum) ray_w of angle bp_ang, the sums being part_in added block by block, and
+ * part_out = the block sums of the FP of angle fp_ang over x_out
+ * ([ceil(n / 64)][n_dets]).  An angle < 0 leaves its half out (no bp_ang:
+ * x_out is not written and the FP is that of x_in).  x_in and x_out are
+ * different buffers unless fp_ang < 0, part_in and part_out always.  trans:
+ * both buffers hold the transposed image; it has to be set if and only if
+ * fp_ang is horizontal (|sin| > |cos|), and may be either without an FP.
+ * starts: uirk_fp_block_starts of the geometry with dir -1, or NULL; sin_h and
+ * cos_h: the LUT in host memory; n_xcd: uirk_plan_num_xcd().
+ * Bit-identical to uirk_fp_ref and uirk_bp_ref of one angle each. */
+int uirk_sart_ref_step(const float *x_in, float *x_out, const float *b, const float *ray_w, const float *starts,
+                       const float *part_in, float *part_out, const float *sin_h, const float *cos_h, int n,
+                       int n_dets, float axis, float corr, float relax, int bp_ang, int fp_ang, int trans,
+                       int n_xcd, void *stream);
 
 /* Reference-compatible BP (projector-parallel-joseph.cl:158-218) over a list of
  * subsets (runs), one per-run accumulation each: w = r + relax * sum_run.

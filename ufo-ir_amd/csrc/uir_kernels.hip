@@ -320,138 +320,6 @@ __global__ __launch_bounds__(256) void k_transpose(const float *__restrict__ in,
 }
 
 // --------------------------------------------------------------------------
-// The same projection with one wave per ray and the block starts from a table.
-// --------------------------------------------------------------------------
-// A ray's coordinate before sample i is the reference's sequential float walk
-// (:82-90): i additions of the step to the start coordinate.  That walk does
-// not depend on the image, so it is taken once per geometry: the table holds,
-// for every ray, the coordinate at the start of each 64-sample block, reached
-// by the same additions (k_fp_block_starts).  A ray's 64-sample blocks then
-// spread over a wave, 16 samples per lane: a lane replays at most 48 additions
-// from its block's start, loads all 32 taps of its samples at once, and the
-// four lanes of a block add their samples into the block sum one after another
-// in sample order (the value passes lane to lane); the block sums are added in
-// block order.  Every sample sees the coordinate the sequential walk sees and
-// every sum is taken in the reference's order: bit-identical to k_fp_ref.
-constexpr int kSegSamples = 16; // samples per lane; 4 lanes per 64-sample block
-
-__global__ __launch_bounds__(256) void k_fp_block_starts(FpRefArgs p, float *__restrict__ starts)
-{
-    const int s = blockIdx.x * 256 + threadIdx.x;
-    const int ang = p.ang0 + blockIdx.y;
-    if (s >= p.n_dets)
-        return;
-    const int N = p.n, n_blocks = (N + kBlockSamples - 1) / kBlockSamples;
-    float pos = 0.0f, step = 0.0f;
-    int dir = 0;
-    float *out = starts + ((size_t)ang * p.n_dets + s) * n_blocks;
-    if (!fp_ray_setup(s, ang, N, p.n_dets, p.axis, p.sin_lut, p.cos_lut, p.dir, pos, step, dir)) {
-        for (int j = 0; j < n_blocks; ++j)
-            out[j] = 0.0f;
-        return;
-    }
-    for (int j = 0; j < n_blocks; ++j) {
-        out[j] = pos;
-#pragma unroll
-        for (int k = 0; k < kBlockSamples; ++k)
-            pos += step;
-    }
-}
-
-__global__ __launch_bounds__(256) void k_fp_ref_seg(FpRefArgs p, const float *__restrict__ starts)
-{
-    const int lane = threadIdx.x & 63;
-    const int s = blockIdx.x * 4 + (threadIdx.x >> 6); // one ray per wave
-    const int ang = p.ang0 + blockIdx.y;
-    if (s >= p.n_dets)
-        return; // uniform over the wave
-    const int N = p.n, n_blocks = (N + kBlockSamples - 1) / kBlockSamples;
-    float pos0 = 0.0f, step = 0.0f;
-    int dir = 0;
-    const size_t o = (size_t)ang * p.n_dets + s;
-    if (!fp_ray_setup(s, ang, N, p.n_dets, p.axis, p.sin_lut, p.cos_lut, p.dir, pos0, step, dir)) {
-        if (lane == 0)
-            fp_inactive(p, o);
-        return;
-    }
-    const float *st = starts + o * n_blocks;
-    const int q = lane & 3; // this lane's quarter of its block
-    // the epilogue's operands, loaded while the samples are taken
-    const float r_in = lane == 0 ? p.r_sino[o] : 0.0f;
-    const float rw_in = (lane == 0 && p.ray_w) ? p.ray_w[o] : 0.0f;
-    float acc = 0.0f;
-    for (int jb0 = 0; jb0 < n_blocks; jb0 += 16) {
-        const int jb = jb0 + (lane >> 2);
-        float pos = jb < n_blocks ? st[jb] : 0.0f;
-#pragma unroll
-        for (int r = 0; r < 3; ++r) {
-            if (r < q) {
-#pragma unroll
-                for (int k = 0; k < kSegSamples; ++k)
-                    pos += step;
-            }
-        }
-        const int i0 = jb * kBlockSamples + kSegSamples * q;
-        float va[kSegSamples], vb[kSegSamples], w[kSegSamples];
-        int c0[kSegSamples];
-#pragma unroll
-        for (int k = 0; k < kSegSamples; ++k) {
-            const int i = min(i0 + k, N - 1); // lanes past the image load a valid address, unused
-            const float v = pos - 0.5f;
-            const float fv = floorf(v);
-            c0[k] = (int)fv;
-            w[k] = v - fv;
-            const int ca = min(max(c0[k], 0), N - 1), cb = min(max(c0[k] + 1, 0), N - 1);
-            const size_t oa = dir == 0 ? (size_t)ca * N + i : (size_t)i * N + ca;
-            const size_t ob = dir == 0 ? (size_t)cb * N + i : (size_t)i * N + cb;
-            va[k] = p.vol[oa];
-            vb[k] = p.vol[ob];
-            pos += step;
-        }
-#pragma unroll
-        for (int k = 0; k < kSegSamples; ++k)
-            asm volatile("" : "+v"(va[k]), "+v"(vb[k]));
-        float val[kSegSamples];
-#pragma unroll
-        for (int k = 0; k < kSegSamples; ++k) {
-            const float t0 = (c0[k] >= 0 && c0[k] < N) ? va[k] : 0.0f;
-            const float t1 = (c0[k] + 1 >= 0 && c0[k] + 1 < N) ? vb[k] : 0.0f;
-            const float omw = 1.0f - w[k];
-            val[k] = omw * t0 + w[k] * t1;
-        }
-        // the block sum, lane q continuing from lane q - 1 (:84-89 order);
-        // the hand-over is a DPP row shift by one lane (lanes of a block
-        // share a row of 16)
-        float run = 0.0f;
-#pragma unroll
-        for (int stage = 0; stage < 4; ++stage) {
-            const float from = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(run), 0x111, 0xf, 0xf, false));
-            if (q == stage) {
-                float a = stage == 0 ? 0.0f : from;
-#pragma unroll
-                for (int k = 0; k < kSegSamples; ++k)
-                    if (i0 + k < N)
-                        a = a + val[k];
-                run = a;
-            }
-        }
-        // block sums in block order (:89)
-#pragma unroll
-        for (int jj = 0; jj < 16; ++jj) {
-            const float bs = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(run), 4 * jj + 3));
-            if (jb0 + jj < n_blocks)
-                acc = acc + bs;
-        }
-    }
-    if (lane == 0) { // fp_epilogue with the prefetched operands (:92-94)
-        float w = r_in + acc * p.corr;
-        if (p.ray_w)
-            w = w * rw_in;
-        p.w_sino[o] = w;
-    }
-}
-
-// --------------------------------------------------------------------------
 // Backprojection, R pixels per thread, per-run accumulation.
 // --------------------------------------------------------------------------
 struct BpRefArgs {
@@ -602,20 +470,97 @@ template <int R> void launch_bp_gather(const BpRefArgs &a, hipStream_t st)
 }
 
 // --------------------------------------------------------------------------
-// Backprojection of one angle, four pixels per thread (SART's per-angle BP).
+// SART: the BP of one angle and the FP of the next in one launch
 // --------------------------------------------------------------------------
-// The arithmetic of k_bp_ref with one run of one angle (:196-216) in
-// accumulate mode: w = r + relax * (0 + lerp).  Row-aligned buffers (N a
-// multiple of 4, 16-byte aligned pointers) move four pixels per load and
-// store.
-template <bool VEC>
-__global__ __launch_bounds__(256) void k_bp_ref_angle(BpRefArgs p, int ang)
+// SART alternates the FP of one angle and the BP of its weighted residual into
+// the image, so each launch waits for the one before and is short: what bounds
+// a sweep is the chain of launches and, within each, of dependent loads and of
+// instruction fetches (a launch starts with cold instruction caches, and a
+// kilobyte of straight code costs about 0.6 us).  So one launch here applies
+// the BP of angle bp_ang to the image, from x_in to the other buffer x_out, and
+// takes the block sums of the FP of angle fp_ang of that updated image, which
+// it forms on the fly from x_in, and many short waves of little code do it.
+// Two kinds of workgroups share the launch and nothing else:
+//   FP: 64 detectors (lanes) x one 64-sample block, kSeg samples to each wave.
+//       A wave replays at most 60 additions of the step from the block's start, its taps are neighbours on a line, and every tap gets
+//       its BP update by the operations the BP workgroups use; the samples
+//       meet in LDS and one wave adds them in order (:82-90).  The block sum
+//       goes to part_out[block][detector].
+//   BP: a tile of 64 x 64 pixels, kSeg per thread, x_out = x_in + relax BP (:196-216).
+// Both first form the residuals of the bins they need in LDS: the previous
+// launch's block sums added in block order, then (b + corr sum) R (:89-94).
+// The image is held transposed while the angles are horizontal (FP_hor), so
+// that rays always walk its rows.  Every operation and its order is the
+// reference's: bit-identical to k_fp_ref and k_bp_gather angle by angle.
+// A separate FP and BP per angle, the FP gathering along columns for half of
+// the angles, took 11.8 + 7.1 us an angle at 1024 x 1024 / 1448 bins, this
+// takes 7.3 (of them 1.6 for an empty launch, 1.8 to fetch the image, 2.4 for
+// the updates); 5.1 + 2.4 and 4.5 at 128 x 128.
+// Bins a workgroup touches: an FP's 64 rays cover at most 63 sqrt(2) + 63 = 153
+// positions of 64 lines, and its region takes a margin on each side that covers
+// the drift of the float stepping (N additions, each off by at most N 2^-24
+// inside the image), 66 positions for the largest image of 4 GiB: 285 positions
+// x 64 lines are 292 bins apart.  A BP tile needs 90.
+constexpr int kSartBins = 320;
+constexpr int kSeg = 8; // samples or pixels per thread (4 and 16 are slower by up to 0.3 and 1.3 us)
+constexpr int kSartThreads = 4096 / kSeg, kSartWaves = kSartThreads / 64;
+
+struct SartStepArgs {
+    const float *x_in;
+    float *x_out;
+    const float *b, *ray_w;  // rows of angle bp_ang
+    const float *starts;     // of angle fp_ang, [block][detector], or NULL: replay the stepping
+    const float *part_in;
+    float *part_out;         // [block][detector]
+    int n, n_dets;
+    int bp, trans;           // bp: apply the BP; trans: the buffers hold the transposed image
+    int n_fp, n_bp;          // FP and BP workgroups per band of 64 lines
+    int n_xcd;
+    float axis, corr, relax;
+    float kp, kl;            // BP: u = (fP kp - fL kl) + shift at position P of line L
+    float det_step, step;    // FP
+};
+
+// The coordinate at the start of every 64-sample block of every ray of angles
+// [0, n_angles), [angle][block][detector], by the reference's sequential walk
+// (:82-90), which does not depend on the image; inactive rays get 0.
+__global__ __launch_bounds__(256) void k_fp_block_starts(FpRefArgs p, float *__restrict__ starts)
 {
-    const int px0 = (blockIdx.x * 64 + threadIdx.x) * 4;
-    const int py = blockIdx.y * 4 + threadIdx.y;
-    const int N = p.n, D = p.n_dets;
-    if (px0 >= N || py >= N)
+    const int s = blockIdx.x * 256 + threadIdx.x;
+    const int ang = p.ang0 + blockIdx.y;
+    if (s >= p.n_dets)
         return;
+    const int N = p.n, n_blocks = (N + kBlockSamples - 1) / kBlockSamples;
+    float pos = 0.0f, step = 0.0f;
+    int dir = 0;
+    float *out = starts + (size_t)ang * n_blocks * p.n_dets + s;
+    const bool live = fp_ray_setup(s, ang, N, p.n_dets, p.axis, p.sin_lut, p.cos_lut, p.dir, pos, step, dir);
+    for (int j = 0; j < n_blocks; ++j) {
+        out[(size_t)j * p.n_dets] = live ? pos : 0.0f;
+#pragma unroll
+        for (int k = 0; k < kBlockSamples; ++k)
+            pos += step;
+    }
+}
+
+// WINDOW: edge0 <= edge1 (an axis with active detectors): the clamp is a median.
+template <bool WINDOW> __global__ __launch_bounds__(kSartThreads) void k_sart_ref_step(SartStepArgs p)
+{
+    __shared__ float row[kSartBins];
+    __shared__ float samples[kBlockSamples][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int N = p.n, D = p.n_dets;
+    const int n_blocks = (N + kBlockSamples - 1) / kBlockSamples;
+    // a band's workgroups, FP and BP, run on one XCD (workgroup g on XCD g mod
+    // n_xcd), in this launch and the next: its L2 holds the band's pixels
+    const uint32_t turn = blockIdx.x / (uint32_t)p.n_xcd, per_band = (uint32_t)(p.n_fp + p.n_bp);
+    const int band = (int)((blockIdx.x - turn * (uint32_t)p.n_xcd) + (turn / per_band) * (uint32_t)p.n_xcd);
+    const int item = (int)(turn % per_band);
+    if (band * 64 >= p.n)
+        return;
+    const bool fp = item < p.n_fp; // uniform
+    const int at = fp ? item : item - p.n_fp;
+
     // projector-parallel-joseph.cl:174-190 (detector quantities use n_dets)
     const float required_width = p.axis * 2;
     const float diff = (float)D - required_width;
@@ -623,50 +568,162 @@ __global__ __launch_bounds__(256) void k_bp_ref_angle(BpRefArgs p, int ang)
     const float edge0 = p.axis - half_active + 0.5f;
     const float edge1 = p.axis + half_active - 0.5f;
     const float rot = diff / 2.0f;
-    const float det_shift = (float)D / 2.0f;
     const float origin_shift = (float)N / 2.0f;
-    const float shift = det_shift - rot;
-    const float fY = (float)py + 0.5f - origin_shift;
-    const float st = p.sin_lut[ang], ct = p.cos_lut[ang];
-    const float *row = p.sino + (size_t)ang * D;
-    const size_t o = (size_t)py * N + px0;
-    float in[4];
-    if (VEC) {
-        const float4 v = *(const float4 *)(p.r_vol + o);
-        in[0] = v.x, in[1] = v.y, in[2] = v.z, in[3] = v.w;
+    const float shift = (float)D / 2.0f - rot;
+
+    // this workgroup's lines [l0, l1) and positions [c_lo, c_hi] of the image
+    const int l0 = band * 64, l1 = min(N, l0 + 64);
+    float c_lo = (float)(at * 64), c_hi = fminf(c_lo + 63.0f, (float)(N - 1));
+
+    // the image values first: their loads overlap the residuals' below
+    float va[kSeg], vb[kSeg], fv[kSeg], w[kSeg];
+    const int s = at * 64 + lane;                                    // FP: this lane's ray; BP: its position
+    const int i0 = fp ? l0 + kSeg * wave : l0 + wave;         // this wave's first line
+    bool live = false;
+    if (fp) {
+        live = s < D && !((diff < 0 && (float)s < fabsf(diff)) || (diff > 0 && (float)s > required_width)); // :63-66
+        float pos = 0.0f;
+        const float step = p.step;
+        if (p.starts) {
+            if (live)
+                pos = p.starts[(size_t)band * D + s];
+        } else {
+            const double t = ((0.5 + (double)rot) + (double)s) - (double)(0.5f * (float)D); // :73, :134
+            pos = (float)(t * (double)p.det_step + (double)((-origin_shift) * step) + (double)(0.5f * (float)N));
+#pragma unroll 8
+            for (int k = 0; k < l0; ++k)
+                pos += step;
+        }
+        // the region: the positions of the first and last ray on the first and
+        // last line, and a margin
+        const float pa = ((float)(at * 64) + 0.5f - p.axis) * p.det_step + (0.5f * (float)N + ((float)l0 - 0.5f * (float)N) * step);
+        const float pb = pa + 63.0f * p.det_step, dl = 63.0f * step;
+        const float margin = 2.0f + ceilf((float)N * (float)N * 0x1p-24f);
+        c_lo = fminf(fmaxf(floorf(fminf(pa, pb) + fminf(dl, 0.0f)) - margin, 0.0f), (float)(N - 1));
+        c_hi = fmaxf(fminf(floorf(fmaxf(pa, pb) + fmaxf(dl, 0.0f)) + margin, (float)(N - 1)), c_lo);
+#pragma unroll 1
+        for (int r = 0; r < wave; ++r) {
+#pragma unroll
+            for (int k = 0; k < kSeg; ++k)
+                pos += step;
+        }
+#pragma unroll
+        for (int k = 0; k < kSeg; ++k) {
+            const float v = pos - 0.5f;
+            fv[k] = floorf(v);
+            w[k] = v - fv[k];
+            const int line = i0 + k, c = (int)fv[k];
+            const __amdgpu_buffer_rsrc_t r = row_rsrc(p.x_in + (size_t)line * N, line < N ? (uint32_t)N : 0u);
+            va[k] = row_load(r, c);
+            vb[k] = row_load(r, opaque(c + 1));
+            pos += step;
+        }
     } else {
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
-            in[k] = px0 + k < N ? p.r_vol[o + k] : 0.0f;
+        for (int k = 0; k < kSeg; ++k) {
+            const int line = i0 + kSartWaves * k;
+            va[k] = row_load(row_rsrc(p.x_in + (size_t)line * N, line < N ? (uint32_t)N : 0u), s);
+        }
     }
-    float out[4];
+
+    // residuals of the bins under the region
+    int umin = 0;
+    if (p.bp) {
+        const float cx0 = (c_lo + 0.5f - origin_shift) * p.kp, cx1 = (c_hi + 0.5f - origin_shift) * p.kp;
+        const float cy0 = ((float)l0 + 0.5f - origin_shift) * p.kl, cy1 = ((float)(l1 - 1) + 0.5f - origin_shift) * p.kl;
+        float umn = (fminf(cx0, cx1) - fmaxf(cy0, cy1)) + shift, umx = (fmaxf(cx0, cx1) - fminf(cy0, cy1)) + shift;
+        const float e_lo = fminf(edge0, edge1), e_hi = fmaxf(edge0, edge1);
+        umn = fminf(fmaxf(umn, e_lo), e_hi);
+        umx = WINDOW ? fminf(fmaxf(umx, e_lo), e_hi) : e_hi;
+        if (!WINDOW)
+            umn = e_lo;
+        umin = (int)floorf(umn - 0.5f) - 2;
+        const int width = min((int)(umx - umn) + 6, kSartBins);
+        for (int e0 = threadIdx.x; e0 < width; e0 += kSartThreads) {
+            const int bin = umin + e0;
+            float r = 0.0f;
+            if (bin >= 0 && bin < D) {
+                r = p.b[bin];
+                const float rw = p.ray_w[bin];
+                float acc = 0.0f;
+#pragma unroll 1
+                for (int j = 0; j < n_blocks; j += 8) {
+                    float v[8];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const float fX = (float)(px0 + k) + 0.5f - origin_shift;
-        float u = fX * ct - fY * st + shift;
-        if (u > edge1)
-            u = edge1;
-        else if (u < edge0)
-            u = edge0;
-        const float w = u - 0.5f;
-        const float fw = floorf(w);
-        const int i0 = (int)fw;
-        const float a = w - fw;
+                    for (int e = 0; e < 8; ++e)
+                        v[e] = j + e < n_blocks ? p.part_in[(size_t)(j + e) * D + bin] : 0.0f;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        acc = acc + v[e]; // :89 (the sum is never -0: adding 0 past the last block keeps it)
+                }
+                if (!((diff < 0 && (float)bin < fabsf(diff)) || (diff > 0 && (float)bin > required_width)))
+                    r = r + acc * p.corr; // :92-94
+                r = r * rw;
+            }
+            row[e0] = r;
+        }
+        __syncthreads();
+    }
+    auto update = [&](float x, float fP, float lineterm) { // :196-216
+        float u = (fP * p.kp - lineterm) + shift;
+        if (WINDOW) {
+            u = __builtin_amdgcn_fmed3f(u, edge0, edge1);
+        } else {
+            if (u > edge1)
+                u = edge1;
+            else if (u < edge0)
+                u = edge0;
+        }
+        const float v = u - 0.5f;
+        const float f = floorf(v);
+        // a tap outside the region is not used: any entry of the row
+        const int b0 = (int)min((uint32_t)((int)f - umin), (uint32_t)(kSartBins - 2));
+        const float a = v - f;
         const float oma = 1.0f - a;
-        const float t0 = (i0 >= 0 && i0 < D) ? row[i0] : 0.0f;
-        const float t1 = (i0 + 1 >= 0 && i0 + 1 < D) ? row[i0 + 1] : 0.0f;
-        float value = 0.0f;
-        value += oma * t0 + a * t1;
-        out[k] = in[k] + p.relax * value; // :216
-    }
-    if (VEC) {
-        *(float4 *)(p.w_vol + o) = make_float4(out[0], out[1], out[2], out[3]);
-    } else {
+        // (the reference adds the sample to 0 first, which only turns a -0 into
+        // +0: no difference to x, which is never -0)
+        return x + p.relax * (oma * row[b0] + a * row[b0 + 1]);
+    };
+
+    if (!fp) {
+        const float fP = (float)s + 0.5f - origin_shift;
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
-            if (px0 + k < N)
-                p.w_vol[o + k] = out[k];
+        for (int k = 0; k < kSeg; ++k) {
+            const int line = i0 + kSartWaves * k;
+            if (s < N && line < N)
+                p.x_out[(size_t)line * N + s] = update(va[k], fP, ((float)line + 0.5f - origin_shift) * p.kl);
+        }
+        return;
     }
+
+#pragma unroll
+    for (int k = 0; k < kSeg; ++k) {
+        float t0 = va[k], t1 = vb[k];
+        if (p.bp) {
+            const float lt = ((float)(i0 + k) + 0.5f - origin_shift) * p.kl;
+            const float fP = fv[k] + (0.5f - origin_shift); // half-integers: exact in any order
+            const float ta = update(t0, fP, lt);
+            const float tb = update(t1, fP + 1.0f, lt);
+            t0 = fv[k] >= 0.0f && fv[k] < (float)N ? ta : 0.0f;
+            t1 = fv[k] >= -1.0f && fv[k] < (float)(N - 1) ? tb : 0.0f;
+        }
+        const float omw = 1.0f - w[k];
+        samples[kSeg * wave + k][lane] = omw * t0 + w[k] * t1;
+    }
+    __syncthreads();
+    if (wave != 0)
+        return;
+    float run = 0.0f;
+    int k = 0;
+    for (; k + 8 <= l1 - l0; k += 8) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            run = run + samples[k + e][lane];
+    }
+    for (; k < l1 - l0; ++k)
+        run = run + samples[k][lane];
+    if (s < D)
+        p.part_out[(size_t)band * D + s] = live ? run : 0.0f;
 }
 
 // --------------------------------------------------------------------------
@@ -1068,40 +1125,51 @@ int uirk_fp_block_starts(const float *sin_lut, const float *cos_lut, int n, int 
     return (int)hipGetLastError();
 }
 
-int uirk_fp_ref_seg(const float *vol, const float *r_sino, float *w_sino, const float *ray_w,
-                    const float *sin_lut, const float *cos_lut, int n, int n_dets, float axis,
-                    float corr, int ang0, int n_ang, int dir, const float *starts, void *stream)
+int uirk_sart_ref_step(const float *x_in, float *x_out, const float *b, const float *ray_w, const float *starts,
+                       const float *part_in, float *part_out, const float *sin_h, const float *cos_h, int n,
+                       int n_dets, float axis, float corr, float relax, int bp_ang, int fp_ang, int trans,
+                       int n_xcd, void *stream)
 {
-    if (n_ang <= 0 || n_dets <= 0)
+    if (n <= 0 || n_dets <= 0)
         return 0;
-    FpRefArgs a{vol, r_sino, w_sino, ray_w, sin_lut, cos_lut, n, n_dets, ang0, n_ang, dir, axis, corr};
-    dim3 grid((n_dets + 3) / 4, n_ang);
-    hipLaunchKernelGGL(k_fp_ref_seg, grid, dim3(256), 0, (hipStream_t)stream, a, starts);
-    return (int)hipGetLastError();
-}
-
-int uirk_bp_ref_angle(const float *r_vol, float *w_vol, const float *sino, const float *sin_lut,
-                      const float *cos_lut, int n, int n_dets, float axis, float relax, int ang, void *stream)
-{
-    if (n <= 0)
-        return 0;
-    BpRefArgs a;
-    memset(&a, 0, sizeof a);
-    a.r_vol = r_vol;
-    a.w_vol = w_vol;
-    a.sino = sino;
-    a.sin_lut = sin_lut;
-    a.cos_lut = cos_lut;
+    const int nt = (n + 63) / 64; // blocks and tiles are both 64 lines
+    SartStepArgs a{};
+    a.x_in = x_in;
+    a.x_out = x_out;
+    a.part_in = part_in;
+    a.part_out = part_out;
     a.n = n;
     a.n_dets = n_dets;
+    a.bp = bp_ang >= 0;
+    a.trans = trans;
+    a.n_bp = bp_ang >= 0 ? nt : 0;
+    a.n_xcd = n_xcd > 0 ? n_xcd : 1;
     a.axis = axis;
+    a.corr = corr;
     a.relax = relax;
-    dim3 block(64, 4), grid((n + 255) / 256, (n + 3) / 4);
-    const bool vec = (n & 3) == 0 && (((uintptr_t)r_vol | (uintptr_t)w_vol) & 15) == 0;
-    if (vec)
-        hipLaunchKernelGGL(k_bp_ref_angle<true>, grid, block, 0, (hipStream_t)stream, a, ang);
+    if (bp_ang >= 0) {
+        a.b = b + (size_t)bp_ang * n_dets;
+        a.ray_w = ray_w + (size_t)bp_ang * n_dets;
+        // X cos - Y sin with X, Y = P, L or, transposed, L, P (the signs go with the factors)
+        a.kp = trans ? -sin_h[bp_ang] : cos_h[bp_ang];
+        a.kl = trans ? -cos_h[bp_ang] : sin_h[bp_ang];
+    }
+    if (fp_ang >= 0) {
+        const float st = sin_h[fp_ang], ct = cos_h[fp_ang];
+        a.starts = starts ? starts + (size_t)fp_ang * nt * n_dets : nullptr;
+        a.det_step = trans ? -1.0f / st : 1.0f / ct; // :51-75 / :112-136
+        a.step = trans ? ct / st : st / ct;
+        a.n_fp = (n_dets + 63) / 64;
+    }
+    const int grid = a.n_xcd * ((nt + a.n_xcd - 1) / a.n_xcd) * (a.n_fp + a.n_bp);
+    if (grid <= 0)
+        return 0;
+    const float half = (float)n_dets - axis * 2 < 0 ? (float)n_dets - axis : axis;
+    const bool window = axis - half + 0.5f <= axis + half - 0.5f;
+    if (window)
+        hipLaunchKernelGGL(k_sart_ref_step<true>, dim3(grid), dim3(kSartThreads), 0, (hipStream_t)stream, a);
     else
-        hipLaunchKernelGGL(k_bp_ref_angle<false>, grid, block, 0, (hipStream_t)stream, a, ang);
+        hipLaunchKernelGGL(k_sart_ref_step<false>, dim3(grid), dim3(kSartThreads), 0, (hipStream_t)stream, a);
     return (int)hipGetLastError();
 }
 

@@ -25,6 +25,12 @@ typedef enum { P_FLOAT = UIR_PROP_FLOAT, P_UINT = UIR_PROP_UINT, P_BOOL = UIR_PR
 
 #define N_TMP 32
 
+typedef struct {
+    const void *x, *b, *t0, *t1, *part, *sino_tmp, *ray_w, *starts, *sin, *cos, *line;
+    uint32_t n, D, A, lut_gen;
+    float axis, relax, corr;
+} sart_graph_key;
+
 struct uir_task {
     int refcount;
     task_kind kind;
@@ -87,11 +93,7 @@ struct uir_task {
     /* one SART sweep captured as a hipGraph, valid for sart_key */
     hipGraph_t sart_graph;
     hipGraphExec_t sart_exec;
-    struct {
-        const void *x, *b, *tmp, *ray_w, *sin, *cos, *starts, *line;
-        uint32_t n, D, A;
-        float axis, relax, corr;
-    } sart_key;
+    sart_graph_key sart_key;
 };
 
 typedef struct {
@@ -1119,48 +1121,83 @@ static uir_status sirt_run(uir_task *t, const float *b, float *x, float relax, u
 }
 
 /* SART process, ufo-ir-sart-task.c:173-228: per angle, FP of the row with the
- * ray weighting fused (subset_fp + op_mulRows), then BP of that row into x. */
-/* One SART sweep (ufo-ir-sart-task.c:208-220): per angle in order, FP of that
- * angle with the residual and ray weights fused (w = (b - A_a x) R_a), then
- * its BP x = x + relax A_a^T w.  One angle is only n_dets rays, so the FP
- * gives each ray a wave, starting its 64-sample blocks from the geometry's
- * block-start table (starts; without one, 16 threads per ray replay the float
- * stepping); both are bit-identical to the one-thread-per-ray walk.  The BP
- * takes four pixels per thread. */
-static uir_status sart_fp_angle(mctx *c, const float *x, float *sino_tmp, const float *ray_w, float axis,
-                                const float *starts, uint32_t a)
+ * ray weighting fused (subset_fp + op_mulRows, w = (b - A_a x) R_a), then BP of
+ * that row into x (x = x + relax A_a^T w). */
+typedef struct {
+    float *ray_w;     /* R = inv(FP(1)) */
+    float axis;
+    /* joseph: two images that the steps go back and forth between, the block
+     * sums of two angles, and the FP block-start table (may be NULL) */
+    float *t[2], *part[2], *starts;
+    float *sino_tmp;  /* line model: the residual rows */
+} sart_prep;
+
+static int sart_horizontal(const uir_task *p, uint32_t a) { return !(fabsf(p->h_sin[a]) <= fabsf(p->h_cos[a])); }
+
+static uir_status sart_step(mctx *c, const sart_prep *sp, const float *b, const float *x_in, float *x_out, int pi,
+                            int bp, int fp, int trans)
 {
     uir_task *p = c->p;
-    if (p->line) /* the line model: each ray over 16 lanes */
-        return uir_check_hip(uirk_fp_line(x, sino_tmp, sino_tmp, ray_w, p->d_line, p->h_line[a].family, (int)c->n,
-                                          (int)c->D, (int)a, 1, p->correction_scale, 1, c->st), "FP launch");
-    if (starts)
-        return uir_check_hip(uirk_fp_ref_seg(x, sino_tmp, sino_tmp, ray_w, p->d_sin, p->d_cos, (int)c->n, (int)c->D,
-                                             axis, p->correction_scale, (int)a, 1, -1, starts, c->st), "FP launch");
-    return uir_check_hip(uirk_fp_ref_split(x, sino_tmp, sino_tmp, ray_w, p->d_sin, p->d_cos, (int)c->n, (int)c->D,
-                                           axis, p->correction_scale, (int)a, 1, -1, c->st), "FP launch");
+    return uir_check_hip(uirk_sart_ref_step(x_in, x_out, b, sp->ray_w, sp->starts, sp->part[pi], sp->part[!pi], p->h_sin,
+                                            p->h_cos, (int)c->n, (int)c->D, sp->axis, p->correction_scale,
+                                            p->relaxation, bp, fp, trans, uirk_plan_num_xcd(), c->st),
+                         "SART step launch");
 }
 
-static uir_status sart_bp_angle(mctx *c, float *x, const float *sino_tmp, float axis, uint32_t a)
+/* The line model's angle: FP of the row, each ray over 16 lanes, and its BP. */
+static uir_status sart_line_fp(mctx *c, const float *x, float *sino_tmp, const float *ray_w, uint32_t a)
 {
     uir_task *p = c->p;
-    if (p->line)
-        return uir_check_hip(uirk_bp_line(x, x, sino_tmp, NULL, 0, p->d_line, (int)c->n, (int)c->D, (int)a, 1,
-                                          p->relaxation, c->st), "BP launch");
-    return uir_check_hip(uirk_bp_ref_angle(x, x, sino_tmp, p->d_sin, p->d_cos, (int)c->n, (int)c->D, axis,
-                                           p->relaxation, (int)a, c->st), "BP launch");
+    return uir_check_hip(uirk_fp_line(x, sino_tmp, sino_tmp, ray_w, p->d_line, p->h_line[a].family, (int)c->n,
+                                      (int)c->D, (int)a, 1, p->correction_scale, 1, c->st), "FP launch");
 }
 
-static uir_status sart_sweep(uir_task *t, mctx *c, const float *b, float *x, float *sino_tmp, const float *ray_w,
-                             float axis, const float *starts)
+static uir_status sart_line_bp(mctx *c, float *x, const float *sino_tmp, uint32_t a)
 {
-    HIPTRY(hipMemcpyAsync(sino_tmp, b, c->ns * 4, hipMemcpyDeviceToDevice, c->st), "copy");
-    for (uint32_t a = 0; a < c->A; ++a) {
-        TRY(sart_fp_angle(c, x, sino_tmp, ray_w, axis, starts, a));
-        TRY(sart_bp_angle(c, x, sino_tmp, axis, a));
+    uir_task *p = c->p;
+    return uir_check_hip(uirk_bp_line(x, x, sino_tmp, NULL, 0, p->d_line, (int)c->n, (int)c->D, (int)a, 1,
+                                      p->relaxation, c->st), "BP launch");
+}
+
+/* One sweep (:208-220).  Joseph: step a applies the BP of angle a - 1 and sums
+ * the FP of angle a, the image going back and forth between two buffers and
+ * turned over where the angles' direction changes; a last step applies the BP
+ * of the last angle into x. */
+static uir_status sart_sweep(mctx *c, const sart_prep *sp, const float *b, float *x)
+{
+    uir_task *p = c->p;
+    if (p->line) {
+        HIPTRY(hipMemcpyAsync(sp->sino_tmp, b, c->ns * 4, hipMemcpyDeviceToDevice, c->st), "copy");
+        for (uint32_t a = 0; a < c->A; ++a) {
+            TRY(sart_line_fp(c, x, sp->sino_tmp, sp->ray_w, a));
+            TRY(sart_line_bp(c, x, sp->sino_tmp, a));
+        }
+        return UIR_OK;
     }
-    (void)t;
-    return UIR_OK;
+    const float *cur = x;
+    int trans = 0, pi = 0;
+#define OTHER (cur == sp->t[0] ? sp->t[1] : sp->t[0])
+    for (uint32_t a = 0; a < c->A; ++a) {
+        const int hor = sart_horizontal(p, a);
+        if (hor != trans) {
+            float *turned = OTHER;
+            HIPTRY(uirk_transpose(cur, turned, (int)c->n, c->st), "transpose");
+            cur = turned;
+            trans = hor;
+        }
+        float *next = OTHER;
+        TRY(sart_step(c, sp, b, cur, next, pi, (int)a - 1, (int)a, trans));
+        if (a)
+            cur = next;
+        pi = !pi;
+    }
+    if (trans) {
+        float *turned = OTHER;
+        HIPTRY(uirk_transpose(cur, turned, (int)c->n, c->st), "transpose");
+        cur = turned;
+    }
+#undef OTHER
+    return sart_step(c, sp, b, cur, x, pi, (int)c->A - 1, -1, 0);
 }
 
 /* Bytes of the FP block-start table of a geometry; tables above this bound
@@ -1170,30 +1207,32 @@ static uir_status sart_sweep(uir_task *t, mctx *c, const float *b, float *x, flo
 /* SART set-up (ufo-ir-sart-task.c:193-207): ray weights R = inv(FP(1)) per
  * angle, corr = -1, relax = relaxation, x = 0 (unless warm); with `table`,
  * also the FP block-start table of the geometry. */
-typedef struct {
-    float *sino_tmp, *ray_w, *starts;
-    float axis;
-} sart_prep;
-
 static uir_status sart_prepare(uir_task *t, float *x, float relax, int warm, int table, mctx *c, sart_prep *sp)
 {
-    float *vol_tmp;
-    TRY(tmp_get(t, 4, c->ns * 4, &sp->sino_tmp));
-    TRY(tmp_get(t, 5, c->nv * 4, &vol_tmp));
+    memset(sp, 0, sizeof *sp);
+    const size_t blocks = (c->n + 63) / 64;
+    TRY(tmp_get(t, 5, c->nv * 4, &sp->t[0]));
     TRY(tmp_get(t, 6, c->ns * 4, &sp->ray_w));
-    HIPTRY(uirk_set(vol_tmp, c->nv, 1.0f, c->st), "set");          /* :193-200 */
+    if (c->p->line) {
+        TRY(tmp_get(t, 4, c->ns * 4, &sp->sino_tmp));
+    } else {
+        TRY(tmp_get(t, 4, c->nv * 4, &sp->t[1]));
+        TRY(tmp_get(t, 26, 2 * blocks * c->D * 4, &sp->part[0]));
+        sp->part[1] = sp->part[0] + blocks * c->D;
+    }
+    float *ones = sp->t[0];
+    HIPTRY(uirk_set(ones, c->nv, 1.0f, c->st), "set");              /* :193-200 */
     HIPTRY(uirk_set(sp->ray_w, c->ns, 0.0f, c->st), "set");
     c->p->correction_scale = 1.0f;
-    TRY(proj_fp(c->p, c->n, vol_tmp, sp->ray_w, sp->ray_w, NULL));
+    TRY(proj_fp(c->p, c->n, ones, sp->ray_w, sp->ray_w, NULL));
     HIPTRY(uirk_inv(sp->ray_w, sp->ray_w, c->ns, c->st), "inv");
     c->p->correction_scale = -1.0f;                                 /* :205-207 */
     c->p->relaxation = relax;
     if (!warm)
         HIPTRY(uirk_set(x, c->nv, 0.0f, c->st), "set");
     sp->axis = proj_axis(c->p);
-    sp->starts = NULL;
     /* the rays' block starts: the float stepping taken once per call */
-    const size_t starts_bytes = (size_t)c->A * c->D * ((c->n + 63) / 64) * 4;
+    const size_t starts_bytes = (size_t)c->A * c->D * blocks * 4;
     if (c->p->line) /* the line model's table, built by the FP above */
         TRY(line_plan(c->p, c->n));
     else if (table && starts_bytes <= SART_STARTS_MAX_BYTES) {
@@ -1211,17 +1250,18 @@ static uir_status sart_run(uir_task *t, const float *b, float *x, float relax, u
     TRY(sart_prepare(t, x, relax, warm, iters > 0, c, &sp));
     if (iters == 0)
         return UIR_OK;
-    float *sino_tmp = sp.sino_tmp, *ray_w = sp.ray_w, *starts = sp.starts;
-    const float axis = sp.axis;
-    /* 2 A launches per sweep: capture one sweep and replay it (:208-220) */
-    const int same = t->sart_exec && t->sart_key.x == x && t->sart_key.b == b && t->sart_key.tmp == sino_tmp &&
-                     t->sart_key.starts == starts && t->sart_key.line == (c->p->line ? c->p->d_line : NULL) &&
-                     t->sart_key.ray_w == ray_w && t->sart_key.sin == c->p->d_sin && t->sart_key.cos == c->p->d_cos &&
-                     t->sart_key.n == c->n && t->sart_key.D == c->D && t->sart_key.A == c->A &&
-                     t->sart_key.axis == axis && t->sart_key.relax == c->p->relaxation &&
-                     t->sart_key.corr == c->p->correction_scale;
+    /* a launch per angle and more: capture one sweep and replay it (:208-220) */
+    const sart_graph_key key = {x, b, sp.t[0], sp.t[1], sp.part[0], sp.sino_tmp, sp.ray_w, sp.starts, c->p->d_sin,
+                                c->p->d_cos, c->p->line ? c->p->d_line : NULL, c->n, c->D, c->A, c->p->lut_gen,
+                                sp.axis, c->p->relaxation, c->p->correction_scale};
+    const sart_graph_key *k = &t->sart_key;
+    const int same = t->sart_exec && k->x == key.x && k->b == key.b && k->t0 == key.t0 && k->t1 == key.t1 &&
+                     k->part == key.part && k->sino_tmp == key.sino_tmp && k->ray_w == key.ray_w &&
+                     k->starts == key.starts && k->sin == key.sin && k->cos == key.cos && k->line == key.line &&
+                     k->n == key.n && k->D == key.D && k->A == key.A && k->lut_gen == key.lut_gen &&
+                     k->axis == key.axis && k->relax == key.relax && k->corr == key.corr;
     if (!same && iters == 1) /* a capture pays off from the second replay on */
-        return sart_sweep(t, c, b, x, sino_tmp, ray_w, axis, starts);
+        return sart_sweep(c, &sp, b, x);
     if (!same) {
         if (t->sart_exec)
             (void)hipGraphExecDestroy(t->sart_exec);
@@ -1230,7 +1270,7 @@ static uir_status sart_run(uir_task *t, const float *b, float *x, float relax, u
         t->sart_exec = NULL;
         t->sart_graph = NULL;
         HIPTRY(hipStreamBeginCapture(c->st, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
-        uir_status s = sart_sweep(t, c, b, x, sino_tmp, ray_w, axis, starts);
+        uir_status s = sart_sweep(c, &sp, b, x);
         hipGraph_t g = NULL;
         const int e = hipStreamEndCapture(c->st, &g);
         if (s != UIR_OK || e != hipSuccess) {
@@ -1240,20 +1280,7 @@ static uir_status sart_run(uir_task *t, const float *b, float *x, float relax, u
         }
         t->sart_graph = g;
         HIPTRY(hipGraphInstantiate(&t->sart_exec, g, NULL, NULL, 0), "hipGraphInstantiate");
-        t->sart_key.x = x;
-        t->sart_key.b = b;
-        t->sart_key.tmp = sino_tmp;
-        t->sart_key.starts = starts;
-        t->sart_key.line = c->p->line ? c->p->d_line : NULL;
-        t->sart_key.ray_w = ray_w;
-        t->sart_key.sin = c->p->d_sin;
-        t->sart_key.cos = c->p->d_cos;
-        t->sart_key.n = c->n;
-        t->sart_key.D = c->D;
-        t->sart_key.A = c->A;
-        t->sart_key.axis = axis;
-        t->sart_key.relax = c->p->relaxation;
-        t->sart_key.corr = c->p->correction_scale;
+        t->sart_key = key;
     }
     for (uint32_t it = 0; it < iters; ++it)
         HIPTRY(hipGraphLaunch(t->sart_exec, c->st), "hipGraphLaunch");
@@ -1658,25 +1685,30 @@ uir_status uir_task_time_kernels(uir_task *t, const uir_buffer *inputs, uir_buff
     float *x = (float *)output->data;
     sart_prep sp;
     TRY(sart_prepare(t, x, t->relaxation_factor, 0, 1, &c, &sp));
-    HIPTRY(hipMemcpyAsync(sp.sino_tmp, b, c.ns * 4, hipMemcpyDeviceToDevice, c.st), "copy");
+    if (c.p->line)
+        HIPTRY(hipMemcpyAsync(sp.sino_tmp, b, c.ns * 4, hipMemcpyDeviceToDevice, c.st), "copy");
     hipEvent_t ev[3] = {NULL, NULL, NULL};
     uir_status s = UIR_OK;
     for (int i = 0; i < 3 && s == UIR_OK; ++i)
         s = uir_check_hip(hipEventCreate(&ev[i]), "hipEventCreate");
     double fp_sum = 0, bp_sum = 0;
     uint32_t timed = 0;
-    /* one sweep in order, as sart_sweep launches it; every stride-th angle's
-     * FP and BP are each bracketed by events */
+    /* one sweep with the FP and the BP of each angle launched apart; every
+     * stride-th angle's launches are each bracketed by events */
     for (uint32_t a = 0; a < c.A && s == UIR_OK; ++a) {
         const int tm = a % stride == 0;
-        if (tm)
+        const int hor = !c.p->line && sart_horizontal(c.p, a);
+        if (hor)
+            s = uir_check_hip(uirk_transpose(x, sp.t[0], (int)c.n, c.st), "transpose");
+        if (s == UIR_OK && tm)
             s = uir_check_hip(hipEventRecord(ev[0], c.st), "hipEventRecord");
         if (s == UIR_OK)
-            s = sart_fp_angle(&c, x, sp.sino_tmp, sp.ray_w, sp.axis, sp.starts, a);
+            s = c.p->line ? sart_line_fp(&c, x, sp.sino_tmp, sp.ray_w, a)
+                          : sart_step(&c, &sp, b, hor ? sp.t[0] : x, NULL, 0, -1, (int)a, hor);
         if (s == UIR_OK && tm)
             s = uir_check_hip(hipEventRecord(ev[1], c.st), "hipEventRecord");
         if (s == UIR_OK)
-            s = sart_bp_angle(&c, x, sp.sino_tmp, sp.axis, a);
+            s = c.p->line ? sart_line_bp(&c, x, sp.sino_tmp, a) : sart_step(&c, &sp, b, x, x, 1, (int)a, -1, 0);
         if (s == UIR_OK && tm) {
             float f = 0, g = 0;
             s = uir_check_hip(hipEventRecord(ev[2], c.st), "hipEventRecord");
