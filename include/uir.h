@@ -317,7 +317,7 @@ void       uir_asdpocs_params_default(uir_asdpocs_params *p);
 /* `iterations` ASD-POCS iterations of every slice from x = 0; the result
  * replaces the slice images (uir_batch_get_image).  Asynchronous on the batch
  * stream.  The first call allocates the method's own buffers (a second image
- * and an FP32 gradient per slice).  The batch's slices must share one
+ * and one of 4 bytes a pixel per slice).  The batch's slices must share one
  * projection model (UIR_ERR_UNSUPPORTED otherwise). */
 uir_status uir_batch_asdpocs(uir_batch *batch, uint32_t iterations, const uir_asdpocs_params *p, int use_graph);
 /* Rows (dd, dp, dg, dtgv) of slice `slice` from the last uir_batch_asdpocs,

@@ -138,78 +138,132 @@ __global__ __launch_bounds__(kThreads) void k_asd_sino(const uirk_asd_slice *__r
     block_sum(acc, &partials[(size_t)blockIdx.y * nblk + blockIdx.x]);
 }
 
-template <typename TI> __device__ __forceinline__ float nb(const TI *img, int n, int x, int y)
+// The smoothed TV gradient (ufo-math-tvstd-method.cl:5-57, eps 1e-3) is, with
+// f(x, y) = 0 outside the image and R(x, y) = 1 / sqrt(eps + (f(x, y) - f(x - 1, y))^2
+// + (f(x, y) - f(x, y + 1))^2),
+//   (2 f(x, y) - f(x - 1, y) - f(x, y + 1)) R(x, y)
+//     - (f(x + 1, y) - f(x, y)) R(x + 1, y) - (f(x, y - 1) - f(x, y)) R(x, y - 1),
+// so that each pixel's reciprocal root (the hardware's, ~1 ulp, a quarter of
+// the rate of other operations) serves three gradients.
+__device__ __forceinline__ float tv_root(float f, float left, float below)
 {
-    if (x < 0 || y < 0 || x >= n || y >= n)
-        return 0.0f;
-    return ld(img, (uint32_t)y * (uint32_t)n + (uint32_t)x);
+    const float eps = 0.001f;
+    return __builtin_amdgcn_rsqf(eps + (f - left) * (f - left) + (f - below) * (f - below));
+}
+__device__ __forceinline__ float tv_df(float f, float left, float right, float above, float below, float root,
+                                       float root_right, float root_above)
+{
+    return (2.0f * f - left - below) * root - (right - f) * root_right - (above - f) * root_above;
 }
 
-// g = l1_grad(x) (ufo-math-tvstd-method.cl:5-57: smoothed TV gradient, eps
-// 1e-3, zero outside the image) and the partial of |g| for this TV step;
-// nothing once the slice's TV steps have ended.  Block c of a slice covers
-// columns [256 (c % cx), +256) x rows [kTvRows (c / cx), +kTvRows): each thread
-// walks down one column with the 3 x 3 neighbourhood in registers, loading
-// one row (x - 1, x, x + 1) per pixel, all coalesced.  The three quotients
-// v / sqrt(w) are formed as v * rsqrt(w) (hardware reciprocal square root,
-// ~1 ulp).
+// The value of the next lower / higher lane (column x - 1 / x + 1).
+__device__ __forceinline__ float lane_below(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, false)); // wave_shr:1
+}
+__device__ __forceinline__ float lane_above(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, false)); // wave_shl:1
+}
+
+// v as the image's storage holds it
+__device__ __forceinline__ float stored(const float *, float v) { return v; }
+__device__ __forceinline__ float stored(const __half *, float v) { return __half2float(__float2half(v)); }
+__device__ __forceinline__ float stored(const __hip_bfloat16 *, float v)
+{
+    return __bfloat162float(__float2bfloat16(v));
+}
+
+// One TV step and the gradient norm the next one needs, in one pass: x1 = x -
+// factor g(x) (operation_deduction2, ufo-ir-basic-ops.cl:104-125, factor = dtgv /
+// |g| from the slice's state), from one of the slice's two buffers (S.x, S.g) to
+// the other, and the partial of |g(x1)|.  step 0: x1 = x, not written (the norm
+// before the first step); norm 0: no partial (the last step).  A slice whose TV
+// steps have ended keeps its image.
+// A wave owns 60 columns x kTvRows rows and walks down them with the rows in
+// registers: lane i holds column base - 2 + i, its neighbours' values come by
+// DPP shifts, g(x) is right on lanes 1 .. 62 and g(x1) on lanes 2 .. 61.  So a
+// step reads and writes the image once (8 bytes a pixel in FP32); a gradient
+// kernel and a step kernel moved 20: 307 us a step over 64 slices of 1024 x
+// 1024, this takes 146 (3.5 TB/s).
+constexpr int kTvRows = UIRK_ASD_TV_ROWS;
+constexpr int kTvCols = UIRK_ASD_TV_COLS;
+
 template <typename TI>
-__global__ __launch_bounds__(kThreads) void k_asd_tvgrad(const uirk_asd_slice *__restrict__ sl,
-                                                         const uirk_asd_state *__restrict__ state, int l2,
-                                                         double *__restrict__ partials, int nblk)
+__global__ __launch_bounds__(kThreads) void k_asd_tv(const uirk_asd_slice *__restrict__ sl,
+                                                     const uirk_asd_state *__restrict__ state, int from_g, int step,
+                                                     int norm, int l2, double *__restrict__ partials, int nblk)
 {
     const uirk_asd_slice S = sl[blockIdx.y];
     const int n = (int)S.n;
-    const int cx = (n + kThreads - 1) / kThreads, cy = (n + UIRK_ASD_TV_ROWS - 1) / UIRK_ASD_TV_ROWS;
+    const int lane = threadIdx.x & 63;
+    const int strips = (n + kTvCols - 1) / kTvCols, bands = (n + kTvRows - 1) / kTvRows;
+    const int w = (int)blockIdx.x * (kThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const bool stop = state[blockIdx.y].stop != 0;
     double acc = 0;
-    if ((int)blockIdx.x < cx * cy && !state[blockIdx.y].stop) {
-        const TI *img = (const TI *)S.x;
-        const int x = (int)(blockIdx.x % cx) * kThreads + threadIdx.x;
-        const int y0 = (int)(blockIdx.x / cx) * UIRK_ASD_TV_ROWS;
-        const int y1 = min(y0 + UIRK_ASD_TV_ROWS, n);
-        if (x < n) {
-            const float eps = 0.001f;
-            // rows y - 1 (a), y (b); columns x - 1 (m), x (0), x + 1 (p)
-            float am = nb(img, n, x - 1, y0 - 1), a0 = nb(img, n, x, y0 - 1);
-            float bm = nb(img, n, x - 1, y0), b0 = nb(img, n, x, y0), bp = nb(img, n, x + 1, y0);
-            for (int y = y0; y < y1; ++y) {
-                const float cm = nb(img, n, x - 1, y + 1), c0 = nb(img, n, x, y + 1), cp = nb(img, n, x + 1, y + 1);
-                const float f0 = am, f1 = a0, f2 = bm, f3 = b0, f4 = bp, f5 = c0, f6 = cp;
-                const float w0 = eps + (f3 - f2) * (f3 - f2) + (f3 - f5) * (f3 - f5);
-                const float w1 = eps + (f4 - f3) * (f4 - f3) + (f4 - f6) * (f4 - f6);
-                const float w2 = eps + (f1 - f3) * (f1 - f3) + (f1 - f0) * (f1 - f0);
-                const float df = (2.0f * f3 - f2 - f5) * __builtin_amdgcn_rsqf(w0) -
-                                 (f4 - f3) * __builtin_amdgcn_rsqf(w1) - (f1 - f3) * __builtin_amdgcn_rsqf(w2);
-                S.g[(uint32_t)y * (uint32_t)n + (uint32_t)x] = df;
-                acc += measure(df, l2);
-                am = bm;
-                a0 = b0;
-                bm = cm;
-                b0 = c0;
-                bp = cp;
+    if (w < strips * bands && (step || !stop)) {
+        const TI *in = from_g ? (const TI *)S.g : (const TI *)S.x;
+        TI *out = from_g ? (TI *)S.x : (TI *)S.g;
+        const float factor = state[blockIdx.y].factor;
+        const int c = (w % strips) * kTvCols - 2 + lane;
+        const bool cin = c >= 0 && c < n, own = cin && lane >= 2 && lane < 2 + kTvCols;
+        const int y0 = (w / strips) * kTvRows, y1 = min(y0 + kTvRows, n);
+        auto load = [&](int y) { // 0 outside the image
+            return cin && y >= 0 && y < n ? ld(in, (uint32_t)y * (uint32_t)n + (uint32_t)c) : 0.0f;
+        };
+        constexpr int kAhead = 4; // rows loaded ahead
+        float next[kAhead];
+        float a = load(y0 - 2), b = load(y0 - 1);
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k)
+            next[k] = load(y0 + k);
+        float bl = lane_below(b), br = lane_above(b);
+        float a_root = tv_root(a, lane_below(a), b);
+        // x1 of the rows above the current one, their neighbours and roots
+        float p2 = 0, p2_root = 0, p1 = 0, p1l = 0, p1r = 0;
+        for (int r0 = y0 - 1; r0 <= y1; r0 += kAhead) {
+            float cur[kAhead];
+#pragma unroll
+            for (int k = 0; k < kAhead; ++k) {
+                cur[k] = next[k];
+                next[k] = load(r0 + 1 + kAhead + k);
+            }
+#pragma unroll
+            for (int k = 0; k < kAhead; ++k) {
+                const int r = r0 + k; // x rows r - 1 (a), r (b), r + 1 (d)
+                if (r > y1)
+                    break;
+                const float d = cur[k];
+                float v = b;
+                if (step && !stop) {
+                    const float b_root = tv_root(b, bl, d);
+                    v = stored(in, b - factor * tv_df(b, bl, br, a, d, b_root, lane_above(b_root), a_root));
+                    v = cin && r >= 0 && r < n ? v : 0.0f;
+                    a_root = b_root;
+                }
+                if (step && own && r >= y0 && r < y1)
+                    st(out, (uint32_t)r * (uint32_t)n + (uint32_t)c, v);
+                if (norm && !stop) {
+                    const float p1_root = tv_root(p1, p1l, v);
+                    if (r > y0) {
+                        const float df = tv_df(p1, p1l, p1r, p2, v, p1_root, lane_above(p1_root), p2_root);
+                        acc += own ? measure(df, l2) : 0.0;
+                    }
+                    p2_root = p1_root;
+                }
+                p2 = p1;
+                p1 = v;
+                p1l = lane_below(v);
+                p1r = lane_above(v);
+                a = b;
+                b = d;
+                bl = lane_below(d);
+                br = lane_above(d);
             }
         }
     }
-    block_sum(acc, &partials[(size_t)blockIdx.y * nblk + blockIdx.x]);
-}
-
-// x = x - factor * g (operation_deduction2, ufo-ir-basic-ops.cl:104-125),
-// factor = dtgv / |g| from the slice's state.
-template <typename TI>
-__global__ __launch_bounds__(kThreads) void k_asd_tvstep(const uirk_asd_slice *__restrict__ sl,
-                                                         const uirk_asd_state *__restrict__ state)
-{
-    const uirk_asd_slice S = sl[blockIdx.y];
-    const uint32_t nv = S.n * S.n, base = blockIdx.x * kChunk;
-    if (base >= nv || state[blockIdx.y].stop)
-        return;
-    const float f = state[blockIdx.y].factor;
-    TI *x = (TI *)S.x;
-    for (int k = 0; k < kPer; ++k) {
-        const uint32_t i = base + k * kThreads + threadIdx.x;
-        if (i < nv)
-            st(x, i, ld(x, i) - f * S.g[i]);
-    }
+    if (norm)
+        block_sum(acc, &partials[(size_t)blockIdx.y * nblk + blockIdx.x]);
 }
 
 // One block per slice: the slice's partials added in a fixed order, then the
@@ -270,16 +324,14 @@ __global__ __launch_bounds__(kThreads) void k_asd_finish(uirk_asd_state *__restr
 }
 
 template <typename TI>
-int launch_image(int kind, const uirk_asd_slice *sl, int n_slices, int nblk, const uirk_asd_state *state, int flag,
-                 int l2, double *partials, hipStream_t stm)
+int launch_image(int kind, const uirk_asd_slice *sl, int n_slices, int nblk, int flag, int l2, double *partials,
+                 hipStream_t stm)
 {
     const dim3 grid(nblk, n_slices);
     switch (kind) {
     case 0: hipLaunchKernelGGL(k_asd_begin<TI>, grid, dim3(kThreads), 0, stm, sl, flag); break;
     case 1: hipLaunchKernelGGL(k_asd_posc_dp<TI>, grid, dim3(kThreads), 0, stm, sl, flag, l2, partials, nblk); break;
-    case 2: hipLaunchKernelGGL(k_asd_diff<TI>, grid, dim3(kThreads), 0, stm, sl, l2, partials, nblk); break;
-    case 3: hipLaunchKernelGGL(k_asd_tvgrad<TI>, grid, dim3(kThreads), 0, stm, sl, state, l2, partials, nblk); break;
-    default: hipLaunchKernelGGL(k_asd_tvstep<TI>, grid, dim3(kThreads), 0, stm, sl, state); break;
+    default: hipLaunchKernelGGL(k_asd_diff<TI>, grid, dim3(kThreads), 0, stm, sl, l2, partials, nblk); break;
     }
     return (int)hipGetLastError();
 }
@@ -288,19 +340,48 @@ int launch_image(int kind, const uirk_asd_slice *sl, int n_slices, int nblk, con
 
 extern "C" {
 
-int uirk_asd_image(int kind, int img_dtype, const uirk_asd_slice *d_sl, int n_slices, int nblk,
-                   const uirk_asd_state *d_state, int flag, int l2, double *d_partials, void *stream)
+int uirk_asd_image(int kind, int img_dtype, const uirk_asd_slice *d_sl, int n_slices, int nblk, int flag, int l2,
+                   double *d_partials, void *stream)
 {
     if (n_slices <= 0 || nblk <= 0 || n_slices > 65535)
         return n_slices == 0 ? 0 : (int)hipErrorInvalidValue;
     hipStream_t stm = (hipStream_t)stream;
     switch (img_dtype) {
-    case UIR_DTYPE_F32: return launch_image<float>(kind, d_sl, n_slices, nblk, d_state, flag, l2, d_partials, stm);
-    case UIR_DTYPE_F16: return launch_image<__half>(kind, d_sl, n_slices, nblk, d_state, flag, l2, d_partials, stm);
+    case UIR_DTYPE_F32: return launch_image<float>(kind, d_sl, n_slices, nblk, flag, l2, d_partials, stm);
+    case UIR_DTYPE_F16: return launch_image<__half>(kind, d_sl, n_slices, nblk, flag, l2, d_partials, stm);
     case UIR_DTYPE_BF16:
-        return launch_image<__hip_bfloat16>(kind, d_sl, n_slices, nblk, d_state, flag, l2, d_partials, stm);
+        return launch_image<__hip_bfloat16>(kind, d_sl, n_slices, nblk, flag, l2, d_partials, stm);
     default: return (int)hipErrorInvalidValue;
     }
+}
+
+int uirk_asd_tv(int img_dtype, const uirk_asd_slice *d_sl, int n_slices, int max_n, int nblk,
+                const uirk_asd_state *d_state, int from_g, int step, int norm, int l2, double *d_partials, void *stream)
+{
+    if (n_slices <= 0 || nblk <= 0 || n_slices > 65535)
+        return n_slices == 0 ? 0 : (int)hipErrorInvalidValue;
+    const int waves = ((max_n + kTvCols - 1) / kTvCols) * ((max_n + kTvRows - 1) / kTvRows);
+    const int blocks = (waves + kThreads / 64 - 1) / (kThreads / 64);
+    if (blocks > nblk)
+        return (int)hipErrorInvalidValue;
+    const dim3 grid(norm ? nblk : blocks, n_slices); // every partial of a norm is written
+    hipStream_t stm = (hipStream_t)stream;
+    switch (img_dtype) {
+    case UIR_DTYPE_F32:
+        hipLaunchKernelGGL(k_asd_tv<float>, grid, dim3(kThreads), 0, stm, d_sl, d_state, from_g, step, norm, l2,
+                           d_partials, nblk);
+        break;
+    case UIR_DTYPE_F16:
+        hipLaunchKernelGGL(k_asd_tv<__half>, grid, dim3(kThreads), 0, stm, d_sl, d_state, from_g, step, norm, l2,
+                           d_partials, nblk);
+        break;
+    case UIR_DTYPE_BF16:
+        hipLaunchKernelGGL(k_asd_tv<__hip_bfloat16>, grid, dim3(kThreads), 0, stm, d_sl, d_state, from_g, step, norm,
+                           l2, d_partials, nblk);
+        break;
+    default: return (int)hipErrorInvalidValue;
+    }
+    return (int)hipGetLastError();
 }
 
 int uirk_asd_sino_norm(int dtype, const uirk_asd_slice *d_sl, int n_slices, int nblk, int l2, double *d_partials,

@@ -319,14 +319,16 @@ int uirk_sb_shrink(const void *u, int dtype, float *bx, float *by, float *ex, fl
 
 /* ---- Batched ASD-POCS steps between the projections (uir_asd.hip) ----
  * Grids are (nblk, n_slices): block (c, s) covers elements [c, c + 1) *
- * UIRK_ASD_CHUNK of slice s (TVGRAD: a 256 x UIRK_ASD_TV_ROWS tile; nblk
- * must cover the largest image both ways; sinograms are strided over the
- * nblk blocks) and writes partials[s * nblk + c]. */
+ * UIRK_ASD_CHUNK of slice s (uirk_asd_tv: four UIRK_ASD_TV_COLS x
+ * UIRK_ASD_TV_ROWS pieces; nblk must cover the largest image both ways;
+ * sinograms are strided over the nblk blocks) and writes
+ * partials[s * nblk + c]. */
 #define UIRK_ASD_CHUNK 4096
-#define UIRK_ASD_TV_ROWS 16 /* TVGRAD blocks: 256 columns x 16 rows */
+#define UIRK_ASD_TV_COLS 60
+#define UIRK_ASD_TV_ROWS 32
 typedef struct {
     void *x, *x_prev;    /* image and its checkpoint (image dtype) */
-    float *g;            /* TV gradient (FP32) */
+    float *g;            /* second image buffer (image dtype) of the SART and TV steps */
     const void *r;       /* residual sinogram b - A x (sinogram dtype) */
     uint32_t n, n_sino;  /* image edge; n_angles * n_dets */
 } uirk_asd_slice;
@@ -340,12 +342,17 @@ typedef struct {
 } uirk_asd_params;
 /* kind: BEGIN (flag 0: x = 0, 1: x_prev = x, 2: x = x_prev, 3: x = g as image
  * dtype), POSC_DP (flag = posc:
- * x = max(x, 0), partial |x - x_prev|, x_prev = x), DIFF (partial |x - x_prev|),
- * TVGRAD (g = l1_grad(x), partial |g|), TVSTEP (x -= factor g); l2 selects
- * sums of squares over sums of magnitudes. */
-enum { UIRK_ASD_BEGIN = 0, UIRK_ASD_POSC_DP = 1, UIRK_ASD_DIFF = 2, UIRK_ASD_TVGRAD = 3, UIRK_ASD_TVSTEP = 4 };
-int uirk_asd_image(int kind, int img_dtype, const uirk_asd_slice *d_sl, int n_slices, int nblk,
-                   const uirk_asd_state *d_state, int flag, int l2, double *d_partials, void *stream);
+ * x = max(x, 0), partial |x - x_prev|, x_prev = x), DIFF (partial |x - x_prev|);
+ * l2 selects sums of squares over sums of magnitudes. */
+enum { UIRK_ASD_BEGIN = 0, UIRK_ASD_POSC_DP = 1, UIRK_ASD_DIFF = 2 };
+int uirk_asd_image(int kind, int img_dtype, const uirk_asd_slice *d_sl, int n_slices, int nblk, int flag, int l2,
+                   double *d_partials, void *stream);
+/* One TV step (step != 0): the other of (x, g) = y - factor l1_grad(y) with y =
+ * g when from_g, else x; with norm, the partial |l1_grad| of the result (step
+ * 0: of y).  A slice with stop set in its state is copied. */
+int uirk_asd_tv(int img_dtype, const uirk_asd_slice *d_sl, int n_slices, int max_n, int nblk,
+                const uirk_asd_state *d_state, int from_g, int step, int norm, int l2, double *d_partials,
+                void *stream);
 /* partial |r| over the residual sinograms */
 int uirk_asd_sino_norm(int dtype, const uirk_asd_slice *d_sl, int n_slices, int nblk, int l2, double *d_partials,
                        void *stream);

@@ -12,7 +12,8 @@
  *               (uirk_sart_rows);
  *   POSC + dp   x = max(x, 0), dp = |x - x_prev|, x_prev = x;
  *   dd          r = b - A x over all angles (the batch's FP tables), |r|;
- *   TV          ng times: g = l1_grad(x), |g|, x -= dtgv / |g| g;
+ *   TV          |g| of g = l1_grad(x), then ng times x -= dtgv / |g| g in one
+ *               pass with the next |g| (uirk_asd_tv);
  *   dg          |x - x_prev|, then the dtgv / beta updates.
  * A batch of the line model runs each SART angle as the model's FP rows and
  * BP update over every slice (uirk_sart_line: two launches, the image updated
@@ -33,9 +34,9 @@
 #define HIP(x, what) TRY(uir_check_hip((x), (what)))
 
 struct uir_asd {
-    void *mem;                 /* per slice: x_prev (image dtype), g (FP32), SART partial sums (FP32) */
+    void *mem;                 /* per slice: x_prev, g (a second image, 4 bytes a pixel), SART partial sums */
     uirk_asd_slice *d_sl;
-    uirk_sart_slice *d_sart[2]; /* fused SART step: x -> g, g -> x (g is free during the data step) */
+    uirk_sart_slice *d_sart[2]; /* fused SART step: x -> g, g -> x */
     uirk_slice *d_dd_sl;       /* residual FP r = b - A x for dd */
     uint32_t n_max, d_max, a_max;
     int line;                  /* every slice has the line model */
@@ -109,9 +110,10 @@ static uir_status asd_create(uir_batch *b, struct uir_asd **out)
         const size_t nv = (size_t)sp->n * sp->n;
         const size_t part = (size_t)((sp->n + 63) / 64) * 3 * sp->n_dets;
         total += align_up(nv * b->esi) + align_up(nv * 4) + align_up(part * 4);
-        const size_t tiles = (size_t)((sp->n + 255) / 256) * ((sp->n + UIRK_ASD_TV_ROWS - 1) / UIRK_ASD_TV_ROWS);
+        const size_t tiles = (size_t)((sp->n + UIRK_ASD_TV_COLS - 1) / UIRK_ASD_TV_COLS) *
+                             ((sp->n + UIRK_ASD_TV_ROWS - 1) / UIRK_ASD_TV_ROWS);
         max_nv = nv > max_nv ? nv : max_nv;
-        max_tv = tiles > max_tv ? tiles : max_tv;
+        max_tv = (tiles + 3) / 4 > max_tv ? (tiles + 3) / 4 : max_tv;
         a->n_max = sp->n > a->n_max ? sp->n : a->n_max;
         a->d_max = sp->n_dets > a->d_max ? sp->n_dets : a->d_max;
         a->a_max = sp->n_angles > a->a_max ? sp->n_angles : a->a_max;
@@ -154,7 +156,7 @@ static uir_status asd_create(uir_batch *b, struct uir_asd **out)
             /* fused SART step: r[k] = (b[k] - A_k x) R[k], x += relax A_k^T r[k] */
             uirk_sart_slice *f = &sa[i];
             f->x_in = b->x[i];
-            f->x_out = sl[i].g; /* holds image-dtype data while the data step runs */
+            f->x_out = sl[i].g; /* holds image-dtype data */
             f->r = b->r[i];
             f->b = b->b[i];
             f->ray_w = G->d_ray_w;
@@ -222,7 +224,7 @@ static uir_status launch_asd_iteration(uir_batch *b, const uir_asdpocs_params *p
 #define FINISH(what)                                                                                              \
     HIP(uirk_asd_finish(a->d_state, a->d_partials, S, nblk, (what), &kp, a->d_diag, (int)diag_iters, st),     \
         "ASD-POCS reduction")
-    HIP(uirk_asd_image(UIRK_ASD_BEGIN, b->idt, a->d_sl, S, nblk, a->d_state, tb ? 1 : 0, tb, a->d_partials, st),
+    HIP(uirk_asd_image(UIRK_ASD_BEGIN, b->idt, a->d_sl, S, nblk, tb ? 1 : 0, tb, a->d_partials, st),
         "ASD-POCS start");
     /* SART passes: launch j applies the BP of angle j - 1 and sums the FP of
      * angle j, from buffer j % 2 to (j + 1) % 2 (x, g); the last launch only
@@ -241,10 +243,10 @@ static uir_status launch_asd_iteration(uir_batch *b, const uir_asdpocs_params *p
                 HIP(uirk_sart_rows(a->d_sart[j % 2], S, (int)a->d_max, b->sdt, fp, st), "SART residual launch");
         }
         if ((A + 1) % 2)
-            HIP(uirk_asd_image(UIRK_ASD_BEGIN, b->idt, a->d_sl, S, nblk, a->d_state, 3, 0, a->d_partials, st),
+            HIP(uirk_asd_image(UIRK_ASD_BEGIN, b->idt, a->d_sl, S, nblk, 3, 0, a->d_partials, st),
                 "SART copy");
     }
-    HIP(uirk_asd_image(UIRK_ASD_POSC_DP, b->idt, a->d_sl, S, nblk, a->d_state, p->positive_constraint ? 1 : 0, tb,
+    HIP(uirk_asd_image(UIRK_ASD_POSC_DP, b->idt, a->d_sl, S, nblk, p->positive_constraint ? 1 : 0, tb,
                        a->d_partials, st), "ASD-POCS POSC");
     FINISH(UIRK_ASD_DP);
     for (int g = 0; g < UIR_FP_SHAPES; ++g) {
@@ -259,14 +261,23 @@ static uir_status launch_asd_iteration(uir_batch *b, const uir_asdpocs_params *p
     HIP(uirk_asd_sino_norm(b->sdt, a->d_sl, S, nblk, tb, a->d_partials, st), "residual norm");
     FINISH(UIRK_ASD_DD);
     const uint32_t ng = tb ? p->ng : 20; /* tvstd :573 takes 20 steps; ng is unused there */
-    for (uint32_t k = 0; k < ng; ++k) {
-        HIP(uirk_asd_image(UIRK_ASD_TVGRAD, b->idt, a->d_sl, S, nblk, a->d_state, 0, tb, a->d_partials, st),
+    /* step k reads x (even k) or g (odd k) and writes the other, and sums the
+     * gradient norm of what it wrote for step k + 1 */
+    if (ng) {
+        HIP(uirk_asd_tv(b->idt, a->d_sl, S, (int)a->n_max, nblk, a->d_state, 0, 0, 1, tb, a->d_partials, st),
             "TV gradient");
         FINISH(UIRK_ASD_G);
-        HIP(uirk_asd_image(UIRK_ASD_TVSTEP, b->idt, a->d_sl, S, nblk, a->d_state, 0, tb, a->d_partials, st),
-            "TV step");
     }
-    HIP(uirk_asd_image(UIRK_ASD_DIFF, b->idt, a->d_sl, S, nblk, a->d_state, 0, tb, a->d_partials, st), "TV distance");
+    for (uint32_t k = 0; k < ng; ++k) {
+        const int more = k + 1 < ng;
+        HIP(uirk_asd_tv(b->idt, a->d_sl, S, (int)a->n_max, nblk, a->d_state, (int)(k & 1), 1, more, tb, a->d_partials,
+                        st), "TV step");
+        if (more)
+            FINISH(UIRK_ASD_G);
+    }
+    if (ng & 1)
+        HIP(uirk_asd_image(UIRK_ASD_BEGIN, b->idt, a->d_sl, S, nblk, 3, 0, a->d_partials, st), "TV copy");
+    HIP(uirk_asd_image(UIRK_ASD_DIFF, b->idt, a->d_sl, S, nblk, 0, tb, a->d_partials, st), "TV distance");
     FINISH(UIRK_ASD_DG);
 #undef FINISH
     return UIR_OK;
@@ -329,7 +340,7 @@ uir_status uir_batch_asdpocs(uir_batch *b, uint32_t iterations, const uir_asdpoc
         const size_t nv = (size_t)b->specs[i].n * b->specs[i].n;
         HIP(hipMemsetAsync(b->x[i], 0, nv * b->esi, st), "hipMemsetAsync");
     }
-    HIP(uirk_asd_image(UIRK_ASD_BEGIN, b->idt, a->d_sl, (int)S, a->nblk, a->d_state, 1, 0, a->d_partials, st),
+    HIP(uirk_asd_image(UIRK_ASD_BEGIN, b->idt, a->d_sl, (int)S, a->nblk, 1, 0, a->d_partials, st),
         "ASD-POCS start");
     if (iterations == 0)
         return UIR_OK;
@@ -362,7 +373,7 @@ uir_status uir_batch_asdpocs(uir_batch *b, uint32_t iterations, const uir_asdpoc
             HIP(hipGraphLaunch(a->exec, st), "hipGraphLaunch");
     }
     if (p->compat) /* the reference's output is the image before the last TV steps */
-        HIP(uirk_asd_image(UIRK_ASD_BEGIN, b->idt, a->d_sl, (int)S, a->nblk, a->d_state, 2, 0, a->d_partials, st),
+        HIP(uirk_asd_image(UIRK_ASD_BEGIN, b->idt, a->d_sl, (int)S, a->nblk, 2, 0, a->d_partials, st),
             "ASD-POCS output");
     return UIR_OK;
 }
