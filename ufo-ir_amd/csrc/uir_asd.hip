@@ -138,22 +138,23 @@ __global__ __launch_bounds__(kThreads) void k_asd_sino(const uirk_asd_slice *__r
     block_sum(acc, &partials[(size_t)blockIdx.y * nblk + blockIdx.x]);
 }
 
-// The smoothed TV gradient (ufo-math-tvstd-method.cl:5-57, eps 1e-3) is, with
-// f(x, y) = 0 outside the image and R(x, y) = 1 / sqrt(eps + (f(x, y) - f(x - 1, y))^2
-// + (f(x, y) - f(x, y + 1))^2),
-//   (2 f(x, y) - f(x - 1, y) - f(x, y + 1)) R(x, y)
-//     - (f(x + 1, y) - f(x, y)) R(x + 1, y) - (f(x, y - 1) - f(x, y)) R(x, y - 1),
-// so that each pixel's reciprocal root (the hardware's, ~1 ulp, a quarter of
-// the rate of other operations) serves three gradients.
+// The smoothed TV gradient of one pixel (ufo-math-tvstd-method.cl:5-57, eps
+// 1e-3).  The three quotients v / sqrt(w) are formed as v * rsqrt(w) (hardware
+// reciprocal square root, ~1 ulp, a quarter of the rate of other operations);
+// the second is the first of the pixel to the right, bit for bit, and comes from
+// its lane.  (The third is the first of the pixel above but for the order of two
+// additions, which the TV steps amplify: it stays its own.)
+constexpr float kTvEps = 0.001f;
 __device__ __forceinline__ float tv_root(float f, float left, float below)
 {
-    const float eps = 0.001f;
-    return __builtin_amdgcn_rsqf(eps + (f - left) * (f - left) + (f - below) * (f - below));
+    return __builtin_amdgcn_rsqf(kTvEps + (f - left) * (f - left) + (f - below) * (f - below));
 }
-__device__ __forceinline__ float tv_df(float f, float left, float right, float above, float below, float root,
-                                       float root_right, float root_above)
+__device__ __forceinline__ float tv_df(float f, float left, float right, float above, float above_left, float below,
+                                       float root, float root_right)
 {
-    return (2.0f * f - left - below) * root - (right - f) * root_right - (above - f) * root_above;
+    const float w2 = kTvEps + (above - f) * (above - f) + (above - above_left) * (above - above_left);
+    return (2.0f * f - left - below) * root - (right - f) * root_right -
+           (above - f) * __builtin_amdgcn_rsqf(w2);
 }
 
 // The value of the next lower / higher lane (column x - 1 / x + 1).
@@ -185,7 +186,7 @@ __device__ __forceinline__ float stored(const __hip_bfloat16 *, float v)
 // DPP shifts, g(x) is right on lanes 1 .. 62 and g(x1) on lanes 2 .. 61.  So a
 // step reads and writes the image once (8 bytes a pixel in FP32); a gradient
 // kernel and a step kernel moved 20: 307 us a step over 64 slices of 1024 x
-// 1024, this takes 146 (3.5 TB/s).
+// 1024, this takes 166 (3.1 TB/s).
 constexpr int kTvRows = UIRK_ASD_TV_ROWS;
 constexpr int kTvCols = UIRK_ASD_TV_COLS;
 
@@ -217,10 +218,9 @@ __global__ __launch_bounds__(kThreads) void k_asd_tv(const uirk_asd_slice *__res
 #pragma unroll
         for (int k = 0; k < kAhead; ++k)
             next[k] = load(y0 + k);
-        float bl = lane_below(b), br = lane_above(b);
-        float a_root = tv_root(a, lane_below(a), b);
-        // x1 of the rows above the current one, their neighbours and roots
-        float p2 = 0, p2_root = 0, p1 = 0, p1l = 0, p1r = 0;
+        float al = lane_below(a), bl = lane_below(b), br = lane_above(b);
+        // x1 of the rows above the current one, and their neighbours
+        float p2 = 0, p2l = 0, p1 = 0, p1l = 0, p1r = 0;
         for (int r0 = y0 - 1; r0 <= y1; r0 += kAhead) {
             float cur[kAhead];
 #pragma unroll
@@ -236,26 +236,24 @@ __global__ __launch_bounds__(kThreads) void k_asd_tv(const uirk_asd_slice *__res
                 const float d = cur[k];
                 float v = b;
                 if (step && !stop) {
-                    const float b_root = tv_root(b, bl, d);
-                    v = stored(in, b - factor * tv_df(b, bl, br, a, d, b_root, lane_above(b_root), a_root));
+                    const float root = tv_root(b, bl, d);
+                    v = stored(in, b - factor * tv_df(b, bl, br, a, al, d, root, lane_above(root)));
                     v = cin && r >= 0 && r < n ? v : 0.0f;
-                    a_root = b_root;
                 }
                 if (step && own && r >= y0 && r < y1)
                     st(out, (uint32_t)r * (uint32_t)n + (uint32_t)c, v);
-                if (norm && !stop) {
-                    const float p1_root = tv_root(p1, p1l, v);
-                    if (r > y0) {
-                        const float df = tv_df(p1, p1l, p1r, p2, v, p1_root, lane_above(p1_root), p2_root);
-                        acc += own ? measure(df, l2) : 0.0;
-                    }
-                    p2_root = p1_root;
+                if (norm && !stop && r > y0) {
+                    const float root = tv_root(p1, p1l, v);
+                    const float df = tv_df(p1, p1l, p1r, p2, p2l, v, root, lane_above(root));
+                    acc += own ? measure(df, l2) : 0.0;
                 }
                 p2 = p1;
+                p2l = p1l;
                 p1 = v;
                 p1l = lane_below(v);
                 p1r = lane_above(v);
                 a = b;
+                al = bl;
                 b = d;
                 bl = lane_below(d);
                 br = lane_above(d);

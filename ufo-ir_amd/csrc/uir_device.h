@@ -384,7 +384,7 @@ typedef struct {
     const uirk_line_angle *line; /* the line model (uirk_sart_line) only */
 } uirk_sart_slice;
 int uirk_sart_step(const uirk_sart_slice *d_slices, const uirk_asd_state *d_state, int n_slices, int max_n,
-                   int dtype, int img_dtype, int bp_angle, int fp_angle, int *d_err, void *stream);
+                   int dtype, int img_dtype, int bp_angle, int fp_angle, int n_xcd, int *d_err, void *stream);
 int uirk_sart_rows(const uirk_sart_slice *d_slices, int n_slices, int max_d, int dtype, int angle, void *stream);
 /* The same SART angle for slices of the line model (uir_line.hip), in two
  * launches: r[angle] = (b + corr FP) * ray_w, then x_out = x_in + relax

@@ -1245,62 +1245,52 @@ __global__ __launch_bounds__(256, LINE ? 4 : (PAIR ? (NA == 32 ? 3 : 4) : 6)) vo
 // ------------------------------------------------------------------------
 // Fused SART step: the BP of angle k - 1 and the FP of angle k in one pass
 // ------------------------------------------------------------------------
-// Block (t, s) owns the 64 x 64 tile t of slice s.  It stages the tile with a
-// one-pixel halo (66 x 66) from x_in, applies the BP of angle bp_angle to
-// every staged pixel (x += relax * A^T r[bp_angle], fast-path arithmetic:
-// exact per-pixel detector coordinate, clamp-to-edge bins as k_bp_tab),
-// writes the 64 x 64 interior to x_out (a different buffer: the
-// halo belongs to the neighbours) and keeps the updated tile in LDS.  It then
-// sums, for angle fp_angle, every Joseph sample whose left (lower) tap c0
-// lies in the tile's positions (tile 0 also owns c0 = -1) over the tile's 64
-// lines, ray by ray.  Each ray's partial goes to part[band][tile % 3][ray]:
-// a ray's samples in one band of lines touch at most three consecutive tiles
-// (even with the margins below), so tiles sharing a slot never share a ray.
-// k_sart_rows then adds the partials of the tiles each ray crosses.
+// A workgroup owns one 64 x 64 tile of one slice.  It loads the tile with a
+// one-pixel halo (66 x 66) from x_in, applies the BP of angle bp_angle to it
+// (x += relax * A^T r[bp_angle], exact per-pixel detector coordinate clamped to
+// the active window, the residual row's bins from LDS), writes the interior to
+// x_out (a different buffer: the halo belongs to the neighbours) and keeps the
+// updated tile in LDS, line by line of the FP's walk.  It then sums, for angle
+// fp_angle, every Joseph sample whose left (lower) tap c0 lies in the tile's
+// positions (tile 0 also owns c0 = -1) over the tile's 64 lines.  Each ray's
+// partial goes to part[band][tile % 3][ray]: a ray's samples in one band of
+// lines touch at most three consecutive tiles (even with the margins below), so
+// tiles sharing a slot never share a ray.  k_sart_rows then adds the partials of
+// the tiles each ray crosses.
 //
 // The sample-to-tile assignment must not depend on the tile: every tile
 // evaluates the tap position of (ray, line) as fma(line, step, q0) in float,
-// q0 the ray's position at line 0 rounded once from double, and visits only
-// the lines whose taps can fall in its positions (with a one-position margin).
+// q0 the ray's position at line 0 rounded once from double, and takes the
+// samples whose tap is its own.  A thread walks 32 lines of one candidate ray.
+//
+// What bounds it is memory: 8 bytes a pixel in FP32 and the halo.  A band's
+// tiles run on one XCD, whose L2 then serves the halo columns.  Over 64 slices
+// of 1024 x 1024 a launch takes 120 us (4.5 TB/s), from 173 when every pixel
+// gathered its two bins from the row in memory and every ray solved for its
+// lines in double.
 constexpr int kSt = 64;          // tile edge
 constexpr int kSl = kSt + 2;     // staged edge
+constexpr int kSs = kSl + 1;     // stride of a staged line (odd: no bank conflicts either way)
 constexpr int kSartRays = 128;   // candidate rays per tile (at most 98 by construction)
-
-// Candidate rays of a tile: those whose tap position c = pos - 0.5 falls in
-// [p_base - 3, p_base + 67) on a line of [la, lb]; pos(s, l) = (s + 0.5 - axis)
-// det_step + C + l step is affine in (s, l), so the set is the interval between
-// the corner solutions (one more ray of margin each side).
-__device__ __forceinline__ void sart_candidates(double det_step, double step, double C, double axis, int la, int lb,
-                                                int p_base, int D, int &s_lo, int &s_hi)
-{
-    double smin = 1e300, smax = -1e300;
-    const int ls[2] = {la, lb};
-    const double cs[2] = {(double)p_base - 3.0, (double)p_base + 67.0};
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const double s = (cs[j] + 0.5 - C - (double)ls[i] * step) / det_step - 0.5 + axis;
-            smin = fmin(smin, s);
-            smax = fmax(smax, s);
-        }
-    s_lo = max((int)floor(smin) - 1, 0);
-    s_hi = min((int)ceil(smax) + 1, D - 1);
-}
+constexpr int kSartWb = 104;     // staged bins (66 sqrt(2) and margins: 99)
 
 template <typename T, typename TI>
 __global__ __launch_bounds__(256) void k_sart_step(const uirk_sart_slice *__restrict__ slices,
                                                    const uirk_asd_state *__restrict__ state, int bp_angle,
-                                                   int fp_angle, int *__restrict__ err)
+                                                   int fp_angle, int n_xcd, int *__restrict__ err)
 {
-    __shared__ float tile[kSl * kSl];
+    __shared__ float tile[kSl * kSs];
+    __shared__ float bins[kSartWb];
     __shared__ float half_sum[kSartRays];
     const uirk_sart_slice *S = &slices[blockIdx.y];
     const int N = S->n, D = S->n_dets;
     const int nt = (N + kSt - 1) / kSt;
-    if ((int)blockIdx.x >= nt * nt)
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // workgroup g of a slice runs on XCD g mod n_xcd
+    const int turn = (int)blockIdx.x / n_xcd;
+    const int ty = (int)blockIdx.x % n_xcd + turn / nt * n_xcd, tx = turn % nt;
+    if (ty >= nt)
         return; // uniform over the block
-    const int tx = (int)blockIdx.x % nt, ty = (int)blockIdx.x / nt;
     const int x0 = tx * kSt, y0 = ty * kSt;
     const TI *xin = uniform((const TI *)S->x_in);
     TI *xout = uniform((TI *)S->x_out);
@@ -1309,142 +1299,160 @@ __global__ __launch_bounds__(256) void k_sart_step(const uirk_sart_slice *__rest
     const float required_width = axis_f * 2;
     const float diff = (float)D - required_width;
     const float origin_shift = (float)N / 2.0f;
+    const bool do_bp = bp_angle >= 0 && bp_angle < S->n_angles, do_fp = fp_angle >= 0 && fp_angle < S->n_angles;
 
-    // BP of bp_angle (projector-parallel-joseph.cl:174-190 geometry, clamp-to-edge bins)
-    const bool do_bp = bp_angle >= 0 && bp_angle < S->n_angles;
-    float bst = 0.0f, bct = 0.0f, gain = 0.0f;
-    float w_lo = 0.0f, w_hi = 0.0f;
-    const T *row = nullptr;
+    // Loads: the interior (one column and 16 rows per thread) and the halo ring
+    // (wave 0 and 1: the rows above and below, 2 and 3: the columns left and
+    // right, then the four entries left over); zero outside the image.
+    const __amdgpu_buffer_rsrc_t img = buf_rsrc(xin, (uint32_t)N * (uint32_t)N);
+    auto pixel = [&](int i, int j) { // staged entry (i, j): pixel (y0 - 1 + i, x0 - 1 + j)
+        const int py = y0 - 1 + i, px = x0 - 1 + j;
+        return bload(img, xin, (uint32_t)px < (uint32_t)N ? py * N + px : -1);
+    };
+    constexpr int kRows = kSt / 4;
+    float xv[kRows];
+#pragma unroll
+    for (int k = 0; k < kRows; ++k)
+        xv[k] = pixel(wave + 4 * k + 1, lane + 1);
+    const int hi = wave == 0 ? 0 : (wave == 1 ? kSl - 1 : lane + 1), hj = wave < 2 ? lane : (wave == 2 ? 0 : kSl - 1);
+    const float hv = pixel(hi, hj);
+    const int ci = threadIdx.x & 2 ? kSl - 1 : 0, cj = kSt + (threadIdx.x & 1);
+    float cv = 0.0f;
+    if (threadIdx.x < 4)
+        cv = pixel(ci, cj);
+
+    float bst = 0.0f, bct = 0.0f, gain = 0.0f, w_lo = 0.0f, w_hi = 0.0f;
+    const float shift = (float)D / 2.0f - diff / 2.0f;
+    int umin = 0;
     if (do_bp) {
+        // projector-parallel-joseph.cl:174-190 (detector quantities use n_dets)
         bst = gload(trig, 2 * bp_angle);
         bct = gload(trig, 2 * bp_angle + 1);
-        const float half_active = diff < 0 ? (float)D - axis_f : axis_f;
-        // the clamp window of u - 0.5 (:180-182, :203-210)
-        w_lo = (axis_f - half_active + 0.5f) - 0.5f;
-        w_hi = (axis_f + half_active - 0.5f) - 0.5f;
         gain = state[blockIdx.y].relax;
-        row = uniform((const T *)S->r) + (size_t)bp_angle * D;
+        const float half_active = diff < 0 ? (float)D - axis_f : axis_f;
+        const float edge0 = axis_f - half_active + 0.5f, edge1 = axis_f + half_active - 0.5f;
+        const float cx0 = (float)x0 - 0.5f - origin_shift, cx1 = cx0 + (float)(kSl - 1);
+        const float cy0 = (float)y0 - 0.5f - origin_shift, cy1 = cy0 + (float)(kSl - 1);
+        const float u00 = cx0 * bct - cy0 * bst, u10 = cx1 * bct - cy0 * bst;
+        const float u01 = cx0 * bct - cy1 * bst, u11 = cx1 * bct - cy1 * bst;
+        const float umn = fminf(fmaxf(fminf(fminf(u00, u10), fminf(u01, u11)) + shift, edge0), edge1);
+        const float umx = fminf(fmaxf(fmaxf(fmaxf(u00, u10), fmaxf(u01, u11)) + shift, edge0), edge1);
+        umin = (int)floorf(umn - 0.5f) - 1;
+        if ((int)floorf(umx - 0.5f) + 2 - umin >= kSartWb && threadIdx.x == 0)
+            atomicOr(err, 8); // cannot happen: reported, never silent
+        // the clamp window of u - 0.5 (:180-182, :203-210)
+        w_lo = edge0 - 0.5f;
+        w_hi = edge1 - 0.5f;
+        if (threadIdx.x < kSartWb) {
+            const T *row = uniform((const T *)S->r);
+            const int bin = min(max(umin + (int)threadIdx.x, 0), D - 1);
+            bins[threadIdx.x] = gload(row, (uint32_t)bp_angle * (uint32_t)D + (uint32_t)bin);
+        }
+        __syncthreads();
     }
-    const float shift = (float)D / 2.0f - diff / 2.0f;
-    // The BP taps of one pixel: u = X cos - Y sin + axis - 0.5, clamped to the
-    // active window; the bins are also kept inside the row whatever the axis.
-    auto bp_taps = [&](int px, int py, float &a, float &t0, float &t1) {
-        const float fX = (float)px + 0.5f - origin_shift, fY = (float)py + 0.5f - origin_shift;
-        const float u = __builtin_amdgcn_fmed3f(__builtin_fmaf(-fY, bst, __builtin_fmaf(fX, bct, shift - 0.5f)),
-                                                w_lo, w_hi);
-        const int bin = cvt_flr(u);
-        a = u - floorf(u);
-        const int b0 = min(max(bin, 0), D - 1), b1 = min(max(bin + 1, 0), D - 1);
-        t0 = gload(row, (uint32_t)b0);
-        t1 = gload(row, (uint32_t)b1);
+    // x of the pixel with column term cterm = fma(fX, cos, shift - 1/2) and row
+    // coordinate fY: u = X cos - Y sin + axis - 0.5
+    auto update = [&](float x, float cterm, float fY) {
+        const float u = __builtin_amdgcn_fmed3f(__builtin_fmaf(-fY, bst, cterm), w_lo, w_hi);
+        const float *t = bins + (cvt_flr(u) - umin);
+        const float t0 = t[0], t1 = t[1];
+        return __builtin_fmaf(__builtin_fmaf(fract_pos(u), t1 - t0, t0), gain, x);
     };
-    // Staged (i, j) is pixel (y0 - 1 + i, x0 - 1 + j); out-of-image entries are 0.
-    // Interior: one column and 16 rows per thread, in two batches of 8 rows
-    // whose loads are all issued first.
+
+    // the FP's direction decides how the tile is laid out: tile[line][position]
+    const float st = do_fp ? gload(trig, 2 * fp_angle) : 0.0f, ct = do_fp ? gload(trig, 2 * fp_angle + 1) : 1.0f;
+    const bool hor = !(fabsf(st) <= fabsf(ct));
+    const int si = hor ? 1 : kSs, sj = hor ? kSs : 1;
     {
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-        const int px = x0 + lane;
-        const bool col_in = px < N;
-        constexpr int kRows = 8;
-        for (int k0 = 0; k0 < kSt / 4; k0 += kRows) {
-            float xv[kRows], t0[kRows], t1[kRows], a[kRows];
+        const float cterm = __builtin_fmaf((float)(x0 + lane) + 0.5f - origin_shift, bct, shift - 0.5f);
+        const bool col_in = x0 + lane < N;
 #pragma unroll
-            for (int k = 0; k < kRows; ++k) {
-                const int py = min(y0 + wave + 4 * (k0 + k), N - 1), pxc = min(px, N - 1);
-                xv[k] = gload(xin, (uint32_t)py * (uint32_t)N + (uint32_t)pxc);
-                a[k] = t0[k] = t1[k] = 0.0f;
-                if (do_bp)
-                    bp_taps(pxc, py, a[k], t0[k], t1[k]);
-            }
-#pragma unroll
-            for (int k = 0; k < kRows; ++k) {
-                const int py = y0 + wave + 4 * (k0 + k);
-                float v = 0.0f;
-                if (col_in && py < N) {
-                    v = do_bp ? __builtin_fmaf(__builtin_fmaf(a[k], t1[k] - t0[k], t0[k]), gain, xv[k]) : xv[k];
-                    gstore(xout, (uint32_t)py * (uint32_t)N + (uint32_t)px, v);
-                }
-                tile[(wave + 4 * (k0 + k) + 1) * kSl + lane + 1] = v;
-            }
+        for (int k = 0; k < kRows; ++k) {
+            const int i = wave + 4 * k + 1;
+            float v = xv[k];
+            if (do_bp)
+                v = update(v, cterm, (float)(y0 - 1 + i) + 0.5f - origin_shift);
+            if (col_in && y0 - 1 + i < N)
+                gstore(xout, (uint32_t)(y0 - 1 + i) * (uint32_t)N + (uint32_t)(x0 + lane), v);
+            else
+                v = 0.0f;
+            tile[i * si + (lane + 1) * sj] = v;
         }
+        auto halo = [&](int i, int j, float x) {
+            if (do_bp)
+                x = update(x, __builtin_fmaf((float)(x0 - 1 + j) + 0.5f - origin_shift, bct, shift - 0.5f),
+                           (float)(y0 - 1 + i) + 0.5f - origin_shift);
+            const bool in = (uint32_t)(y0 - 1 + i) < (uint32_t)N && (uint32_t)(x0 - 1 + j) < (uint32_t)N;
+            tile[i * si + j * sj] = in ? x : 0.0f;
+        };
+        halo(hi, hj, hv);
+        if (threadIdx.x < 4)
+            halo(ci, cj, cv);
     }
-    // Halo ring (4 * 65 entries): updated here, written by the neighbours.
-    for (int e = threadIdx.x; e < 4 * (kSl - 1); e += 256) {
-        int i, j;
-        if (e < kSl) {
-            i = 0;
-            j = e;
-        } else if (e < 2 * kSl) {
-            i = kSl - 1;
-            j = e - kSl;
-        } else if (e < 2 * kSl + kSt) {
-            i = e - 2 * kSl + 1;
-            j = 0;
-        } else {
-            i = e - 2 * kSl - kSt + 1;
-            j = kSl - 1;
-        }
-        const int py = y0 - 1 + i, px = x0 - 1 + j;
-        float v = 0.0f;
-        if (py >= 0 && py < N && px >= 0 && px < N) {
-            v = gload(xin, (uint32_t)py * (uint32_t)N + (uint32_t)px);
-            if (do_bp) {
-                float a, t0, t1;
-                bp_taps(px, py, a, t0, t1);
-                v = __builtin_fmaf(__builtin_fmaf(a, t1 - t0, t0), gain, v);
-            }
-        }
-        tile[i * kSl + j] = v;
-    }
-    if (fp_angle < 0 || fp_angle >= S->n_angles)
+    if (!do_fp)
         return; // uniform over the block
-    __syncthreads();
 
     // FP of fp_angle over the tile (the fast FP's geometry, exact anchors)
-    const float st = gload(trig, 2 * fp_angle), ct = gload(trig, 2 * fp_angle + 1);
-    const bool hor = !(fabsf(st) <= fabsf(ct));
+    const double inv_det = hor ? -(double)st : (double)ct;
     const double det_step = hor ? -1.0 / (double)st : 1.0 / (double)ct;
     const double step = hor ? (double)ct / (double)st : (double)st / (double)ct;
     const double C = -0.5 * (double)N * step + 0.5 * (double)N;
-    const int l0 = hor ? x0 : y0, p_base = hor ? y0 : x0;
-    const int nl = min(kSt, N - l0);
-    int s_lo, s_hi;
-    sart_candidates(det_step, step, C, (double)axis_f, l0, l0 + nl - 1, p_base, D, s_lo, s_hi);
+    const int l0 = hor ? x0 : y0, p_base = hor ? y0 : x0, nl = min(kSt, N - l0);
+    // Candidate rays: those whose tap position falls in [p_base - 3, p_base + 67)
+    // on a line of the tile; pos(s, l) = (s + 0.5 - axis) det_step + C + l step is
+    // affine in (s, l), so the set lies between the corner solutions (one more
+    // ray of margin each side).
+    const double s_at = ((double)p_base + 0.5 - C - (double)l0 * step) * inv_det - 0.5 + (double)axis_f;
+    const double sa = -3.0 * inv_det, sb = 67.0 * inv_det, sl = -(double)(nl - 1) * step * inv_det;
+    const int s_lo = max((int)floor(s_at + fmin(sa, sb) + fmin(sl, 0.0)) - 1, 0);
+    const int s_hi = min((int)ceil(s_at + fmax(sa, sb) + fmax(sl, 0.0)) + 1, D - 1);
     if (s_hi - s_lo + 1 > kSartRays && threadIdx.x == 0)
         atomicOr(err, 8); // cannot happen (at most 98): reported, never silent
-    const int r = threadIdx.x & (kSartRays - 1), h = threadIdx.x / kSartRays;
+    const int n_cand = max(min(s_hi - s_lo + 1, kSartRays), 0);
+    __syncthreads();
+    // thread: ray s_lo + r, lines [l0 + 32 h, + 32) (the candidates of both
+    // halves side by side, so that whole waves are left over)
+    const int h = (int)threadIdx.x >= n_cand, r = (int)threadIdx.x - (h ? n_cand : 0);
     const int s = s_lo + r;
     const float rot = diff / 2.0f;
-    const bool cand = s <= s_hi;
+    const bool cand = r < n_cand;
     const bool on = cand && !((diff < 0 && (float)s < fabsf(diff)) || (diff > 0 && (float)s > required_width));
     float acc = 0.0f;
     if (on) {
         const double tdet = ((0.5 + (double)rot) + (double)s) - (double)(0.5f * (float)D);
         const double q0 = tdet * det_step + C - 0.5; // tap coordinate at line 0
         const float q0f = (float)q0, se = (float)step;
-        const int c_min = p_base == 0 ? -1 : p_base, c_max = p_base + kSt - 1;
-        int lb = l0 + 32 * h, le = min(lb + 32, l0 + nl);
-        if (fabs(step) > 1e-9) { // lines whose tap is within one position of [c_min, c_max + 1)
-            const double la = ((double)c_min - 1.0 - q0) / step, lz = ((double)c_max + 2.0 - q0) / step;
-            lb = max(lb, (int)floor(fmin(la, lz)) - 1);
-            le = min(le, (int)ceil(fmax(la, lz)) + 2);
-        }
-        for (int l = lb; l < le; ++l) {
-            const float qa = __builtin_fmaf((float)l, se, q0f);
-            const int c0 = cvt_flr(qa);
-            if (c0 >= c_min && c0 <= c_max) {
-                const float a = __builtin_amdgcn_fractf(qa);
-                const int i0 = c0 - p_base + 1, li = l - l0 + 1; // staged indices, i0 in [0, 64]
-                const float t0 = hor ? tile[i0 * kSl + li] : tile[li * kSl + i0];
-                const float t1 = hor ? tile[(i0 + 1) * kSl + li] : tile[li * kSl + i0 + 1];
-                acc = __builtin_fmaf(a, t1 - t0, acc + t0);
+        const int first = p_base == 0 ? 0 : 1; // entries first .. 64 of a line hold the tile's own lower taps
+        const int li0 = 32 * h, n_lines = min(32, nl - li0);
+        float l = (float)(l0 + li0);
+        const float *L = tile + (li0 + 1) * kSs;
+        // four lines at a time (the tile holds them all; those past the image
+        // are not added), their taps in flight before the first is used
+        for (int q = 0; q < n_lines; q += 4) {
+            float a[4], t0[4], t1[4];
+            bool own[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float qa = __builtin_fmaf(l, se, q0f);
+                const int i0 = cvt_flr(qa) - (p_base - 1); // staged index of the lower tap
+                own[e] = (uint32_t)(i0 - first) <= (uint32_t)(kSt - first) && q + e < n_lines;
+                a[e] = __builtin_amdgcn_fractf(qa);
+                const float *t = L + (q + e) * kSs + min((uint32_t)i0, (uint32_t)kSt);
+                t0[e] = t[0];
+                t1[e] = t[1];
+                l += 1.0f;
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float sum = __builtin_fmaf(a[e], t1[e] - t0[e], acc + t0[e]);
+                acc = own[e] ? sum : acc;
             }
         }
     }
-    if (h == 1)
+    if (h == 1 && cand)
         half_sum[r] = acc;
     __syncthreads();
-    if (h == 0 && cand) {
+    if (h == 0) {
         const int band = hor ? tx : ty, slot = (hor ? ty : tx) % 3;
         S->part[((size_t)band * 3 + (size_t)slot) * (size_t)D + (size_t)s] = acc + half_sum[r];
     }
@@ -1482,17 +1490,33 @@ __global__ __launch_bounds__(256) void k_sart_rows(const uirk_sart_slice *__rest
         const int nt = (N + kSt - 1) / kSt;
         const float *part = uniform(S->part);
         float sum = 0.0f;
-        for (int band = 0; band < nt; ++band) {
-            const int la = band * kSt, lb = min(la + kSt - 1, N - 1);
-            const double ca = p0 + (double)la * step - 0.5, cb = p0 + (double)lb * step - 0.5;
-            int lo = (int)floor(fmin(ca, cb)) - 1, hi = (int)floor(fmax(ca, cb)) + 1;
-            if (hi < -1 || lo > N - 1)
-                continue;
-            lo = max(lo, -1);
-            hi = min(hi, N - 1);
-            const int t_lo = lo < 0 ? 0 : lo / kSt, t_hi = hi < 0 ? 0 : hi / kSt;
-            for (int t = t_lo; t <= t_hi; ++t)
-                sum += part[((size_t)band * 3 + (size_t)(t % 3)) * (size_t)D + (size_t)s];
+        // four bands at a time, at most three tiles each: their partials are all
+        // in flight before the first is added
+        constexpr int kBands = 4;
+        for (int band0 = 0; band0 < nt; band0 += kBands) {
+            float v[kBands][3];
+            int n_tiles[kBands];
+#pragma unroll
+            for (int e = 0; e < kBands; ++e) {
+                const int band = band0 + e, la = band * kSt, lb = min(la + kSt - 1, N - 1);
+                const double ca = p0 + (double)la * step - 0.5, cb = p0 + (double)lb * step - 0.5;
+                int lo = (int)floor(fmin(ca, cb)) - 1, hi = (int)floor(fmax(ca, cb)) + 1;
+                const bool in = band < nt && hi >= -1 && lo <= N - 1;
+                lo = max(lo, -1);
+                hi = min(hi, N - 1);
+                const int t_lo = lo < 0 ? 0 : lo / kSt, t_hi = hi < 0 ? 0 : hi / kSt;
+                n_tiles[e] = in ? t_hi - t_lo + 1 : 0;
+#pragma unroll
+                for (int t = 0; t < 3; ++t)
+                    v[e][t] = t < n_tiles[e] ? part[((size_t)band * 3 + (size_t)((t_lo + t) % 3)) * (size_t)D + (size_t)s]
+                                             : 0.0f;
+            }
+#pragma unroll
+            for (int e = 0; e < kBands; ++e)
+#pragma unroll
+                for (int t = 0; t < 3; ++t)
+                    if (t < n_tiles[e])
+                        sum += v[e][t];
         }
         w = bval + sum * S->corr;
     }
@@ -1504,11 +1528,13 @@ __global__ __launch_bounds__(256) void k_sart_rows(const uirk_sart_slice *__rest
 
 template <typename T, typename TI>
 int launch_sart(const uirk_sart_slice *sl, const uirk_asd_state *state, int n_slices, int max_n, int bp_angle,
-                int fp_angle, int *err, hipStream_t st)
+                int fp_angle, int n_xcd, int *err, hipStream_t st)
 {
     const int t = (max_n + kSt - 1) / kSt;
-    hipLaunchKernelGGL((k_sart_step<T, TI>), dim3(t * t, n_slices), dim3(256), 0, st, sl, state, bp_angle, fp_angle,
-                       err);
+    const int nx = n_xcd > 0 ? n_xcd : 1;
+    // bands in turns of one per XCD; a slice smaller than the largest leaves the last ones
+    hipLaunchKernelGGL((k_sart_step<T, TI>), dim3(nx * ((t + nx - 1) / nx) * t, n_slices), dim3(256), 0, st, sl, state,
+                       bp_angle, fp_angle, nx, err);
     return (int)hipGetLastError();
 }
 
@@ -1785,7 +1811,7 @@ int uirk_ray_weights64(const float *d_trig, int n, int n_dets, int n_angles, flo
 }
 
 int uirk_sart_step(const uirk_sart_slice *d_slices, const uirk_asd_state *d_state, int n_slices, int max_n,
-                   int dtype, int img_dtype, int bp_angle, int fp_angle, int *d_err, void *stream)
+                   int dtype, int img_dtype, int bp_angle, int fp_angle, int n_xcd, int *d_err, void *stream)
 {
     if (!d_slices || !d_state || n_slices > 65535 || max_n > 16384)
         return (int)hipErrorInvalidValue;
@@ -1795,12 +1821,12 @@ int uirk_sart_step(const uirk_sart_slice *d_slices, const uirk_asd_state *d_stat
     if (img_dtype == UIR_DTYPE_F32) {
         switch (dtype) {
         case UIR_DTYPE_F16:
-            return launch_sart<__half, float>(d_slices, d_state, n_slices, max_n, bp_angle, fp_angle, d_err, st);
+            return launch_sart<__half, float>(d_slices, d_state, n_slices, max_n, bp_angle, fp_angle, n_xcd, d_err, st);
         case UIR_DTYPE_BF16:
-            return launch_sart<__hip_bfloat16, float>(d_slices, d_state, n_slices, max_n, bp_angle, fp_angle, d_err,
-                                                      st);
+            return launch_sart<__hip_bfloat16, float>(d_slices, d_state, n_slices, max_n, bp_angle, fp_angle, n_xcd,
+                                                      d_err, st);
         case UIR_DTYPE_F32:
-            return launch_sart<float, float>(d_slices, d_state, n_slices, max_n, bp_angle, fp_angle, d_err, st);
+            return launch_sart<float, float>(d_slices, d_state, n_slices, max_n, bp_angle, fp_angle, n_xcd, d_err, st);
         default: return (int)hipErrorInvalidValue;
         }
     }
@@ -1808,10 +1834,10 @@ int uirk_sart_step(const uirk_sart_slice *d_slices, const uirk_asd_state *d_stat
         return (int)hipErrorInvalidValue;
     switch (dtype) {
     case UIR_DTYPE_F16:
-        return launch_sart<__half, __half>(d_slices, d_state, n_slices, max_n, bp_angle, fp_angle, d_err, st);
+        return launch_sart<__half, __half>(d_slices, d_state, n_slices, max_n, bp_angle, fp_angle, n_xcd, d_err, st);
     case UIR_DTYPE_BF16:
         return launch_sart<__hip_bfloat16, __hip_bfloat16>(d_slices, d_state, n_slices, max_n, bp_angle, fp_angle,
-                                                           d_err, st);
+                                                           n_xcd, d_err, st);
     default: return (int)hipErrorInvalidValue;
     }
 }

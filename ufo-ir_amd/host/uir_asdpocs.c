@@ -230,6 +230,7 @@ static uir_status launch_asd_iteration(uir_batch *b, const uir_asdpocs_params *p
      * angle j, from buffer j % 2 to (j + 1) % 2 (x, g); the last launch only
      * backprojects.  An odd launch count leaves the image in g. */
     const uint32_t A = a->a_max;
+    const int n_xcd = uirk_plan_num_xcd();
     for (uint32_t pass = 0; pass < p->df_iterations && a->line; ++pass)
         for (uint32_t j = 0; j < A; ++j)
             HIP(uirk_sart_line(a->d_sart[0], a->d_state, S, (int)a->n_max, (int)a->d_max, b->sdt, b->idt, (int)j, st),
@@ -237,8 +238,8 @@ static uir_status launch_asd_iteration(uir_batch *b, const uir_asdpocs_params *p
     for (uint32_t pass = 0; pass < p->df_iterations && !a->line; ++pass) {
         for (uint32_t j = 0; j <= A; ++j) {
             const int fp = j < A ? (int)j : -1;
-            HIP(uirk_sart_step(a->d_sart[j % 2], a->d_state, S, (int)a->n_max, b->sdt, b->idt, (int)j - 1, fp, b->d_err,
-                               st), "SART step launch");
+            HIP(uirk_sart_step(a->d_sart[j % 2], a->d_state, S, (int)a->n_max, b->sdt, b->idt, (int)j - 1, fp, n_xcd,
+                               b->d_err, st), "SART step launch");
             if (fp >= 0)
                 HIP(uirk_sart_rows(a->d_sart[j % 2], S, (int)a->d_max, b->sdt, fp, st), "SART residual launch");
         }
