@@ -62,8 +62,11 @@ def test_bp_matches_oracle(res, n, d, a, step):
 @pytest.mark.parametrize("n,d,a,axis", [
     (1, 1, 1, -1.0), (3, 5, 2, -1.0), (64, 64, 9, -1.0),
     (71, 101, 12, -1.0), (130, 184, 10, 85.25),   # a last block of 7 and of 2 lines; inactive detectors
-    (640, 906, 6, -1.0), (641, 907, 6, -1.0),     # both sides of the staged work table's line
-    (200, 283, 40, 260.5),
+    (640, 906, 6, -1.0), (641, 907, 6, -1.0), (200, 283, 40, 260.5),
+    (1024, 1449, 5, -1.0), (1025, 1450, 5, -1.0),  # both sides of the work table's line in the edge
+    (9, 17, 5294, -1.0), (9, 17, 5295, -1.0),      # and in the rays: 89998 and 90015
+    (71, 101, 900, 30.25), (63, 200, 460, -1.0),   # last chunks of 7 and 31 lines; inactive detectors
+    (33, 91, 13000, -1.0),                         # items of 8 angles
 ])
 def test_fp_bit_exact(res, n, d, a, axis):
     """The FP runs the reference's operations in its order

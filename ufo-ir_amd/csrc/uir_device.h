@@ -226,7 +226,7 @@ typedef struct {
 /* Tile shapes of the fast path, chosen per geometry by the autotuner
  * (host/uir_tune.c): FP angles per work item (16, 8 or 32), BP angles per staged
  * batch (32 or 16) and BP tile rows (64 or 32; tiles are 64 pixels wide).
- * The reference-compatible mode takes the default {16, 32, 64} only. */
+ */
 typedef struct {
     int32_t fp_angles, bp_angles, bp_rows;
     /* FP staging: 0 = (e, d) pairs (k_fp_pairs, windows up to UIRK_FP_WMAX),
@@ -238,15 +238,19 @@ typedef struct {
 /* Footprint width limit of a tile's FP. */
 #define UIRK_TILE_FP_WMAX(t) ((t).fp_single ? UIRK_FP_WMAX_SINGLE : UIRK_FP_WMAX)
 
-/* mode: 0 = reference-compatible FP32 arithmetic (FP only), 1 = fast path (FP32 math on
- * FP32 / FP16 / BF16 storage), 3 = (BP only) the fast path over slice pairs
+/* The reference-compatible FP (FP32) of one slice over a work table planned
+ * with at most `angles` (4 or 8) angles an item and windows of UIRK_FP_WMAX. */
+int uirk_fp_ref_table(const uirk_slice *one, const uirk_fp_item *d_items, int n_items, int angles,
+                      const uirk_xcd_part *part, int grid, int *d_err, void *stream);
+
+/* mode: 1 = fast path (FP32 math on FP32 / FP16 / BF16 storage), 3 = (BP only) the fast path over slice pairs
  * (items with pair set cover slices slice and slice + 1 of one geometry, with
  * the same results as mode 1; d_slices required), 4 = (BP only) mode 2 over
  * slice pairs, 2 = the fast path with the line model (weights
  * from each slice's `line` table; the tile's bp_rows (64 or 32) only, the rest
  * default; BP: pix_w, when given, multiplies the update).  dtype: uir_dtype (FP32 / FP16 / BF16) of the
  * sinogram buffers (b, r); img_dtype: of the image buffers (x, x_out), either
- * dtype or FP32 (the reference-compatible mode takes FP32 only).  d_slices: device
+ * dtype or FP32.  d_slices: device
  * descriptor array indexed by item.slice, or NULL to use *one (host memory,
  * passed by value as a kernel argument; item.slice must then be 0).
  * err: device int, set non-zero if a footprint exceeded the staging window. */
@@ -287,10 +291,16 @@ void uirk_plan_trig(const float *sin_lut, const float *cos_lut, uint32_t n, floa
  * that the hardware's dispatch balances the items' uneven costs. */
 int uirk_plan_grid_xcd(const uirk_xcd_part *part, int n_items);
 int uirk_plan_num_xcd(void);
+/* 4 workgroups per CU of the current device. */
+int uirk_plan_device_slots(void);
 /* Splits items [0, n) into n_xcd contiguous ranges of about equal total cost
  * (cost[i] >= 0; NULL = unit cost). */
 void uirk_plan_xcd(const double *cost, int n, int n_xcd, uirk_xcd_part *out);
 double uirk_fp_item_cost(const uirk_fp_item *it);
+/* Orders each XCD's range of an FP table by falling cost, so that the light
+ * items fill in at the end of a launch.  For tables of one slice (few
+ * workgroups per CU); a table over many slices stays slice by slice. */
+void uirk_plan_sort_fp(uirk_fp_item *v, const uirk_xcd_part *part);
 /* BP slice pairs halve the workgroups of a launch and hold fewer waves per
  * SIMD, so they are used only while the paired table keeps at least this
  * many items: 4 workgroups per CU of the current device, or the value of the

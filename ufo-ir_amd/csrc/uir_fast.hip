@@ -1,7 +1,7 @@
 // uir_fast.hip -- table-driven, LDS-staged Joseph projector pair for gfx950.
 //
 // Two paths:
-//   reference-compatible FP (k_fp_tab with REF): the reference's FP32
+//   reference-compatible FP (k_fp_ref_tab): the reference's FP32
 //                 arithmetic operation for operation (exact incremental float
 //                 ray stepping from the double start coordinate, 64-sample
 //                 blocked sums), bit-identical to the one-thread-per-ray
@@ -12,8 +12,8 @@
 //                 epilogues.  Its FP is k_fp_pairs (staged (e, d) pairs, one
 //                 float add for the index and one FMA per sample) or, for
 //                 geometries whose angle blocks need windows wider than the
-//                 pairs' (sparse angles on large images), k_fp_tab without REF
-//                 (single staged values, fract); its BP is k_bp_tab.
+//                 pairs' (sparse angles on large images), k_fp_tab (single
+//                 staged values, fract); its BP is k_bp_tab.
 // Work is described by tables (uirk_fp_item / uirk_bp_item) over any number
 // of slices of any geometry; the kernels stride over the table (launched with
 // one workgroup per item, so that the hardware's dispatch balances the items'
@@ -413,10 +413,239 @@ __device__ __forceinline__ void fast_ray(const float *trig, int ang, bool hor, d
 // ------------------------------------------------------------------------
 // Forward projection
 // ------------------------------------------------------------------------
-// FP over a work table with single-value staging: the reference-compatible
-// FP (REF) and the fast path for geometries whose angle blocks need windows
-// wider than the pair staging holds (fp_single tiles).
-template <typename T, typename TI, bool REF, int APT>
+// The reference-compatible FP over a work table (FP32): a thread follows the
+// rays of one detector at kRefA angles, with the reference's float stepping and
+// 64-sample block sums; a chunk of kRefL lines of the workgroup's footprint is
+// staged in LDS at a time.  What bounds it is the VALU (12 operations a sample,
+// three of them at half rate) and the wait for each chunk, so: the chunk's
+// window comes from the first and last active ray of each angle (a ray's
+// position is monotone in its detector) by lane reads; 6 workgroups fit a CU,
+// and the host hands out an XCD's items by falling cost, so that the CUs end
+// together; chunks end where blocks do.  The items hold 8 angles where there
+// are many of them, else 4 (host/uir_tasks.c).  1024 / 720 / 1448 takes 267 us,
+// 777 / 401 / 1099 110, 2048 / 900 / 2897 1114, from 321, 170 and 1323 with
+// items of 16 angles in table order, windows by wave shuffles and clamped
+// loads.  Also measured: 16-line chunks 293 / 137 / 1155 with 8 angles and
+// 314 / 155 / 1172 with 16.
+constexpr int kRefL = 32;           // lines per chunk: divides the reference's 64-sample block
+constexpr int kRefW = UIRK_FP_WMAX; // widest window
+constexpr int kRefS = kRefW + 1;    // stride of a staged line (odd: transposed stores hit distinct banks)
+
+__device__ __forceinline__ float lane_f32(float v, int lane)
+{
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+
+// Stages lines [l0, l0 + kRefL) x positions [pmin, pmin + W) to lds[line * kRefS
+// + position - pmin], zero outside the image.  The buffer resource of the
+// transposed staging starts at the window's first row, so that offsets below
+// and past the window's rows stay beyond it at any image size.
+__device__ __forceinline__ void fp_stage_ref(float (&lds)[kRefL * kRefS], const float *img, int N, bool hor, int l0,
+                                             int pmin, int W, int lane, int wave)
+{
+    if (hor) {
+        // line = column l0 + lane % kRefL, position = row pmin + p: a wave
+        // instruction covers kRefL columns of kSub rows; columns past the
+        // image are lines that are never sampled
+        const int r0 = max(pmin, 0), r1 = min(pmin + W, N);
+        const __amdgpu_buffer_rsrc_t r = buf_rsrc(img + (size_t)r0 * (size_t)N, (uint32_t)(r1 - r0) * (uint32_t)N);
+        constexpr int kSub = 64 / kRefL;
+        const int l = lane & (kRefL - 1), p0 = kSub * wave + lane / kRefL;
+        const int o0 = (pmin - r0 + p0) * N + l0 + l;
+        for (int pb = 0; pb < W; pb += 64) {
+            float v[kRefL / 4];
+#pragma unroll
+            for (int e = 0; e < kRefL / 4; ++e)
+                v[e] = bload(r, img, o0 + (pb + 4 * kSub * e) * N);
+#pragma unroll
+            for (int e = 0; e < kRefL / 4; ++e)
+                lds[l * kRefS + pb + p0 + 4 * kSub * e] = v[e];
+        }
+    } else {
+        // line = row l0 + l, position = column pmin + p: a wave takes every fourth line
+        for (int pb = 0; pb < W; pb += 64) {
+            // opaque: an immediate part of the offset would leave a negative
+            // rest, which the range check takes for out of range
+            int c = pmin + pb + lane;
+            asm("" : "+v"(c));
+            float v[kRefL / 4];
+#pragma unroll
+            for (int e = 0; e < kRefL / 4; ++e) {
+                const int line = l0 + wave + 4 * e;
+                v[e] = bload(buf_rsrc(img + (size_t)line * (size_t)N, line < N ? (uint32_t)N : 0u), img, c);
+            }
+#pragma unroll
+            for (int e = 0; e < kRefL / 4; ++e)
+                lds[(wave + 4 * e) * kRefS + pb + lane] = v[e];
+        }
+    }
+}
+
+template <int kRefA> // angles per wave
+__global__ __launch_bounds__(256, 6) void k_fp_ref_tab(uirk_slice S, const uirk_fp_item *__restrict__ items, int n_items,
+                                                       uirk_xcd_part part, int *__restrict__ err)
+{
+    __shared__ float lds[kRefL * kRefS];
+    __shared__ float red[2][4];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const ItemRange range = item_range(part, n_items);
+    const float *img = (const float *)S.x;
+    const int N = S.n, D = S.n_dets;
+
+    for (int it = range.first; it < range.end; it += range.stride) {
+        const uirk_fp_item item = items[it];
+        if (item.na > 4 * kRefA) { // planned for a wider variant: report, never drop angles silently
+            if (threadIdx.x == 0)
+                atomicOr(err, 4);
+            continue;
+        }
+        const int s = item.d0 + lane;
+        const bool hor = item.dir == 0;
+
+        // projector-parallel-joseph.cl:51-66 (detector quantities use n_dets)
+        const float required_width = S.axis * 2;
+        const float diff = (float)D - required_width;
+        const float rot = diff / 2.0f;
+        const float origin_shift = (float)N / 2.0f;
+        const bool in_range = s < D;
+        const bool det_on = in_range && !((diff < 0 && (float)s < fabsf(diff)) || (diff > 0 && (float)s > required_width));
+        const double tdet = ((0.5 + (double)rot) + (double)s) - (double)(0.5f * (float)D);
+
+        float pos[kRefA], stp[kRefA], acc[kRefA], inner[kRefA];
+#pragma unroll
+        for (int j = 0; j < kRefA; ++j) {
+            const int k = wave * kRefA + j;
+            const int ang = item.a0 + (k < item.na ? k : 0);
+            const float st = S.trig[2 * ang], ct = S.trig[2 * ang + 1];
+            float det_step;
+            if (hor) {
+                det_step = -1.0f / st;
+                stp[j] = ct / st;
+            } else {
+                det_step = 1.0f / ct;
+                stp[j] = st / ct;
+            }
+            // start coordinate: double expression rounded to float (:73, :134)
+            pos[j] = (float)(tdet * (double)det_step + (double)((-origin_shift) * stp[j]) + (double)(0.5f * (float)N));
+            acc[j] = 0.0f;
+            inner[j] = 0.0f;
+        }
+        const unsigned long long active = __ballot(det_on); // the same in every wave
+        const int l_lo = active ? item.l_lo & ~(kRefL - 1) : item.l_hi;
+        // lines before l_lo read only the zero border: their float steps alone
+        for (int l = 0; l < l_lo; l += kRefL) {
+#pragma unroll
+            for (int e = 0; e < kRefL; ++e)
+#pragma unroll
+                for (int j = 0; j < kRefA; ++j)
+                    pos[j] += stp[j];
+        }
+        const int first = active ? __builtin_ctzll(active) : 0, last = active ? 63 - __builtin_clzll(active) : 0;
+        // inactive rays walk with the first active one, in the window; their
+        // sums are never written
+        if (!det_on) {
+#pragma unroll
+            for (int j = 0; j < kRefA; ++j)
+                pos[j] = lane_f32(pos[j], first);
+        }
+        for (int l0 = l_lo; l0 < item.l_hi; l0 += kRefL) {
+            const int nl = min(kRefL, item.l_hi - l0);
+            float lo = 3.0e38f, hi = -3.0e38f;
+#pragma unroll
+            for (int j = 0; j < kRefA; ++j) {
+                if (wave * kRefA + j < item.na) { // uniform
+                    const float a = lane_f32(pos[j], first), b = lane_f32(pos[j], last);
+                    const float d = (float)(nl - 1) * stp[j];
+                    lo = fminf(lo, fminf(fminf(a, b), fminf(a + d, b + d)));
+                    hi = fmaxf(hi, fmaxf(fmaxf(a, b), fmaxf(a + d, b + d)));
+                }
+            }
+            if (lane == 0) {
+                red[0][wave] = lo;
+                red[1][wave] = hi;
+            }
+            __syncthreads(); // also: the previous chunk's reads are done
+            lo = fminf(fminf(red[0][0], red[0][1]), fminf(red[0][2], red[0][3]));
+            hi = fmaxf(fmaxf(red[1][0], red[1][1]), fmaxf(red[1][2], red[1][3]));
+            const int pmin = __builtin_amdgcn_readfirstlane((int)floorf(lo - 0.5f) - 1);
+            const int W = __builtin_amdgcn_readfirstlane((int)floorf(hi - 0.5f) + 3) - pmin;
+            // A footprint wider than the staging window is reported and the
+            // chunk's samples are skipped (the host sizes angle blocks so that
+            // this does not happen); no sample ever reads outside the window.
+            const bool overflow = W > kRefW;
+            if (overflow && threadIdx.x == 0)
+                atomicOr(err, 1);
+            const bool outside = overflow || pmin + W <= 0 || pmin >= N;
+            if (!outside)
+                fp_stage_ref(lds, img, N, hor, l0, pmin, W, lane, wave);
+            __syncthreads();
+            if (outside || wave * kRefA >= item.na) {
+                // zero samples, or no angle for this wave: the stepping goes on
+#pragma unroll
+                for (int e = 0; e < kRefL; ++e)
+                    if (e < nl)
+#pragma unroll
+                        for (int j = 0; j < kRefA; ++j)
+                            pos[j] += stp[j];
+            } else {
+                const float *L = lds - pmin;
+                auto line = [&](const float *P) {
+                    float t0[kRefA], t1[kRefA], b[kRefA];
+#pragma unroll
+                    for (int j = 0; j < kRefA; ++j) {
+                        const float v = pos[j] - 0.5f;
+                        const float fv = floorf(v);
+                        const int i0 = (int)fv;
+                        b[j] = v - fv;
+                        t0[j] = P[i0];
+                        t1[j] = P[i0 + 1];
+                        pos[j] += stp[j];
+                    }
+#pragma unroll
+                    for (int j = 0; j < kRefA; ++j) {
+                        const float omb = 1.0f - b[j];
+                        inner[j] += omb * t0[j] + b[j] * t1[j];
+                    }
+                };
+                int l = 0;
+                for (; l + 2 <= nl; l += 2, L += 2 * kRefS) {
+                    line(L);
+                    line(L + kRefS);
+                }
+                if (l < nl)
+                    line(L);
+            }
+            if (((l0 + kRefL) & 63) == 0) { // 64-sample blocks (:82-90) end with a chunk
+#pragma unroll
+                for (int j = 0; j < kRefA; ++j) {
+                    acc[j] += inner[j];
+                    inner[j] = 0.0f;
+                }
+            }
+        }
+
+        const float *b = (const float *)S.b;
+        float *r = (float *)S.r;
+#pragma unroll
+        for (int j = 0; j < kRefA; ++j) {
+            const int k = wave * kRefA + j;
+            if (!in_range || k >= item.na)
+                continue;
+            const uint32_t o = (uint32_t)(item.a0 + k) * (uint32_t)D + (uint32_t)s;
+            float w = b[o];
+            if (det_on) // an inactive detector: the reference leaves the value as read
+                w = w + (acc[j] + inner[j]) * S.corr; // :92-94
+            if (S.ray_w)
+                w = w * S.ray_w[o];
+            r[o] = w;
+        }
+    }
+}
+
+// Fast-path FP over a work table with single-value staging, for geometries
+// whose angle blocks need windows wider than the pair staging holds (fp_single
+// tiles).
+template <typename T, typename TI, int APT>
 __global__ __launch_bounds__(256) void k_fp_tab(const uirk_slice *__restrict__ slices, uirk_slice one,
                                                 const uirk_fp_item *__restrict__ items, int n_items,
                                                 uirk_xcd_part part, int *__restrict__ err)
@@ -445,12 +674,11 @@ __global__ __launch_bounds__(256) void k_fp_tab(const uirk_slice *__restrict__ s
         const float required_width = S->axis * 2;
         const float diff = (float)D - required_width;
         const float rot = diff / 2.0f;
-        const float origin_shift = (float)N / 2.0f;
         const bool in_range = s < D;
         const bool det_on = in_range && !((diff < 0 && (float)s < fabsf(diff)) || (diff > 0 && (float)s > required_width));
         const double tdet = ((0.5 + (double)rot) + (double)s) - (double)(0.5f * (float)D);
 
-        float pos[APT], stp[APT], acc[APT], inner[APT];
+        float pos[APT], stp[APT], acc[APT];
         double p0d[APT], sd[APT];
         bool on[APT];
 #pragma unroll
@@ -459,49 +687,23 @@ __global__ __launch_bounds__(256) void k_fp_tab(const uirk_slice *__restrict__ s
             on[j] = det_on && k < item.na;
             const int ang = item.a0 + (k < item.na ? k : 0);
             const float st = gload(trig, 2 * ang), ct = gload(trig, 2 * ang + 1);
-            double p0;
-            if (REF) {
-                float det_step, step;
-                if (hor) {
-                    det_step = -1.0f / st;
-                    step = ct / st;
-                } else {
-                    det_step = 1.0f / ct;
-                    step = st / ct;
-                }
-                // start coordinate: double expression rounded to float (:73, :134)
-                p0 = tdet * (double)det_step + (double)((-origin_shift) * step) + (double)(0.5f * (float)N);
-                sd[j] = (double)step;
-            } else {
-                // exact coordinates: steps and chunk anchors in double
-                const double det_step = hor ? -1.0 / (double)st : 1.0 / (double)ct;
-                sd[j] = hor ? (double)ct / (double)st : (double)st / (double)ct;
-                p0 = tdet * det_step - 0.5 * (double)N * sd[j] + 0.5 * (double)N;
-            }
+            // exact coordinates: steps and chunk anchors in double
+            const double det_step = hor ? -1.0 / (double)st : 1.0 / (double)ct;
+            sd[j] = hor ? (double)ct / (double)st : (double)st / (double)ct;
+            const double p0 = tdet * det_step - 0.5 * (double)N * sd[j] + 0.5 * (double)N;
             p0d[j] = p0;
             pos[j] = (float)p0;
             stp[j] = (float)sd[j];
             acc[j] = 0.0f;
-            inner[j] = 0.0f;
         }
 
-        // Lines before l_lo read only the zero border: the reference-compatible
-        // path replays their float steps exactly, the fast path re-anchors.
-        if (REF) {
-            for (int l = 0; l < item.l_lo; ++l) {
-#pragma unroll
-                for (int j = 0; j < APT; ++j)
-                    pos[j] += stp[j];
-            }
-        }
         for (int l0 = item.l_lo; l0 < item.l_hi; l0 += kFpLines) {
             const int nl = min(kFpLines, item.l_hi - l0);
             // Footprint of this block's rays over the chunk.
             float lo = 3.0e38f, hi = -3.0e38f;
 #pragma unroll
             for (int j = 0; j < APT; ++j) {
-                if (!REF)
-                    pos[j] = (float)(p0d[j] + (double)l0 * sd[j]);
+                pos[j] = (float)(p0d[j] + (double)l0 * sd[j]);
                 if (on[j]) {
                     const float a = pos[j], b = pos[j] + (float)(nl - 1) * stp[j];
                     lo = fminf(lo, fminf(a, b));
@@ -527,61 +729,7 @@ __global__ __launch_bounds__(256) void k_fp_tab(const uirk_slice *__restrict__ s
             // Inactive rays sample a fixed in-window position with zero step;
             // their sums are never written.
             const float park = lo + 1.0f;
-            if (REF) {
-                if (!outside) {
-                    float pp[APT], se[APT];
-#pragma unroll
-                    for (int j = 0; j < APT; ++j) {
-                        pp[j] = on[j] ? pos[j] : park;
-                        se[j] = on[j] ? stp[j] : 0.0f;
-                    }
-                    for (int l = 0; l < nl; ++l) {
-                        const float *L = lds + l * kFpLs - pmin;
-                        float t0[APT], t1[APT], b[APT];
-#pragma unroll
-                        for (int j = 0; j < APT; ++j) {
-                            const float v = pp[j] - 0.5f;
-                            const float fv = floorf(v);
-                            const int i0 = (int)fv;
-                            b[j] = v - fv;
-                            t0[j] = L[i0];
-                            t1[j] = L[i0 + 1];
-                        }
-#pragma unroll
-                        for (int j = 0; j < APT; ++j) {
-                            const float omb = 1.0f - b[j];
-                            inner[j] += omb * t0[j] + b[j] * t1[j];
-                            pp[j] += se[j];
-                        }
-                        if (((l0 + l + 1) & 63) == 0) { // 64-sample blocks (:82-90)
-#pragma unroll
-                            for (int j = 0; j < APT; ++j) {
-                                acc[j] += inner[j];
-                                inner[j] = 0.0f;
-                            }
-                        }
-                    }
-#pragma unroll
-                    for (int j = 0; j < APT; ++j)
-                        if (on[j])
-                            pos[j] = pp[j];
-                } else {
-                    // outside the image: the samples are zero, the exact
-                    // float stepping of the coordinates continues
-                    for (int l = 0; l < nl; ++l) {
-#pragma unroll
-                        for (int j = 0; j < APT; ++j)
-                            pos[j] += stp[j];
-                        if (((l0 + l + 1) & 63) == 0) {
-#pragma unroll
-                            for (int j = 0; j < APT; ++j) {
-                                acc[j] += inner[j];
-                                inner[j] = 0.0f;
-                            }
-                        }
-                    }
-                }
-            } else if (!outside) {
+            if (!outside) {
                 const float off = 0.5f + (float)pmin;
                 float q[APT], st[APT];
 #pragma unroll
@@ -641,8 +789,7 @@ __global__ __launch_bounds__(256) void k_fp_tab(const uirk_slice *__restrict__ s
             const float bval = gload(bsrc, o);
             float w;
             if (on[j]) {
-                const float sum = REF ? acc[j] + inner[j] : acc[j];
-                w = bval + sum * corr; // :92-94
+                w = bval + acc[j] * corr; // :92-94
             } else {
                 w = bval; // inactive detector: the reference leaves the value as read
             }
@@ -1649,11 +1796,11 @@ __global__ __launch_bounds__(256) void k_ray_weights64(const float *__restrict__
     ray_w[(size_t)ang * D + s] = w;
 }
 
-template <typename T, typename TI, bool REF, int APT>
+template <typename T, typename TI, int APT>
 int launch_fp(const uirk_slice *sl, const uirk_slice &one, const uirk_fp_item *items, int n,
               const uirk_xcd_part &part, int grid, int *err, hipStream_t st)
 {
-    hipLaunchKernelGGL((k_fp_tab<T, TI, REF, APT>), dim3(grid), dim3(256), 0, st, sl, one, items, n, part, err);
+    hipLaunchKernelGGL((k_fp_tab<T, TI, APT>), dim3(grid), dim3(256), 0, st, sl, one, items, n, part, err);
     return (int)hipGetLastError();
 }
 
@@ -1684,10 +1831,10 @@ int launch_fp_fast(const uirk_tile &tile, bool line, bool, const uirk_slice *sl,
         return launch_fp_pairs<T, TI, 4, true>(sl, one, items, n, part, grid, err, st);
     if (tile.fp_single) {
         if (tile.fp_angles == 8)
-            return launch_fp<T, TI, false, 2>(sl, one, items, n, part, grid, err, st);
+            return launch_fp<T, TI, 2>(sl, one, items, n, part, grid, err, st);
         if (tile.fp_angles == 32)
-            return launch_fp<T, TI, false, 8>(sl, one, items, n, part, grid, err, st);
-        return launch_fp<T, TI, false, 4>(sl, one, items, n, part, grid, err, st);
+            return launch_fp<T, TI, 8>(sl, one, items, n, part, grid, err, st);
+        return launch_fp<T, TI, 4>(sl, one, items, n, part, grid, err, st);
     }
     if (tile.fp_angles == 8)
         return launch_fp_pairs<T, TI, 2>(sl, one, items, n, part, grid, err, st);
@@ -1787,15 +1934,28 @@ int uirk_fp_table(const uirk_slice *d_slices, const uirk_slice *one, const uirk_
     if (part)
         pt = *part;
     hipStream_t st = (hipStream_t)stream;
-    if (mode == 0) {
-        if (dtype != UIR_DTYPE_F32 || img_dtype != UIR_DTYPE_F32 || tl.fp_angles != UIRK_FP_ANGLES)
-            return (int)hipErrorInvalidValue;
-        return launch_fp<float, float, true, 4>(d_slices, single, d_items, n_items, pt, grid, d_err, st);
-    }
     if (mode != 1 && mode != 2)
         return (int)hipErrorInvalidValue;
     return launch_fast<true>(dtype, img_dtype, tl, mode == 2, false, d_slices, single, d_items, n_items, pt, grid,
                              d_err, st);
+}
+
+int uirk_fp_ref_table(const uirk_slice *one, const uirk_fp_item *d_items, int n_items, int angles,
+                      const uirk_xcd_part *part, int grid, int *d_err, void *stream)
+{
+    if (!one || !part || (angles != 4 && angles != 8))
+        return (int)hipErrorInvalidValue;
+    if (n_items <= 0)
+        return 0;
+    if (grid <= 0 || grid > n_items)
+        grid = n_items;
+    if (angles == 4)
+        hipLaunchKernelGGL(k_fp_ref_tab<1>, dim3(grid), dim3(256), 0, (hipStream_t)stream, *one, d_items, n_items,
+                           *part, d_err);
+    else
+        hipLaunchKernelGGL(k_fp_ref_tab<2>, dim3(grid), dim3(256), 0, (hipStream_t)stream, *one, d_items, n_items,
+                           *part, d_err);
+    return (int)hipGetLastError();
 }
 
 int uirk_ray_weights64(const float *d_trig, int n, int n_dets, int n_angles, float axis, float r_min, float *d_ray_w,

@@ -240,11 +240,8 @@ int uirk_plan_num_xcd(void)
     return nx;
 }
 
-int uirk_plan_pair_min_items(void)
+int uirk_plan_device_slots(void)
 {
-    const char *env = getenv("UIR_PAIR_MIN_ITEMS"); /* override: 0 pairs always */
-    if (env && *env)
-        return atoi(env);
     static int n = 0;
     if (n == 0) {
         int dev = 0, cus = 0;
@@ -255,6 +252,14 @@ int uirk_plan_pair_min_items(void)
             n = 1024;
     }
     return n;
+}
+
+int uirk_plan_pair_min_items(void)
+{
+    const char *env = getenv("UIR_PAIR_MIN_ITEMS"); /* override: 0 pairs always */
+    if (env && *env)
+        return atoi(env);
+    return uirk_plan_device_slots();
 }
 
 int uirk_plan_bp_rows32(size_t items)
@@ -288,6 +293,18 @@ void uirk_plan_xcd(const double *cost, int n, int n_xcd, uirk_xcd_part *out)
     }
     while (x <= n_xcd)
         out->start[x++] = n;
+}
+
+static int by_falling_cost(const void *a, const void *b)
+{
+    const double ca = uirk_fp_item_cost((const uirk_fp_item *)a), cb = uirk_fp_item_cost((const uirk_fp_item *)b);
+    return ca < cb ? 1 : (ca > cb ? -1 : 0);
+}
+
+void uirk_plan_sort_fp(uirk_fp_item *v, const uirk_xcd_part *part)
+{
+    for (int x = 0; x < part->n_xcd; ++x)
+        qsort(v + part->start[x], (size_t)(part->start[x + 1] - part->start[x]), sizeof *v, by_falling_cost);
 }
 
 int uirk_plan_grid_xcd(const uirk_xcd_part *part, int n_items)

@@ -53,7 +53,7 @@ struct uir_task {
     uint32_t plan_gen, plan_n, plan_dets, plan_angles;
     float plan_axis;
     uirk_fp_item *d_fp_items;
-    int n_fp_items;
+    int n_fp_items, fp_angles; /* fp_angles: largest item */
     uirk_xcd_part fp_part;
     float *d_trig;
     int *d_err;
@@ -621,8 +621,18 @@ static uir_status proj_plan(uir_task *p, uint32_t n)
     uirk_fp_vec fv = {0};
     float *trig = (float *)malloc(sizeof(float) * 2 * (p->lut_n ? p->lut_n : 1));
     uir_status s = UIR_OK;
-    if (!trig || uirk_plan_fp(&fv, 0, (int)n, (int)p->n_dets, axis, p->h_sin, p->h_cos, p->runs, p->n_runs,
-                              UIRK_FP_ANGLES, UIRK_FP_WMAX_SINGLE)) {
+    /* Items of 8 angles where they are at least 12 a CU (2048 / 900 / 2897, 20 a
+     * CU: 1114 us against 1208 with 4), else of 4 (1024 / 720 / 1448, 8 a CU: 267
+     * against 278; 777 / 401 / 1099: 110 against 124). */
+    int bad = !trig;
+    for (p->fp_angles = 8; !bad; p->fp_angles = 4) {
+        fv.n = 0;
+        bad = uirk_plan_fp(&fv, 0, (int)n, (int)p->n_dets, axis, p->h_sin, p->h_cos, p->runs, p->n_runs, p->fp_angles,
+                           UIRK_FP_WMAX);
+        if (p->fp_angles == 4 || fv.n >= 3 * (size_t)uirk_plan_device_slots())
+            break;
+    }
+    if (bad) {
         s = uir_set_error(UIR_ERR_OUT_OF_MEMORY, "work table");
         goto done;
     }
@@ -632,13 +642,6 @@ static uir_status proj_plan(uir_task *p, uint32_t n)
         goto done;
     if (!p->d_err && (s = uir_dmalloc((void **)&p->d_err, sizeof(int))) != UIR_OK)
         goto done;
-    if ((s = uir_check_hip(hipMemcpy(p->d_fp_items, fv.v, fv.n * sizeof(uirk_fp_item), hipMemcpyHostToDevice),
-                           "table upload")) != UIR_OK ||
-        (s = uir_check_hip(hipMemcpy(p->d_trig, trig, 2 * sizeof(float) * p->lut_n, hipMemcpyHostToDevice),
-                           "table upload")) != UIR_OK ||
-        (s = uir_check_hip(hipMemset(p->d_err, 0, sizeof(int)), "memset")) != UIR_OK)
-        goto done;
-    p->n_fp_items = (int)fv.n;
     {
         double *cost = (double *)malloc(sizeof(double) * (fv.n ? fv.n : 1));
         if (!cost) {
@@ -648,8 +651,16 @@ static uir_status proj_plan(uir_task *p, uint32_t n)
         for (size_t i = 0; i < fv.n; ++i)
             cost[i] = uirk_fp_item_cost(&fv.v[i]);
         uirk_plan_xcd(cost, (int)fv.n, uirk_plan_num_xcd(), &p->fp_part);
+        uirk_plan_sort_fp(fv.v, &p->fp_part);
         free(cost);
     }
+    if ((s = uir_check_hip(hipMemcpy(p->d_fp_items, fv.v, fv.n * sizeof(uirk_fp_item), hipMemcpyHostToDevice),
+                           "table upload")) != UIR_OK ||
+        (s = uir_check_hip(hipMemcpy(p->d_trig, trig, 2 * sizeof(float) * p->lut_n, hipMemcpyHostToDevice),
+                           "table upload")) != UIR_OK ||
+        (s = uir_check_hip(hipMemset(p->d_err, 0, sizeof(int)), "memset")) != UIR_OK)
+        goto done;
+    p->n_fp_items = (int)fv.n;
     p->plan_gen = p->lut_gen;
     p->plan_n = n;
     p->plan_dets = p->n_dets;
@@ -852,11 +863,16 @@ static void proj_slice(const uir_task *p, uint32_t n, uirk_slice *sl)
     sl->relax = p->relaxation;
 }
 
-/* Images up to this edge take the FP without LDS staging (uirk_fp_blocks with
- * the transpose in front of it), larger ones the work table: 256 / 180 / 367
- * takes 17 us against 80 with the table, 512 / 400 / 725 80 against 111,
- * 777 / 401 / 1099 173 against 170. */
-#define FP_BLOCKS_MAX_N 640
+/* FPs of up to this many rays take uirk_fp_blocks (with the transpose in front
+ * of it), larger ones the work table, whose items follow their rays from end to
+ * end: its time hardly falls below that of one item's walk.  256 / 180 / 367
+ * (66 k rays) takes 20 us against 22 with the table, 512 / 90 / 725 35 against
+ * 54, 1024 / 45 / 1448 65 against 83; 640 / 90 / 905 (81 k) 55 against 53,
+ * 1024 / 66 / 1448 (96 k) 81 against 80; 400 / 180 / 566 (102 k) 38 against 34,
+ * 512 / 400 / 725 110 against 58, 128 / 1000 / 182 24 against 14.  Beyond an
+ * edge of 1024 always the table: the transpose's scratch stays at 4 MiB. */
+#define FP_BLOCKS_MAX_RAYS 90000
+#define FP_BLOCKS_MAX_N 1024
 
 /* forward over all runs (ufo-ir-parallel-projector-task.c:390-408);
  * ray_w != NULL fuses the SIRT ray weighting. */
@@ -865,7 +881,7 @@ static uir_status proj_fp(uir_task *p, uint32_t n, const float *vol, const float
 {
     if (p->line)
         return line_fp(p, n, vol, r_sino, w_sino, ray_w, 0, p->lut_n, 0, p->res->stream);
-    if (n <= FP_BLOCKS_MAX_N && p->lut_n <= 65535) {
+    if (n <= FP_BLOCKS_MAX_N && p->lut_n <= 65535 && (uint64_t)p->lut_n * p->n_dets <= FP_BLOCKS_MAX_RAYS) {
         TRY(proj_limits(p, n));
         float *vol_t = NULL;
         for (uint32_t i = 0; i < p->n_runs && !vol_t; ++i)
@@ -884,8 +900,9 @@ static uir_status proj_fp(uir_task *p, uint32_t n, const float *vol, const float
     sl.b = r_sino;
     sl.r = w_sino;
     sl.ray_w = ray_w;
-    return uir_check_hip(uirk_fp_table(NULL, &sl, p->d_fp_items, p->n_fp_items, &p->fp_part, 0, UIR_DTYPE_F32, UIR_DTYPE_F32, NULL,
-                                       uirk_plan_grid_xcd(&p->fp_part, p->n_fp_items), p->d_err, p->res->stream), "FP launch");
+    return uir_check_hip(uirk_fp_ref_table(&sl, p->d_fp_items, p->n_fp_items, p->fp_angles, &p->fp_part,
+                                           uirk_plan_grid_xcd(&p->fp_part, p->n_fp_items), p->d_err, p->res->stream),
+                         "FP launch");
 }
 
 /* backward over all runs (:410-429).  pix_w == NULL: accumulate form,
