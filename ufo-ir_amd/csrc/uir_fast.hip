@@ -124,19 +124,39 @@ __device__ __forceinline__ float neg_float_of(int n)
     return n == 0 ? -0.0f : __uint_as_float(bits);
 }
 
-// Entry rne_index(x) of an LDS table through a base biased by the bits of
-// 1.5 2^23 (lds_rne_base, once per table): the sample's address is then one
-// shift-add of x + 1.5 2^23's bits.  Unsigned 32-bit arithmetic wraps, so
-// the biased base may lie outside LDS; the sum is the entry's address.
+// Entry rne_index(x) of an LDS table.  Shifts and shift-adds issue at half the
+// rate of float multiply-adds, so the address is one: m = x + 1.5 2^23 is the
+// integer 1.5 2^23 + i, and m 2^-149 size + (base - 1.5 2^23 size) 2^-149 is
+// exactly the denormal whose bits are base + i size, an LDS address (one
+// rounding, of a value that is representable: sizes are 8 or 16 and bases
+// their multiples).  lds_rne_base makes the second term, once per table.
 template <typename E> using lds_ptr = const __attribute__((address_space(3))) E *;
-template <typename E> __device__ __forceinline__ uint32_t lds_rne_base(const E *table)
+template <typename E> __device__ __forceinline__ float lds_rne_base(const E *table)
 {
-    return (uint32_t)(uintptr_t)(lds_ptr<E>)table - 0x4B400000u * (uint32_t)sizeof(E);
+    static_assert(sizeof(E) == 8 || sizeof(E) == 16, "entry size");
+    // -(1.5 2^23 size - base) 2^-149: the mantissa counts down by one per
+    // 8 (16) bytes of base from 1.5 2^26 (2^27) 2^-149
+    constexpr uint32_t kBits = 0x80000000u | ((sizeof(E) == 8 ? 4u : 5u) << 23) | 0x400000u;
+    return __uint_as_float(kBits - (uint32_t)(uintptr_t)(lds_ptr<E>)table / (uint32_t)sizeof(E));
 }
-template <typename E> __device__ __forceinline__ E lds_rne_read(uint32_t base, float x)
+template <typename E> __device__ __forceinline__ E lds_rne_read(float base, float x)
 {
-    const uint32_t a = (uint32_t)__float_as_int(x + 12582912.0f) * (uint32_t)sizeof(E) + base;
-    return *(const E *)(lds_ptr<E>)(uintptr_t)a;
+    const float a = __builtin_fmaf(x + 12582912.0f, __uint_as_float((uint32_t)sizeof(E)), base);
+    return *(const E *)(lds_ptr<E>)(uintptr_t)__float_as_uint(a);
+}
+
+// Column of a lane for the 16-byte reads of a slice pair.  A ds_read_b128
+// serves 16 lanes a clock, in the groups of lanes {0-3, 12-15, 20-27},
+// {4-11, 16-19, 28-31} and the same plus 32 (measured by timing lane pairs on
+// one bank); with 16 adjacent columns in a group, whose entries span at most
+// 16, no two lanes of it use one bank, whatever the angle.  With lane = column
+// the groups span up to 28 entries, and each read took twice as long for
+// |cos| in 0.6 to 0.95.  The BP of 32 slices of 1024 / 720 / 1448 takes 2.18 ms
+// with it and the FMA addresses above, from 2.46.
+__device__ __forceinline__ int pair_column(int lane)
+{
+    // quads of lanes 0..7 of a half wave hold quads 0 4 5 1 6 2 3 7 of columns
+    return (lane & 35) + (int)((0x73261540u >> (lane & 28)) & 7u) * 4;
 }
 
 // The line model's remapped fraction at coordinate x of the pair FP, whose
@@ -1082,6 +1102,7 @@ __global__ __launch_bounds__(256, LINE ? 4 : (PAIR ? (NA == 32 ? 3 : 4) : 6)) vo
     __shared__ float s_base[NA]; // window coordinate at the super-tile's corner
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
+    const int col = PAIR && !LINE ? pair_column(lane) : lane;
     const ItemRange range = item_range(part, n_items);
 
     for (int it = range.first; it < range.end; it += range.stride) {
@@ -1094,7 +1115,7 @@ __global__ __launch_bounds__(256, LINE ? 4 : (PAIR ? (NA == 32 ? 3 : 4) : 6)) vo
         const T *sino2 = PAIR ? uniform((const T *)S2->b) : sino;
         const float *trig = uniform(S->trig);
         const int n_runs = S->n_runs;
-        const int px = item.x0 + lane;
+        const int px = item.x0 + col;
 
         // projector-parallel-joseph.cl:174-190 (detector quantities use n_dets)
         const float axis = S->axis;
@@ -1243,10 +1264,9 @@ __global__ __launch_bounds__(256, LINE ? 4 : (PAIR ? (NA == 32 ? 3 : 4) : 6)) vo
                     // Window coordinates: row q's is fma(-ys_q, st, A), one FMA from
                     // the thread's column term A and the row's offset ys_q in the
                     // super-tile, whatever the tile's rows.  Joseph: less 1/2, so a
-                    // sample's entry is rne_index of it, one float add
-                    // (floor-converts and shifts issue at half the rate of float
-                    // adds), and its address one shift-add.
-                    const float A = __builtin_fmaf((float)lane, ct, s_base[k]);
+                    // sample's entry is rne_index of it, one float add,
+                    // and its address one more FMA.
+                    const float A = __builtin_fmaf((float)col, ct, s_base[k]);
                     if constexpr (LINE) {
                         const float4 L = s_line[k]; // (bp_k, bp_b0, bp_b1, 1/M)
                         if constexpr (PAIR) {
@@ -1296,7 +1316,7 @@ __global__ __launch_bounds__(256, LINE ? 4 : (PAIR ? (NA == 32 ? 3 : 4) : 6)) vo
                             }
                         }
                     } else if (!clamp_u) {
-                        const uint32_t P = lds_rne_base(ldp + k * kBpWb);
+                        const float P = lds_rne_base(ldp + k * kBpWb);
                         // a copy of A per branch: the compiler would otherwise hoist
                         // every row's coordinate above the branch, all live at once
                         float Ab = A;
@@ -1321,7 +1341,7 @@ __global__ __launch_bounds__(256, LINE ? 4 : (PAIR ? (NA == 32 ? 3 : 4) : 6)) vo
                         // u clamped to [edge0, edge1] (:203-210), in window coordinates less 1/2
                         const float wlo = (edge0 - 1.0f) - (float)s_umin[k];
                         const float whi = (edge1 - 1.0f) - (float)s_umin[k];
-                        const uint32_t P = lds_rne_base(ldp + k * kBpWb);
+                        const float P = lds_rne_base(ldp + k * kBpWb);
                         float Ab = A;
                         asm volatile("" : "+v"(Ab));
 #pragma unroll
