@@ -95,6 +95,45 @@ def test_batch_slice_pairs_equal_single_slices(res, storage, monkeypatch):
         assert np.array_equal(bt.image(i), solo.image(0)), (i, c)
 
 
+@pytest.mark.parametrize("model,k,items", [
+    # items of 250 x 250 slices: 16 tiles of 64 rows, 32 of 32; per CU of 256
+    ("joseph", 32, 1024),  # 2 paired items a CU: unpaired, 32 rows
+    ("joseph", 33, 544),   # more: pairs, 32 rows, 32 angles
+    ("joseph", 49, 800),   # more than 3 a CU: 16 angles; a last slice without a partner
+    ("joseph", 66, 528),   # more than 4: 64 rows, 32 angles
+    ("joseph", 98, 784),   # more than 3 in 64 rows: 16 angles
+    ("line", 14, 448), ("line", 16, 256), ("line", 66, 528),
+])
+def test_batch_bp_shapes_equal_single_slices(res, monkeypatch, model, k, items):
+    """Each shape that the rule on the BP's items picks (pairs, tile rows,
+    staged angles) on both sides of its lines: every image equal, bit for bit,
+    to its slice's alone."""
+    monkeypatch.delenv("UIR_PAIR_MIN_ITEMS", raising=False)
+    if uir.probe_ceilings(res)["n_cu"] != 256:
+        pytest.skip("items given for 256 CUs")
+    n, d, a, iters = 250, 355, 21, 2
+    spec = dict(n=n, n_dets=d, n_angles=a, step=float(np.float32(np.pi / a)), relaxation=0.5, model=model,
+                ray_weight_min=0.1 if model == "line" else 0.0)
+    print("case bp shapes", model, k, flush=True)
+    rng = np.random.default_rng(k)
+    sinos = [rng.uniform(0.0, 50.0, (a, d)).astype(np.float32) for _ in range(3)]
+    bt = uir.Batch(res, [spec] * k, "f32")
+    assert bt.info()["bp_items"] == items
+    solo = uir.Batch(res, [spec], "f32")
+    want = []
+    for b in sinos:
+        solo.set_sinogram(0, b)
+        solo.reset()
+        solo.iterate(iters)
+        want.append(solo.image(0))
+    for i in range(k):
+        bt.set_sinogram(i, sinos[i % 3])
+    bt.reset()
+    bt.iterate(iters)
+    for i in range(k):
+        assert np.array_equal(bt.image(i), want[i % 3]), i
+
+
 def test_batch_pairs_slices_by_default_only_at_scale(res, monkeypatch):
     """With the default threshold (4 workgroups per CU), a BP table that
     would hold no more items than that takes tiles of 32 rows instead of 64,

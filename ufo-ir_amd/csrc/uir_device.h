@@ -301,18 +301,28 @@ double uirk_fp_item_cost(const uirk_fp_item *it);
  * items fill in at the end of a launch.  For tables of one slice (few
  * workgroups per CU); a table over many slices stays slice by slice. */
 void uirk_plan_sort_fp(uirk_fp_item *v, const uirk_xcd_part *part);
-/* BP slice pairs halve the workgroups of a launch and hold fewer waves per
- * SIMD, so they are used only while the paired table keeps at least this
- * many items: 4 workgroups per CU of the current device, or the value of the
- * environment variable UIR_PAIR_MIN_ITEMS when set (0: pair whenever two
- * slices of one geometry are adjacent). */
+/* The BP's shape for the slices of one model in one launch sequence.  A pixel's
+ * BP result does not depend on it (its window and sample coordinates are those
+ * of its 64 x 64 super-tile, its angles are summed in order). */
+typedef struct {
+    int pairs;    /* adjacent slices of one geometry share their items */
+    int rows32;   /* tiles of 32 rows */
+    int angles16; /* 16 angles a staged batch */
+} uirk_bp_choice;
+/* all: items of every slice of the launch at its tuned rows; n64: items of the
+ * model's slices in tiles of 64 rows, unpaired; p64, p32: paired, in tiles of
+ * 64 and 32 rows.  The environment variable UIR_PAIR_MIN_ITEMS, when set, is
+ * the least paired table instead (0: pair whenever two slices of one geometry
+ * are adjacent) and the largest one that takes 32 rows. */
+uirk_bp_choice uirk_plan_bp_choose(size_t all, size_t n64, size_t p64, size_t p32, int line);
+/* Adds the items of one n x n slice: *n64 if it is a slice, and *p64, *p32 if
+ * it leads a pair or has no partner. */
+void uirk_plan_bp_count(uint32_t n, int counts_paired, size_t *n64, size_t *p64, size_t *p32);
+/* A geometry's BP tile under the choice: a tuned tile keeps its angles. */
+uirk_tile uirk_plan_bp_tile(uirk_tile t, uirk_bp_choice c, int line);
+/* The least paired table the tuner probes with slice pairs (a full device, or
+ * UIR_PAIR_MIN_ITEMS). */
 int uirk_plan_pair_min_items(void);
-/* 1 if a BP table of this many items (at the tuned tile rows, before
- * pairing) holds no more than uirk_plan_pair_min_items(): too few workgroups
- * to fill the device, so its tiles take 32 rows instead of 64.  A pixel's BP
- * result does not depend on its tile's rows (its window and sample
- * coordinates are those of its 64 x 64 super-tile). */
-int uirk_plan_bp_rows32(size_t items);
 /* FP32 <-> storage conversions */
 int uirk_convert(const void *src, int src_dtype, void *dst, int dst_dtype, size_t n, void *stream);
 

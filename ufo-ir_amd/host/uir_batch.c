@@ -29,13 +29,6 @@ static int fp_shape(const uirk_tile *t)
 static const int k_fp_shape_angles[3] = {UIRK_FP_ANGLES, 8, 32};
 static int bp_shape(const uirk_tile *t) { return (t->bp_angles == 16) * 2 + (t->bp_rows == 32); }
 
-/* BP tile rows of a geometry in this batch: its tuned rows (the line model's
- * 64), or 32 when the batch's table would not fill the device with them */
-static int bp_rows_of(const geom_t *G, int rows32)
-{
-    return rows32 ? 32 : (G->model ? UIRK_BP_TILE : G->tile.bp_rows);
-}
-
 #define TRY(x) do { uir_status s_ = (x); if (s_ != UIR_OK) return s_; } while (0)
 
 static size_t align_up(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -363,34 +356,22 @@ uir_status uir_batch_new(uir_resources *res, uir_dtype storage, const uir_slice_
         s = uir_set_error(UIR_ERR_OUT_OF_MEMORY, "calloc");
         goto fail;
     }
-    /* BP tiles of 32 rows when the table at the tuned rows would not fill the
-     * device; a pixel's BP result does not depend on its tile's rows */
-    size_t bp_items = 0;
-    for (uint32_t i = 0; i < n_slices; ++i) {
-        const geom_t *G = &b->geoms[b->geom_of[i]];
-        const int rows = bp_rows_of(G, 0);
-        bp_items += (size_t)((G->n + UIRK_BP_TILE - 1) / UIRK_BP_TILE) * ((G->n + rows - 1) / rows);
-    }
-    const int rows32 = uirk_plan_bp_rows32(bp_items);
-    /* consecutive slices of one geometry pair up in the BP (modes 3 and 4),
-     * per model if its paired table still fills the device */
-    for (int32_t model = 0; model < 2; ++model) {
-        size_t paired_items = 0;
+    /* the BP's tile shapes, and whether consecutive slices of one geometry pair
+     * up in it (modes 3 and 4), per model */
+    uirk_bp_choice bpc[2];
+    {
+        size_t all = 0, n64[2] = {0, 0}, p64[2] = {0, 0}, p32[2] = {0, 0};
         for (uint32_t i = 0; i < n_slices; ++i) {
             const geom_t *G = &b->geoms[b->geom_of[i]];
-            const int rows = bp_rows_of(G, rows32);
-            const size_t tiles = (size_t)((G->n + UIRK_BP_TILE - 1) / UIRK_BP_TILE) * ((G->n + rows - 1) / rows);
-            if (G->model != model)
-                continue;
-            paired_items += tiles;
-            if (i + 1 < n_slices && b->geom_of[i + 1] == b->geom_of[i]) {
-                lead[i] = 1;
-                ++i;
-            }
+            const int rows = G->model ? UIRK_BP_TILE : G->tile.bp_rows, second = i > 0 && lead[i - 1];
+            all += (size_t)((G->n + UIRK_BP_TILE - 1) / UIRK_BP_TILE) * ((G->n + rows - 1) / rows);
+            lead[i] = !second && i + 1 < n_slices && b->geom_of[i + 1] == b->geom_of[i];
+            uirk_plan_bp_count(G->n, !second, &n64[G->model != 0], &p64[G->model != 0], &p32[G->model != 0]);
         }
-        if (paired_items < (size_t)uirk_plan_pair_min_items())
-            for (uint32_t i = 0; i < n_slices; ++i)
-                lead[i] = b->geoms[b->geom_of[i]].model == model ? 0 : lead[i];
+        for (int m = 0; m < 2; ++m)
+            bpc[m] = uirk_plan_bp_choose(all, n64[m], p64[m], p32[m], m);
+        for (uint32_t i = 0; i < n_slices; ++i)
+            lead[i] = lead[i] && bpc[b->geoms[b->geom_of[i]].model != 0].pairs;
     }
     for (uint32_t i = 0; i < n_slices; ++i) {
         const geom_t *G = &b->geoms[b->geom_of[i]];
@@ -426,7 +407,7 @@ uir_status uir_batch_new(uir_resources *res, uir_dtype storage, const uir_slice_
             const size_t b0 = bvl.n;
             if (uirk_plan_fp_line(&fvl, (int)i, (int)G->n, (int)G->D, G->axis, G->h_sin, G->h_cos, G->runs,
                                   G->n_runs, UIRK_FP_ANGLES, UIRK_FP_WMAX) ||
-                (!second && uirk_plan_bp(&bvl, (int)i, (int)G->n, bp_rows_of(G, rows32)))) {
+                (!second && uirk_plan_bp(&bvl, (int)i, (int)G->n, uirk_plan_bp_tile(G->tile, bpc[1], 1).bp_rows))) {
                 s = uir_set_error(UIR_ERR_OUT_OF_MEMORY, "work table");
                 goto fail;
             }
@@ -436,8 +417,7 @@ uir_status uir_batch_new(uir_resources *res, uir_dtype storage, const uir_slice_
             /* BP slice pairs: slice i + 1 of the same geometry joins slice i's
              * BP items (pair set) */
             const int second = i > 0 && lead[i - 1];
-            uirk_tile bt = G->tile;
-            bt.bp_rows = bp_rows_of(G, rows32);
+            const uirk_tile bt = uirk_plan_bp_tile(G->tile, bpc[0], 0);
             uirk_bp_vec *bvg = &bv[bp_shape(&bt)];
             const size_t b0 = bvg->n;
             if (uirk_plan_fp(&fv[fp_shape(&G->tile)], (int)i, (int)G->n, (int)G->D, G->axis, G->h_sin, G->h_cos,
@@ -515,7 +495,7 @@ uir_status uir_batch_new(uir_resources *res, uir_dtype storage, const uir_slice_
         if (s == UIR_OK) {
             kgroup *k = &b->bpl;
             k->tile = (uirk_tile)UIRK_TILE_DEFAULT;
-            k->tile.bp_rows = rows32 ? 32 : UIRK_BP_TILE;
+            k->tile.bp_rows = bpc[1].rows32 ? 32 : UIRK_BP_TILE;
             k->mode = 2;
             for (size_t i = 0; i < bvl.n; ++i) {
                 cost[i] = (double)specs[bvl.v[i].slice].n_angles;

@@ -262,9 +262,62 @@ int uirk_plan_pair_min_items(void)
     return uirk_plan_device_slots();
 }
 
-int uirk_plan_bp_rows32(size_t items)
+void uirk_plan_bp_count(uint32_t n, int counts_paired, size_t *n64, size_t *p64, size_t *p32)
 {
-    return items <= (size_t)uirk_plan_pair_min_items();
+    const size_t w = (n + UIRK_BP_TILE - 1) / UIRK_BP_TILE, h32 = (n + 31) / 32;
+    *n64 += w * w;
+    if (counts_paired) {
+        *p64 += w * w;
+        *p32 += w * h32;
+    }
+}
+
+/* A pair's item takes 1.4 times the time of one slice's, so pairs gain even
+ * where they leave CUs idle: from more than 2 items a CU in tiles of 32 rows
+ * (line model: from 1).  A CU holds 3 pair items with 32 staged angles and 4
+ * with 16 (line model: 4).  The tiles are of 32 rows while the table is
+ * resident at once that way, else of 64; 32 angles are staged while the table
+ * is resident at once with them (fewer barriers), else 16.  Measured at 400
+ * angles (us; before: pairs from 4 items a CU, in the rows of the unpaired
+ * table): 12 x 512 173 with pairs of 32 rows, 32 angles, 211 before; 16 x 512
+ * 217 with 32 rows, 16 angles, 223 with 64 / 32, 271 before; 6 x 1024 279 with
+ * 64 / 32, 319 with 32 / 16, 349 before; 8 x 1024 345 with 64 / 16, 407 with
+ * 64 / 32 (4 items a CU, 3 at once), 403 before.  At 2 items a CU and below
+ * there is less to gain: 6 x 512 134 against 139 unpaired, 4 x 512
+ * 121 against 120, 2 x 1024 139 against 157.  Line model: 9 x 512 247 with
+ * pairs of 32 rows, 299 unpaired, 315 with 64; 16 x 512 320 against 351 with
+ * 64; 4 x 512 146 against 161 unpaired.  Where too few slices have a partner
+ * to outweigh the rest, which then run the pair kernel at a pair's cost, none
+ * pairs. */
+uirk_bp_choice uirk_plan_bp_choose(size_t all, size_t n64, size_t p64, size_t p32, int line)
+{
+    const size_t cu = (size_t)uirk_plan_device_slots() / 4;
+    uirk_bp_choice c = {0, all <= 4 * cu, 0};
+    const char *env = getenv("UIR_PAIR_MIN_ITEMS");
+    if (env && *env) {
+        const size_t least = (size_t)atoi(env);
+        c.rows32 = all <= least;
+        c.pairs = (c.rows32 ? p32 : p64) >= least;
+        return c;
+    }
+    if (p32 >= (line ? cu : 2 * cu + 1) && 7 * p64 <= 5 * n64) {
+        c.pairs = 1;
+        c.rows32 = p32 <= 4 * cu;
+        c.angles16 = !line && (c.rows32 ? p32 : p64) > 3 * cu;
+    }
+    return c;
+}
+
+uirk_tile uirk_plan_bp_tile(uirk_tile t, uirk_bp_choice c, int line)
+{
+    const uirk_tile def = UIRK_TILE_DEFAULT;
+    if (line)
+        t = def;
+    if (c.angles16 && t.bp_angles == def.bp_angles && t.bp_rows == def.bp_rows)
+        t.bp_angles = 16;
+    if (c.rows32)
+        t.bp_rows = 32;
+    return t;
 }
 
 double uirk_fp_item_cost(const uirk_fp_item *it)

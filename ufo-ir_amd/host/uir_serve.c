@@ -74,7 +74,7 @@ typedef struct sgeom {
     int refs;
     double last_used;
     uirk_tile tile;        /* tuned or default tile shape */
-    int fp_shape, bp_shape; /* group indices of that shape */
+    int fp_shape; /* FP group index of that shape */
     int32_t model;          /* 0 joseph, 1 line */
     /* line model: per-angle constants of the table kernels (8 floats) and of
      * the single-angle kernels, and the pixel weights 1 / BP(1) (n x n),
@@ -331,11 +331,9 @@ static uir_status geom_create(uir_server *s, const uir_slice_spec *sp, sgeom **o
     if (g->model) { /* the line model's groups take the default tile */
         g->tile = (uirk_tile)UIRK_TILE_DEFAULT;
         g->fp_shape = SRV_FP_LINE;
-        g->bp_shape = SRV_BP_LINE;
     } else {
         g->tile = uir_tile_for(sp, s->dtype);
         g->fp_shape = (g->tile.fp_angles == 8 ? 1 : (g->tile.fp_angles == 32 ? 2 : 0)) + 3 * (g->tile.fp_single != 0);
-        g->bp_shape = (g->tile.bp_angles == 16) * 2 + (g->tile.bp_rows == 32);
     }
     {
         uirk_fp_vec fv = {0};
@@ -596,33 +594,48 @@ static uir_status dgrow(void **p, size_t *cap, size_t need, size_t es)
  * Descriptors are laid out geometry by geometry (slot j holds request
  * ord[j]), so that consecutive requests of one geometry share BP items as
  * slice pairs (modes 3 and 4). */
-/* A geometry's BP template items and group in a step: its tuned tile, or
- * tiles of 32 rows when the step's table would not fill the device (rows32) */
-static const uirk_bp_item *geom_bp(const sgeom *g, int rows32, size_t *n)
+/* A geometry's BP template items and group in a step (uirk_plan_bp_choose) */
+static const uirk_bp_item *geom_bp(const sgeom *g, const uirk_bp_choice *bpc, size_t *n)
 {
-    const int r32 = rows32 && g->bp32;
+    const int r32 = bpc[g->model != 0].rows32 && g->bp32;
     *n = r32 ? g->n_bp32 : g->n_bp;
     return r32 ? g->bp32 : g->bp;
 }
-static int geom_bp_shape(const sgeom *g, int rows32)
+static int geom_bp_shape(const sgeom *g, const uirk_bp_choice *bpc)
 {
-    return g->bp_shape == SRV_BP_LINE ? SRV_BP_LINE : (rows32 ? g->bp_shape | 1 : g->bp_shape);
+    if (g->model)
+        return SRV_BP_LINE;
+    const uirk_tile t = uirk_plan_bp_tile(g->tile, bpc[0], 0);
+    return (t.bp_angles == 16) * 2 + (t.bp_rows == 32);
 }
 
 static uir_status tables_build(uir_server *s)
 {
     const uint32_t na = s->n_active;
     size_t nf[SRV_FP_SHAPES] = {0}, nb[SRV_BP_SHAPES] = {0}, ncost = 1, bp_items = 0;
-    for (uint32_t i = 0; i < na; ++i)
-        bp_items += s->active[i]->g->n_bp;
-    const int rows32 = uirk_plan_bp_rows32(bp_items);
-    s->bpg[SRV_BP_LINE].tile.bp_rows = rows32 ? 32 : UIRK_BP_TILE;
+    /* the BP's shapes and pairs per model, from the slices and the pairs that
+     * the active requests make when ordered by geometry */
+    uirk_bp_choice bpc[2];
+    {
+        size_t n64[2] = {0, 0}, p64[2] = {0, 0}, p32[2] = {0, 0};
+        for (uint32_t i = 0; i < na; ++i) {
+            const sgeom *g = s->active[i]->g;
+            int second = 0;
+            for (uint32_t j = 0; j < i; ++j)
+                second ^= s->active[j]->g == g;
+            bp_items += g->n_bp;
+            uirk_plan_bp_count(g->n, !second, &n64[g->model != 0], &p64[g->model != 0], &p32[g->model != 0]);
+        }
+        for (int m = 0; m < 2; ++m)
+            bpc[m] = uirk_plan_bp_choose(bp_items, n64[m], p64[m], p32[m], m);
+    }
+    s->bpg[SRV_BP_LINE].tile.bp_rows = bpc[1].rows32 ? 32 : UIRK_BP_TILE;
     for (uint32_t i = 0; i < na; ++i) {
         const sgeom *g = s->active[i]->g;
         size_t n;
-        (void)geom_bp(g, rows32, &n);
+        (void)geom_bp(g, bpc, &n);
         nf[g->fp_shape] += g->n_fp;
-        nb[geom_bp_shape(g, rows32)] += n;
+        nb[geom_bp_shape(g, bpc)] += n;
     }
     for (int c = 0; c < SRV_FP_SHAPES; ++c)
         ncost = nf[c] > ncost ? nf[c] : ncost;
@@ -657,18 +670,6 @@ static uir_status tables_build(uir_server *s)
         s->fpg[c].n = 0;
     for (int c = 0; c < SRV_BP_SHAPES; ++c)
         s->bpg[c].n = 0;
-    /* BP pairs only while the paired table of the model fills the device */
-    size_t paired[2] = {0, 0};
-    for (uint32_t i = 0; i < na; ++i) {
-        const sgeom *g = s->active[s->ord[i]]->g;
-        size_t n;
-        (void)geom_bp(g, rows32, &n);
-        paired[g->model != 0] += n;
-        if (i + 1 < na && s->active[s->ord[i + 1]]->g == g)
-            ++i;
-    }
-    const int pair_ok[2] = {paired[0] >= (size_t)uirk_plan_pair_min_items(),
-                            paired[1] >= (size_t)uirk_plan_pair_min_items()};
     int lead = 0; /* slot i - 1 led a BP pair */
     for (uint32_t i = 0; i < na; ++i) {
         const sreq *q = s->active[s->ord[i]];
@@ -713,21 +714,21 @@ static uir_status tables_build(uir_server *s)
         } else {
             k->pix_scale = 1.0f / (float)g->A;
         }
-        sgroup *fg = &s->fpg[g->fp_shape], *bg = &s->bpg[geom_bp_shape(g, rows32)];
+        sgroup *fg = &s->fpg[g->fp_shape], *bg = &s->bpg[geom_bp_shape(g, bpc)];
         uirk_fp_item *fi = (uirk_fp_item *)fg->h_items;
         uirk_bp_item *bi = (uirk_bp_item *)bg->h_items;
         size_t n_bp;
-        const uirk_bp_item *gbp = geom_bp(g, rows32, &n_bp);
+        const uirk_bp_item *gbp = geom_bp(g, bpc, &n_bp);
         for (size_t j = 0; j < g->n_fp; ++j) {
             fi[fg->n] = g->fp[j];
             fi[fg->n].slice = (int32_t)i;
             ++fg->n;
         }
         /* a slot followed by one of its geometry leads a BP pair (when the
-         * model's paired table fills the device); the second slot of a pair
-         * has no BP items of its own */
+         * model's slices pair); the second slot of a pair has no BP items of
+         * its own */
         const int second = lead;
-        lead = pair_ok[g->model != 0] && !second && i + 1 < na && s->active[s->ord[i + 1]]->g == g;
+        lead = bpc[g->model != 0].pairs && !second && i + 1 < na && s->active[s->ord[i + 1]]->g == g;
         for (size_t j = 0; j < n_bp && !second; ++j) {
             bi[bg->n] = gbp[j];
             bi[bg->n].slice = (int32_t)i;
