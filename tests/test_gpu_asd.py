@@ -103,6 +103,28 @@ def test_batch_asdpocs_line_model_matches_fp64(res, compat, storage, tol):
         assert np.allclose(bt.asdpocs_diagnostics(i), diag, rtol=max(20 * tol, 2e-3), atol=1e-6)
 
 
+# Sizes at the edges of the TV step's tiles (60 columns, 32 rows) and of the
+# SART step's (64 x 64), several tiles each way, and one slice past 512.
+EDGES = [(5, 8, 9), (31, 45, 9), (32, 46, 9), (33, 47, 9), (59, 84, 9), (60, 85, 9), (61, 87, 9), (63, 90, 9),
+         (64, 91, 9), (65, 92, 9), (66, 94, 9), (120, 170, 9), (121, 172, 9), (129, 183, 9), (513, 726, 7)]
+
+
+@pytest.mark.parametrize("compat", [True, False])
+@pytest.mark.parametrize("ng", [0, 1, 3, 4])  # the steps alternate between two buffers
+def test_batch_asdpocs_tile_edges(res, ng, compat):
+    """One batch of every size against the FP64 oracle, with the bound that
+    four iterations of ten TV steps keep above."""
+    print("case asdpocs tile edges", ng, compat, flush=True)
+    bt, data = _batch(res, "f32", EDGES, seed0=700)
+    bt.asdpocs(2, ng=ng, compat=compat, **KW)
+    for i, (g, b) in enumerate(data):
+        ref = O.asdpocs64(g, b.astype(np.float64), 2, ng=ng, df_iters=1, textbook=not compat, ray_weight_min=RMIN,
+                          df_relax_initial=0.25, **KW)
+        err = O.rel_l2(bt.image(i), ref)
+        print(EDGES[i], "rel-L2 vs FP64 %.3e" % err, flush=True)
+        assert err <= 1e-4
+
+
 def test_batch_asdpocs_slice_independent_of_mix(res):
     """A slice's image is the same alone and in a batch of other geometries."""
     bt, _ = _batch(res, "f32")
