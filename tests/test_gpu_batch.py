@@ -97,8 +97,8 @@ def test_batch_slice_pairs_equal_single_slices(res, storage, monkeypatch):
 
 @pytest.mark.parametrize("model,k,items", [
     # items of 250 x 250 slices: 16 tiles of 64 rows, 32 of 32; per CU of 256
-    ("joseph", 32, 1024),  # 2 paired items a CU: unpaired, 32 rows
-    ("joseph", 33, 544),   # more: pairs, 32 rows, 32 angles
+    ("joseph", 34, 1088),  # 4.25 items a CU: unpaired, 64 rows would be 544
+    ("joseph", 35, 576),   # more: pairs, 32 rows, 32 angles
     ("joseph", 49, 800),   # more than 3 a CU: 16 angles; a last slice without a partner
     ("joseph", 66, 528),   # more than 4: 64 rows, 32 angles
     ("joseph", 98, 784),   # more than 3 in 64 rows: 16 angles

@@ -309,15 +309,15 @@ typedef struct {
     int rows32;   /* tiles of 32 rows */
     int angles16; /* 16 angles a staged batch */
 } uirk_bp_choice;
-/* all: items of every slice of the launch at its tuned rows; n64: items of the
- * model's slices in tiles of 64 rows, unpaired; p64, p32: paired, in tiles of
+/* all: items of every slice of the launch at its tuned rows; n32: items of the
+ * model's slices in tiles of 32 rows, unpaired; p64, p32: paired, in tiles of
  * 64 and 32 rows.  The environment variable UIR_PAIR_MIN_ITEMS, when set, is
  * the least paired table instead (0: pair whenever two slices of one geometry
  * are adjacent) and the largest one that takes 32 rows. */
-uirk_bp_choice uirk_plan_bp_choose(size_t all, size_t n64, size_t p64, size_t p32, int line);
-/* Adds the items of one n x n slice: *n64 if it is a slice, and *p64, *p32 if
- * it leads a pair or has no partner. */
-void uirk_plan_bp_count(uint32_t n, int counts_paired, size_t *n64, size_t *p64, size_t *p32);
+uirk_bp_choice uirk_plan_bp_choose(size_t all, size_t n32, size_t p64, size_t p32, int line);
+/* Adds the items of one n x n slice to *n32, and to *p64, *p32 if it leads a
+ * pair or has no partner (counts_paired). */
+void uirk_plan_bp_count(uint32_t n, int counts_paired, size_t *n32, size_t *p64, size_t *p32);
 /* A geometry's BP tile under the choice: a tuned tile keeps its angles. */
 uirk_tile uirk_plan_bp_tile(uirk_tile t, uirk_bp_choice c, int line);
 /* The least paired table the tuner probes with slice pairs (a full device, or

@@ -124,25 +124,36 @@ __device__ __forceinline__ float neg_float_of(int n)
     return n == 0 ? -0.0f : __uint_as_float(bits);
 }
 
-// Entry rne_index(x) of an LDS table.  Shifts and shift-adds issue at half the
-// rate of float multiply-adds, so the address is one: m = x + 1.5 2^23 is the
-// integer 1.5 2^23 + i, and m 2^-149 size + (base - 1.5 2^23 size) 2^-149 is
-// exactly the denormal whose bits are base + i size, an LDS address (one
-// rounding, of a value that is representable: sizes are 8 or 16 and bases
-// their multiples).  lds_rne_base makes the second term, once per table.
+// Entry rne_index(x) of an LDS table through a base biased by the bits of
+// 1.5 2^23 (lds_rne_base, once per table): the sample's address is then one
+// shift-add of x + 1.5 2^23's bits.  Unsigned 32-bit arithmetic wraps, so
+// the biased base may lie outside LDS; the sum is the entry's address.
 template <typename E> using lds_ptr = const __attribute__((address_space(3))) E *;
-template <typename E> __device__ __forceinline__ float lds_rne_base(const E *table)
+__device__ __forceinline__ uint32_t lds_rne_base(const float2 *table)
 {
-    static_assert(sizeof(E) == 8 || sizeof(E) == 16, "entry size");
-    // -(1.5 2^23 size - base) 2^-149: the mantissa counts down by one per
-    // 8 (16) bytes of base from 1.5 2^26 (2^27) 2^-149
-    constexpr uint32_t kBits = 0x80000000u | ((sizeof(E) == 8 ? 4u : 5u) << 23) | 0x400000u;
-    return __uint_as_float(kBits - (uint32_t)(uintptr_t)(lds_ptr<E>)table / (uint32_t)sizeof(E));
+    return (uint32_t)(uintptr_t)(lds_ptr<float2>)table - 0x4B400000u * 8u;
 }
-template <typename E> __device__ __forceinline__ E lds_rne_read(float base, float x)
+__device__ __forceinline__ float2 lds_rne_read(uint32_t base, float x)
 {
-    const float a = __builtin_fmaf(x + 12582912.0f, __uint_as_float((uint32_t)sizeof(E)), base);
-    return *(const E *)(lds_ptr<E>)(uintptr_t)__float_as_uint(a);
+    const uint32_t a = (uint32_t)__float_as_int(x + 12582912.0f) * 8u + base;
+    return *(const float2 *)(lds_ptr<float2>)(uintptr_t)a;
+}
+// The same for the pairs' 16-byte entries, whose samples are bound by the VALU
+// as much as by LDS.  Shifts and shift-adds issue at half the rate of float
+// multiply-adds, so the address is one of those: m = x + 1.5 2^23 is the integer
+// 1.5 2^23 + i, and m 2^-149 16 + (base - 1.5 2^23 16) 2^-149 is exactly the
+// denormal whose bits are base + 16 i, an LDS address (one rounding, of a value
+// that is representable).  The second term's mantissa counts down by one per
+// 16 bytes of base from 1.5 2^27 2^-149.  Single slices, bound by LDS reads or
+// by latency, keep the shift-add (8 x 206, f16: 95 us against 101).
+__device__ __forceinline__ float lds_rne_base(const float4 *table)
+{
+    return __uint_as_float(0x82C00000u - (uint32_t)(uintptr_t)(lds_ptr<float4>)table / 16u);
+}
+__device__ __forceinline__ float4 lds_rne_read(float base, float x)
+{
+    const float a = __builtin_fmaf(x + 12582912.0f, __uint_as_float(16u), base);
+    return *(const float4 *)(lds_ptr<float4>)(uintptr_t)__float_as_uint(a);
 }
 
 // Column of a lane for the 16-byte reads of a slice pair.  A ds_read_b128
@@ -1265,7 +1276,7 @@ __global__ __launch_bounds__(256, LINE ? 4 : (PAIR ? (NA == 32 ? 3 : 4) : 6)) vo
                     // the thread's column term A and the row's offset ys_q in the
                     // super-tile, whatever the tile's rows.  Joseph: less 1/2, so a
                     // sample's entry is rne_index of it, one float add,
-                    // and its address one more FMA.
+                    // and its address one more operation.
                     const float A = __builtin_fmaf((float)col, ct, s_base[k]);
                     if constexpr (LINE) {
                         const float4 L = s_line[k]; // (bp_k, bp_b0, bp_b1, 1/M)
@@ -1316,7 +1327,7 @@ __global__ __launch_bounds__(256, LINE ? 4 : (PAIR ? (NA == 32 ? 3 : 4) : 6)) vo
                             }
                         }
                     } else if (!clamp_u) {
-                        const float P = lds_rne_base(ldp + k * kBpWb);
+                        const auto P = lds_rne_base(ldp + k * kBpWb);
                         // a copy of A per branch: the compiler would otherwise hoist
                         // every row's coordinate above the branch, all live at once
                         float Ab = A;
@@ -1328,7 +1339,7 @@ __global__ __launch_bounds__(256, LINE ? 4 : (PAIR ? (NA == 32 ? 3 : 4) : 6)) vo
 #pragma unroll
                             for (int h = 0; h < 8; ++h) {
                                 w[h] = __builtin_fmaf(nys[g + h], st, Ab);
-                                p[h] = lds_rne_read<E>(P, w[h]);
+                                p[h] = lds_rne_read(P, w[h]);
                             }
 #pragma unroll
                             for (int h = 0; h < 8; ++h) {
@@ -1341,7 +1352,7 @@ __global__ __launch_bounds__(256, LINE ? 4 : (PAIR ? (NA == 32 ? 3 : 4) : 6)) vo
                         // u clamped to [edge0, edge1] (:203-210), in window coordinates less 1/2
                         const float wlo = (edge0 - 1.0f) - (float)s_umin[k];
                         const float whi = (edge1 - 1.0f) - (float)s_umin[k];
-                        const float P = lds_rne_base(ldp + k * kBpWb);
+                        const auto P = lds_rne_base(ldp + k * kBpWb);
                         float Ab = A;
                         asm volatile("" : "+v"(Ab));
 #pragma unroll
@@ -1351,7 +1362,7 @@ __global__ __launch_bounds__(256, LINE ? 4 : (PAIR ? (NA == 32 ? 3 : 4) : 6)) vo
 #pragma unroll
                             for (int h = 0; h < 8; ++h) {
                                 w[h] = __builtin_amdgcn_fmed3f(__builtin_fmaf(nys[g + h], st, Ab), wlo, whi);
-                                p[h] = lds_rne_read<E>(P, w[h]);
+                                p[h] = lds_rne_read(P, w[h]);
                             }
 #pragma unroll
                             for (int h = 0; h < 8; ++h) {

@@ -262,10 +262,10 @@ int uirk_plan_pair_min_items(void)
     return uirk_plan_device_slots();
 }
 
-void uirk_plan_bp_count(uint32_t n, int counts_paired, size_t *n64, size_t *p64, size_t *p32)
+void uirk_plan_bp_count(uint32_t n, int counts_paired, size_t *n32, size_t *p64, size_t *p32)
 {
     const size_t w = (n + UIRK_BP_TILE - 1) / UIRK_BP_TILE, h32 = (n + 31) / 32;
-    *n64 += w * w;
+    *n32 += w * h32;
     if (counts_paired) {
         *p64 += w * w;
         *p32 += w * h32;
@@ -273,8 +273,9 @@ void uirk_plan_bp_count(uint32_t n, int counts_paired, size_t *n64, size_t *p64,
 }
 
 /* A pair's item takes 1.4 times the time of one slice's, so pairs gain even
- * where they leave CUs idle: from more than 2 items a CU in tiles of 32 rows
- * (line model: from 1).  A CU holds 3 pair items with 32 staged angles and 4
+ * where they leave CUs idle: from more than 4.25 unpaired items a CU in tiles
+ * of 32 rows, of which a CU holds 6, on (line model, of which it holds 4: from 2).
+ * A CU holds 3 pair items with 32 staged angles and 4
  * with 16 (line model: 4).  The tiles are of 32 rows while the table is
  * resident at once that way, else of 64; 32 angles are staged while the table
  * is resident at once with them (fewer barriers), else 16.  Measured at 400
@@ -282,14 +283,15 @@ void uirk_plan_bp_count(uint32_t n, int counts_paired, size_t *n64, size_t *p64,
  * table): 12 x 512 173 with pairs of 32 rows, 32 angles, 211 before; 16 x 512
  * 217 with 32 rows, 16 angles, 223 with 64 / 32, 271 before; 6 x 1024 279 with
  * 64 / 32, 319 with 32 / 16, 349 before; 8 x 1024 345 with 64 / 16, 407 with
- * 64 / 32 (4 items a CU, 3 at once), 403 before.  At 2 items a CU and below
- * there is less to gain: 6 x 512 134 against 139 unpaired, 4 x 512
+ * 64 / 32 (4 items a CU, 3 at once), 403 before.  With 4 unpaired items a CU
+ * and fewer there is less to gain: 6 x 512 134 against 139 unpaired, 4 x 512
  * 121 against 120, 2 x 1024 139 against 157.  Line model: 9 x 512 247 with
  * pairs of 32 rows, 299 unpaired, 315 with 64; 16 x 512 320 against 351 with
- * 64; 4 x 512 146 against 161 unpaired.  Where too few slices have a partner
- * to outweigh the rest, which then run the pair kernel at a pair's cost, none
- * pairs. */
-uirk_bp_choice uirk_plan_bp_choose(size_t all, size_t n64, size_t p64, size_t p32, int line)
+ * 64; 4 x 512 146 against 161 unpaired.  A slice without a partner runs the
+ * pair kernel at a pair's cost: with less than 1.65 slices an item none pairs
+ * (3 x 1024: 211 unpaired, 216 as pairs; 5 x 1024: 297 and 275), line model
+ * 1.8 (5 x 417 / 320: 117 unpaired, 133 as pairs). */
+uirk_bp_choice uirk_plan_bp_choose(size_t all, size_t n32, size_t p64, size_t p32, int line)
 {
     const size_t cu = (size_t)uirk_plan_device_slots() / 4;
     uirk_bp_choice c = {0, all <= 4 * cu, 0};
@@ -300,7 +302,7 @@ uirk_bp_choice uirk_plan_bp_choose(size_t all, size_t n64, size_t p64, size_t p3
         c.pairs = (c.rows32 ? p32 : p64) >= least;
         return c;
     }
-    if (p32 >= (line ? cu : 2 * cu + 1) && 7 * p64 <= 5 * n64) {
+    if (line ? n32 >= 2 * cu && 5 * n32 >= 9 * p32 : 4 * n32 > 17 * cu && 20 * n32 >= 33 * p32) {
         c.pairs = 1;
         c.rows32 = p32 <= 4 * cu;
         c.angles16 = !line && (c.rows32 ? p32 : p64) > 3 * cu;

@@ -617,17 +617,17 @@ static uir_status tables_build(uir_server *s)
      * the active requests make when ordered by geometry */
     uirk_bp_choice bpc[2];
     {
-        size_t n64[2] = {0, 0}, p64[2] = {0, 0}, p32[2] = {0, 0};
+        size_t n32[2] = {0, 0}, p64[2] = {0, 0}, p32[2] = {0, 0};
         for (uint32_t i = 0; i < na; ++i) {
             const sgeom *g = s->active[i]->g;
             int second = 0;
             for (uint32_t j = 0; j < i; ++j)
                 second ^= s->active[j]->g == g;
             bp_items += g->n_bp;
-            uirk_plan_bp_count(g->n, !second, &n64[g->model != 0], &p64[g->model != 0], &p32[g->model != 0]);
+            uirk_plan_bp_count(g->n, !second, &n32[g->model != 0], &p64[g->model != 0], &p32[g->model != 0]);
         }
         for (int m = 0; m < 2; ++m)
-            bpc[m] = uirk_plan_bp_choose(bp_items, n64[m], p64[m], p32[m], m);
+            bpc[m] = uirk_plan_bp_choose(bp_items, n32[m], p64[m], p32[m], m);
     }
     s->bpg[SRV_BP_LINE].tile.bp_rows = bpc[1].rows32 ? 32 : UIRK_BP_TILE;
     for (uint32_t i = 0; i < na; ++i) {
