@@ -99,6 +99,45 @@ def test_sart_steps_bit_exact(res, n, d, a, step, axis):
         assert np.array_equal(got, O.sart(g, b, iters, 0.5), equal_nan=True), iters
 
 
+@pytest.mark.parametrize("model", ["joseph", "line"])
+@pytest.mark.parametrize("method", ["sart", "asdpocs"])
+def test_sart_sweep_of_a_replaced_projector(res, method, model):
+    """A method whose projector is replaced, and the old one given back before
+    the new one builds its tables (which may then lie at the old addresses),
+    takes the new angles: bit for bit a fresh task's result."""
+    n, d, a = 96, 136, 60
+    b = np.random.default_rng(3).random((a, d)).astype(np.float32)
+
+    def projector(step):
+        return uir.Task("parallel-projector", step=float(np.float32(step)), is_forward=False, image_size=n, model=model)
+
+    def task(p):
+        if method == "sart":
+            return uir.Task("sart", projector=p, num_iterations=3, relaxation_factor=0.5).setup(res)
+        return uir.Task("asdpocs", projector=p, num_iterations=2,
+                        df_minimizer=uir.Task("sart", num_iterations=3)).setup(res)
+
+    print("case replaced projector", method, model, flush=True)
+    steps = [np.pi / a, np.pi / a / 2, 2 * np.pi / a, 0.01, 0.08]
+    want = []
+    for step in steps:
+        got, _ = _run(task(projector(step)), b, n)
+        want.append(got)
+    old = projector(steps[0])
+    m = task(old)
+    ds, out = uir.DeviceArray.from_numpy(b), uir.DeviceArray((n, n))
+    for k, step in enumerate(steps):
+        if k:
+            new = projector(step)
+            m["projector"] = new
+            m.setup(res)
+            old.close()
+            old = new
+        assert m.requisition(ds) == (n, n)
+        m.process(ds, out)
+        assert np.array_equal(out.numpy(), want[k]), k
+
+
 @pytest.mark.parametrize("df", ["sart", "sirt"])
 def test_asdpocs(res, df):
     n = d = 96

@@ -27,7 +27,8 @@ typedef enum { P_FLOAT = UIR_PROP_FLOAT, P_UINT = UIR_PROP_UINT, P_BOOL = UIR_PR
 
 typedef struct {
     const void *x, *b, *t0, *t1, *part, *sino_tmp, *ray_w, *starts, *sin, *cos, *line;
-    uint32_t n, D, A, lut_gen;
+    uint32_t n, D, A;
+    uint64_t lut_gen; /* the launches hold values of the LUT and of the line table */
     float axis, relax, corr;
 } sart_graph_key;
 
@@ -50,7 +51,8 @@ struct uir_task {
     uir_subset *runs;
     uint32_t n_runs;
     /* FP work table of the table-driven kernel for the current geometry */
-    uint32_t plan_gen, plan_n, plan_dets, plan_angles;
+    uint64_t plan_gen;
+    uint32_t plan_n, plan_dets, plan_angles;
     float plan_axis;
     uirk_fp_item *d_fp_items;
     int n_fp_items, fp_angles; /* fp_angles: largest item */
@@ -60,7 +62,8 @@ struct uir_task {
     /* the line model (model "line"): per-angle constants of the current
      * geometry (host copy and device table) and the angles' family runs */
     int line;
-    uint32_t lut_gen, line_gen, line_n, line_angles;
+    uint64_t lut_gen, line_gen; /* lut_gen: number of the LUT build, unique over all projectors */
+    uint32_t line_n, line_angles;
     float line_axis;
     uirk_line_angle *h_line, *d_line;
     uir_subset *line_runs;
@@ -510,6 +513,11 @@ uir_status uir_task_setup(uir_task *t, uir_resources *res)
 /* projector geometry (get_requisition, ufo-ir-parallel-projector-task.c:305-347) */
 /* ------------------------------------------------------------------------ */
 
+/* LUT builds of the process.  A captured sweep is kept by the number of the
+ * build, and a method's projector may be replaced by one whose tables lie at
+ * the addresses that the old one gave back. */
+static uint64_t g_lut_builds;
+
 static uir_status proj_build_luts(uir_task *p, uint32_t n_angles)
 {
     p->lut_n = 0; /* a build that fails is taken again by the next call */
@@ -536,7 +544,7 @@ static uir_status proj_build_luts(uir_task *p, uint32_t n_angles)
     }
     p->lut_n = n_angles;
     p->lut_step = p->step;
-    p->lut_gen++;
+    p->lut_gen = __atomic_add_fetch(&g_lut_builds, 1, __ATOMIC_RELAXED);
     return UIR_OK;
 }
 
