@@ -38,6 +38,27 @@ def test_fp_bp_joseph_per_subset(res, n, a):
     assert np.array_equal(vol.numpy(), O.bp(g, ref, vol=x, relax=0.5))
 
 
+@pytest.mark.parametrize("n", [200, 513])  # one and two pixels a thread
+@pytest.mark.parametrize("scale", [0.5, 1.0, 1.75, float("nan")])
+def test_bp_joseph_takes_any_lut(res, n, scale):
+    """The caller's LUT need not hold sines and cosines: pairs scaled by a pixel
+    size, and a NaN, give the oracle's image bit for bit."""
+    print("case bp any lut", n, scale, flush=True)
+    d, a = int(np.ceil(n * 2 ** 0.5)) + 2, 9
+    g = O.Geometry(n, d, a, np.float32(np.pi / a))
+    g.sin[2:] *= np.float32(scale)
+    g.cos[2:] *= np.float32(scale)
+    rng = np.random.default_rng(n)
+    sino, x = rng.random((a, d)).astype(np.float32), rng.random((n, n)).astype(np.float32)
+    vol, ds, dsin, dcos = _dev(x), _dev(sino), _dev(g.sin[None, :]), _dev(g.cos[None, :])
+    dims = uir.GeometryDims(n, n, d, a)
+    for (o, k, dr) in ((0, 3, 0), (3, a - 3, 1)):
+        uir.check(uir.load().uir_bp_joseph(vol.ptr, vol.ptr, ds.ptr, 0.5, dsin.ptr, dcos.ptr, dims, g.axis,
+                                           uir.Subset(o, k, dr), None))
+    want = O.bp(g, sino, vol=x, relax=0.5, subsets=[(0, 3, 0), (3, a - 3, 1)])
+    assert np.array_equal(vol.numpy(), want, equal_nan=True)
+
+
 @pytest.mark.parametrize("n,d,a,axis", [(256, 256, 60, -1.0), (200, 283, 45, -1.0), (128, 128, 30, 70.0),
                                         (1100, 1556, 6, -1.0)])
 def test_fp_joseph_single_angle_split_is_bit_identical(res, n, d, a, axis):

@@ -88,10 +88,11 @@ int uirk_sart_ref_step(const float *x_in, float *x_out, const float *b, const fl
  * subsets (runs), one per-run accumulation each: w = r + relax * sum_run.
  * pix_w == NULL: accumulate mode (r_vol may equal w_vol).
  * pix_w != NULL: SIRT mode, tmp = sum_runs(relax * S_run) (from 0), then
- * w = tmp * pix_w + r (ufo-ir-sirt-task.c:208-212); posc clamps the result. */
+ * w = tmp * pix_w + r (ufo-ir-sirt-task.c:208-212); posc clamps the result.
+ * unit_lut: the LUT holds the sines and cosines of angles (0: any values). */
 int uirk_bp_ref(const float *r_vol, float *w_vol, const float *sino, int n_angles,
                 const float *sin_lut, const float *cos_lut, int n, int n_dets, float axis,
-                float relax, const uirk_runs *runs, const float *pix_w, int posc, void *stream);
+                float relax, const uirk_runs *runs, int unit_lut, const float *pix_w, int posc, void *stream);
 
 /* ---- The line projection model (uir_line.hip) ----
  * Ray s of angle a is the line X c - Y s_ = t, t = s + 1/2 - axis, with (c, s_)

@@ -353,9 +353,9 @@ __device__ __forceinline__ int cvt_flr(float x)
     return r;
 }
 
-// CLAMP 2: any axis.  1: 0.5 <= edge0 <= edge1 <= n_dets - 0.5 (an axis with
-// active detectors), so that the clamp is one median and every lower tap lies
-// in the row.  0: no pixel reaches an edge either, no clamp.
+// CLAMP 2: any axis and any LUT.  1: 0.5 <= edge0 <= edge1 <= n_dets - 0.5 (an
+// axis with active detectors), so that the clamp is one median and every lower
+// tap lies in the row.  0: no pixel reaches an edge either, no clamp.
 template <int R, int CLAMP> __global__ __launch_bounds__(256) void k_bp_gather(BpRefArgs p)
 {
     const int N = p.n, D = p.n_dets;
@@ -450,7 +450,7 @@ template <int R, int CLAMP> __global__ __launch_bounds__(256) void k_bp_gather(B
     }
 }
 
-template <int R> void launch_bp_gather(const BpRefArgs &a, hipStream_t st)
+template <int R> void launch_bp_gather(const BpRefArgs &a, bool unit_lut, hipStream_t st)
 {
     const float half = (float)a.n_dets - a.axis * 2 < 0 ? (float)a.n_dets - a.axis : a.axis;
     const float edge0 = a.axis - half + 0.5f, edge1 = a.axis + half - 0.5f;
@@ -461,7 +461,11 @@ template <int R> void launch_bp_gather(const BpRefArgs &a, hipStream_t st)
     const double reach = 0.7071067811865476 * (a.n - 1) * (1.0 + 1e-5) + 1e-3;
     const bool inside = window && shift - reach > edge0 && shift + reach < edge1;
     const dim3 grid((a.n + 63) / 64, (a.n + 4 * R - 1) / (4 * R));
-    if (inside)
+    // a caller's LUT may hold anything: a pair longer than 1 reaches past the
+    // corners' distance, and a NaN has to stay one (the median drops it)
+    if (!unit_lut)
+        hipLaunchKernelGGL((k_bp_gather<R, 2>), grid, dim3(256), 0, st, a);
+    else if (inside)
         hipLaunchKernelGGL((k_bp_gather<R, 0>), grid, dim3(256), 0, st, a);
     else if (window)
         hipLaunchKernelGGL((k_bp_gather<R, 1>), grid, dim3(256), 0, st, a);
@@ -1175,7 +1179,7 @@ int uirk_sart_ref_step(const float *x_in, float *x_out, const float *b, const fl
 
 int uirk_bp_ref(const float *r_vol, float *w_vol, const float *sino, int n_angles,
                 const float *sin_lut, const float *cos_lut, int n, int n_dets, float axis,
-                float relax, const uirk_runs *runs, const float *pix_w, int posc, void *stream)
+                float relax, const uirk_runs *runs, int unit_lut, const float *pix_w, int posc, void *stream)
 {
     if (n <= 0)
         return 0;
@@ -1198,9 +1202,9 @@ int uirk_bp_ref(const float *r_vol, float *w_vol, const float *sino, int n_angle
     // 180 / 367; at 512 / 400 / 725 both take 46 - 51 us, at 1024 / 720 / 1448
     // two take 197 us and one 269.
     if (n < 512)
-        launch_bp_gather<1>(a, (hipStream_t)stream);
+        launch_bp_gather<1>(a, unit_lut != 0, (hipStream_t)stream);
     else
-        launch_bp_gather<2>(a, (hipStream_t)stream);
+        launch_bp_gather<2>(a, unit_lut != 0, (hipStream_t)stream);
     return (int)hipGetLastError();
 }
 

@@ -596,7 +596,7 @@ uir_status uir_bp_joseph(const float *r_volume, float *w_volume, const float *si
     runs.offset[0] = part.offset;
     runs.n[0] = part.n;
     return uir_check_hip(uirk_bp_ref(r_volume, w_volume, sinogram, (int)dims.n_angles, sin_lut, cos_lut,
-                                     (int)dims.width, (int)dims.n_dets, axis_pos, relax, &runs, NULL, 0,
+                                     (int)dims.width, (int)dims.n_dets, axis_pos, relax, &runs, 0, NULL, 0,
                                      stream), "BP launch");
 }
 

@@ -938,7 +938,7 @@ static uir_status proj_bp_ex(uir_task *p, uint32_t n, const float *sino, float *
         uirk_runs r;
         proj_runs_dev(p, p->runs, p->n_runs, &r, first);
         TRY(uir_check_hip(uirk_bp_ref(vol, vol, sino, (int)p->lut_n, p->d_sin, p->d_cos, (int)n, (int)p->n_dets,
-                                      proj_axis(p), p->relaxation, &r, pix_w, posc, p->res->stream), "BP launch"));
+                                      proj_axis(p), p->relaxation, &r, 1, pix_w, posc, p->res->stream), "BP launch"));
     }
     return UIR_OK;
 }
@@ -1041,7 +1041,7 @@ uir_status uir_parallel_projector_subset_bp(uir_task *p, uir_buffer *volume, con
     proj_runs_dev(p, sub, 1, &r, 0);
     return uir_check_hip(uirk_bp_ref((const float *)volume->data, (float *)volume->data,
                                      (const float *)sinogram->data, (int)p->lut_n, p->d_sin, p->d_cos, (int)n,
-                                     (int)p->n_dets, proj_axis(p), p->relaxation, &r, NULL, 0, p->res->stream),
+                                     (int)p->n_dets, proj_axis(p), p->relaxation, &r, 1, NULL, 0, p->res->stream),
                          "BP launch");
 }
 
