@@ -361,3 +361,36 @@ def test_bp_reads_stay_in_the_staged_window(n, d, a, axis_prop, line):
     assert widest < 100, widest  # the kernel's own footprint check passes
     assert lo >= 0, lo
     assert hi <= 99, hi
+
+
+class Part(C.Structure):
+    _fields_ = [("n_xcd", C.c_int32), ("start", C.c_int32 * 17)]
+
+
+@pytest.mark.parametrize("sizes", [[0], [1], [0, 3, 0, 700], [257, 1, 256]])
+def test_sorted_table_holds_the_same_items_by_falling_cost(sizes):
+    """uirk_plan_sort_fp orders each XCD's range by falling cost (to 1/256 of
+    the range's largest), equal ones in table order, and moves no item to
+    another range."""
+    L = uir.load()
+    n = sum(sizes)
+    rng = np.random.default_rng(n)
+    v = (Item * max(n, 1))()
+    for i in range(n):
+        lo = int(rng.integers(0, 500))
+        v[i] = Item(0, 0, i, int(rng.integers(1, 9)), 0, lo, lo + int(rng.choice([0, 1, 64, rng.integers(0, 3000)])), 0)
+    part = Part(len(sizes), (C.c_int32 * 17)(*np.cumsum([0] + sizes).tolist()))
+
+    def items():
+        return [(it.a0, it.na, it.l_lo, it.l_hi) for it in v[:n]]
+
+    before = items()
+    L.uirk_plan_sort_fp(v, C.byref(part))
+    after = items()
+    for i, k in zip(np.cumsum([0] + sizes), sizes):
+        a, b = before[i:i + k], after[i:i + k]
+        assert sorted(a) == sorted(b)
+        cost = np.array([na * (hi - lo) + 16.0 for _, na, lo, hi in b])  # uirk_fp_item_cost
+        assert not k or np.all(np.diff(cost) <= cost.max() / 256)
+        for j in range(k - 1):
+            assert cost[j] != cost[j + 1] or b[j][0] < b[j + 1][0]

@@ -631,16 +631,14 @@ static uir_status proj_plan(uir_task *p, uint32_t n)
     uir_status s = UIR_OK;
     /* Items of 8 angles where they are at least 12 a CU (2048 / 900 / 2897, 20 a
      * CU: 1114 us against 1208 with 4), else of 4 (1024 / 720 / 1448, 8 a CU: 267
-     * against 278; 777 / 401 / 1099: 110 against 124). */
-    int bad = !trig;
-    for (p->fp_angles = 8; !bad; p->fp_angles = 4) {
-        fv.n = 0;
-        bad = uirk_plan_fp(&fv, 0, (int)n, (int)p->n_dets, axis, p->h_sin, p->h_cos, p->runs, p->n_runs, p->fp_angles,
-                           UIRK_FP_WMAX);
-        if (p->fp_angles == 4 || fv.n >= 3 * (size_t)uirk_plan_device_slots())
-            break;
-    }
-    if (bad) {
+     * against 278; 777 / 401 / 1099: 110 against 124); counted before windows cut
+     * any, so that the table is planned once. */
+    size_t of8 = 0;
+    for (uint32_t i = 0; i < p->n_runs; ++i)
+        of8 += (size_t)((p->runs[i].n + 7) / 8) * ((p->n_dets + UIRK_FP_DETS - 1) / UIRK_FP_DETS);
+    p->fp_angles = of8 >= 3 * (size_t)uirk_plan_device_slots() ? 8 : 4;
+    if (!trig || uirk_plan_fp(&fv, 0, (int)n, (int)p->n_dets, axis, p->h_sin, p->h_cos, p->runs, p->n_runs, p->fp_angles,
+                              UIRK_FP_WMAX)) {
         s = uir_set_error(UIR_ERR_OUT_OF_MEMORY, "work table");
         goto done;
     }
