@@ -102,7 +102,7 @@ def test_batch_slice_pairs_equal_single_slices(res, storage, monkeypatch):
     ("joseph", 49, 800),   # more than 3 a CU: 16 angles; a last slice without a partner
     ("joseph", 66, 528),   # more than 4: 64 rows, 32 angles
     ("joseph", 98, 784),   # more than 3 in 64 rows: 16 angles
-    ("line", 14, 448), ("line", 16, 256), ("line", 66, 528),
+    ("line", 14, 448), ("line", 16, 256), ("line", 17, 288), ("line", 66, 528),
 ])
 def test_batch_bp_shapes_equal_single_slices(res, monkeypatch, model, k, items):
     """Each shape that the rule on the BP's items picks (pairs, tile rows,

@@ -394,3 +394,43 @@ def test_sorted_table_holds_the_same_items_by_falling_cost(sizes):
         assert not k or np.all(np.diff(cost) <= cost.max() / 256)
         for j in range(k - 1):
             assert cost[j] != cost[j + 1] or b[j][0] < b[j + 1][0]
+
+
+class BpChoice(C.Structure):
+    _fields_ = [("pairs", C.c_int), ("rows32", C.c_int), ("angles16", C.c_int)]
+
+
+@pytest.mark.parametrize("line,n,groups,want", [
+    # (slices of each group of one geometry), items a CU of 256: (pairs, rows32, angles16)
+    (0, 1024, [1], (0, 1, 0)), (0, 1024, [2], (0, 1, 0)),
+    (0, 512, [9], (1, 1, 0)),             # 4.5 items, 1.8 slices an item
+    (0, 512, [8], (0, 1, 0)),             # 4: below the line
+    (0, 1024, [6], (1, 0, 0)), (0, 1024, [10], (1, 0, 1)),
+    (0, 512, [5] * 16, (1, 0, 1)),        # 1.67 slices an item
+    (0, 1024, [3] * 10, (0, 0, 0)),       # 1.5
+    (1, 417, [5], (0, 1, 0)),             # 1.9 items a CU
+    (1, 512, [4], (1, 1, 0)),             # 2
+    (1, 417, [3] * 2, (1, 1, 0)), (1, 1024, [3], (1, 1, 0)), (1, 1024, [3] * 10, (1, 0, 0)),  # 1.5 slices an item
+    (1, 640, [3] * 3, (1, 1, 0)), (1, 800, [3] * 2, (1, 0, 0)),  # 4.7 and 5.1 paired items of 32 rows a CU
+    (1, 800, [5], (1, 1, 0)), (1, 1024, [7], (1, 0, 0)),
+    (1, 512, [2, 1, 1] * 8, (1, 0, 0)),   # 1.33, 6 paired items of 64 rows a CU
+    (1, 417, [2, 1, 1] * 3, (0, 1, 0)),   # 1.33, 1.7 (588 unpaired tiles of 64 rows: 32 rows)
+    (1, 1024, [1] * 20, (0, 0, 0)),       # no two slices share
+])
+def test_bp_shape_rule(monkeypatch, line, n, groups, want):
+    """uirk_plan_bp_choose on both sides of its lines (256 CUs), with the
+    items counted by uirk_plan_bp_count; untuned tiles."""
+    monkeypatch.delenv("UIR_PAIR_MIN_ITEMS", raising=False)
+    L = uir.load()
+    if L.uirk_plan_device_slots() != 1024:
+        pytest.skip("items given for 256 CUs")
+    size = C.c_size_t
+    L.uirk_plan_bp_choose.restype = BpChoice
+    L.uirk_plan_bp_choose.argtypes = [size, size, size, size, C.c_int]
+    L.uirk_plan_bp_count.argtypes = [C.c_uint32, C.c_int] + [C.POINTER(size)] * 3
+    n32, p64, p32 = size(0), size(0), size(0)
+    for g in groups:
+        for i in range(g):
+            L.uirk_plan_bp_count(n, i % 2 == 0, C.byref(n32), C.byref(p64), C.byref(p32))
+    c = L.uirk_plan_bp_choose(sum(groups) * ((n + 63) // 64) ** 2, n32, p64, p32, line)
+    assert (c.pairs, c.rows32, c.angles16) == want

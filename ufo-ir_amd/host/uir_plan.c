@@ -275,25 +275,32 @@ void uirk_plan_bp_count(uint32_t n, int counts_paired, size_t *n32, size_t *p64,
     }
 }
 
-/* A pair's item takes 1.4 times the time of one slice's, so pairs gain even
- * where they leave CUs idle: from more than 4.25 unpaired items a CU in tiles
- * of 32 rows, of which a CU holds 6, on (line model, of which it holds 4: from 2).
- * A CU holds 3 pair items with 32 staged angles and 4
- * with 16 (line model: 4).  The tiles are of 32 rows while the table is
- * resident at once that way, else of 64; 32 angles are staged while the table
- * is resident at once with them (fewer barriers), else 16.  Measured at 400
- * angles (us; before: pairs from 4 items a CU, in the rows of the unpaired
- * table): 12 x 512 173 with pairs of 32 rows, 32 angles, 211 before; 16 x 512
- * 217 with 32 rows, 16 angles, 223 with 64 / 32, 271 before; 6 x 1024 279 with
- * 64 / 32, 319 with 32 / 16, 349 before; 8 x 1024 345 with 64 / 16, 407 with
- * 64 / 32 (4 items a CU, 3 at once), 403 before.  With 4 unpaired items a CU
- * and fewer there is less to gain: 6 x 512 134 against 139 unpaired, 4 x 512
- * 121 against 120, 2 x 1024 139 against 157.  Line model: 9 x 512 247 with
- * pairs of 32 rows, 299 unpaired, 315 with 64; 16 x 512 320 against 351 with
- * 64; 4 x 512 146 against 161 unpaired.  A slice without a partner runs the
- * pair kernel at a pair's cost: with less than 1.65 slices an item none pairs
- * (3 x 1024: 211 unpaired, 216 as pairs; 5 x 1024: 297 and 275), line model
- * 1.8 (5 x 417 / 320: 117 unpaired, 133 as pairs). */
+/* A pair's item takes 1.4 times the time of one slice's (line model: 1.25), so
+ * pairs gain even where they leave CUs idle.  A CU holds 6 unpaired items of 32
+ * rows (line model: 4), 3 pair items with 32 staged angles and 4 with 16 (line
+ * model: 4).  The tiles are of 32 rows while the paired table is resident at
+ * once that way, else of 64; 32 angles are staged while the table is resident at
+ * once with them (fewer barriers), else 16.  A slice without a partner runs the
+ * pair kernel at a pair's cost, so the slices an item holds count as well.
+ *   Joseph: from more than 4.25 unpaired items of 32 rows a CU on, with at least
+ * 1.65 slices an item.  BP in us (f16 sinograms, 200 to 700 angles), unpaired
+ * against pairs: 9 x 512 (4.5 a CU) 91 / 83, 4 x 800 229 / 186, 12 x 512 273 /
+ * 221, 4 x 1024 259 / 209, 12 x 1024 904 / 738; 7 x 640 (1.75 slices an item)
+ * 217 / 211, 5 x 1024 (1.67) 447 / 407, 16 groups of 5 x 512 892 / 840; with 1.5
+ * they come out even (10 groups of 3 x 1024 1288 / 1329, 6 of 3 x 417 157 / 165,
+ * 6 of 3 x 512 144 / 126).  Below the line they lose to about 3 a CU (8 x 300
+ * 76 / 80, 4 x 512 134 / 142, 6 x 512 199 / 202); from 3 to 4 they would mostly
+ * gain (8 x 417 220 / 200, 2 x 1024 163 / 145, 5 x 640 234 / 245), but one or two
+ * slices of 1024 are documented to run unpaired in tiles of 32 rows.
+ *   Line model: from 2 unpaired items a CU on (5 x 417, 1.9: 137 / 155; 16 x 256
+ * 125 / 118, 2 groups of 3 x 417, 2.3: 289 / 261), with at least 1.5 slices an
+ * item (3 x 1024 421 / 359, 5 x 800 555 / 430, 10 groups of 3 x 512 499 / 421; at
+ * worst even: 2 groups of 3 x 640 383 / 387), or 1.25 if the paired table of 64
+ * rows holds 4 items a CU (pairs alternating with two single slices, 1.33: 8 x 4
+ * x 512 597 / 543, 2 x 4 x 1024 697 / 650; 1.25: 5 x 5 x 512 973 / 964, 3 x 5 x 640
+ * 507 / 536; with fewer 1.33 is even or loses: 3 x 4 x 417 170 / 175).  Up to 5 paired
+ * items of 32 rows a CU they keep the 32 rows that the unpaired table would take
+ * (3 groups of 3 x 640, 4.7: 191 against 200 with 64; 2 of 3 x 800, 5.1: 376 / 345). */
 uirk_bp_choice uirk_plan_bp_choose(size_t all, size_t n32, size_t p64, size_t p32, int line)
 {
     const size_t cu = (size_t)uirk_plan_device_slots() / 4;
@@ -305,9 +312,10 @@ uirk_bp_choice uirk_plan_bp_choose(size_t all, size_t n32, size_t p64, size_t p3
         c.pairs = (c.rows32 ? p32 : p64) >= least;
         return c;
     }
-    if (line ? n32 >= 2 * cu && 5 * n32 >= 9 * p32 : 4 * n32 > 17 * cu && 20 * n32 >= 33 * p32) {
+    if (line ? n32 >= 2 * cu && (2 * n32 >= 3 * p32 || (4 * n32 >= 5 * p32 && p64 >= 4 * cu))
+             : 4 * n32 > 17 * cu && 20 * n32 >= 33 * p32) {
         c.pairs = 1;
-        c.rows32 = p32 <= 4 * cu;
+        c.rows32 = p32 <= 4 * cu || (line && all <= 4 * cu && p32 <= 5 * cu);
         c.angles16 = !line && (c.rows32 ? p32 : p64) > 3 * cu;
     }
     return c;
