@@ -80,6 +80,8 @@ def test_sart_bit_exact(res, n, d, a, axis, iters):
     (1, 1, 1, 0.4, -1.0), (2, 3, 2, 1.6, -1.0),
     (200, 283, 7, 1.3, -1.0),    # one angle far from the next, the direction changing at almost every one
     (129, 183, 5, 0.79, -1.0),   # a last block of one line
+    (130, 184, 16, 1.57079633, -1.0), (193, 273, 14, 1.94161104, -1.0),  # turned over at (almost) every step
+    (64, 91, 15, 1.5707, 30.25),
     (130, 140, 6, 0.9, 61.25),   # pixels beyond the detector, inactive detectors
     (320, 320, 9, 0.35, -1.0),
     (64, 91, 6, 0.5, 0.2),       # no active detector

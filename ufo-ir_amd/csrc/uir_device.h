@@ -75,13 +75,14 @@ int uirk_fp_block_starts(const float *sin_lut, const float *cos_lut, int n, int 
  * x_out is not written and the FP is that of x_in).  x_in and x_out are
  * different buffers unless fp_ang < 0, part_in and part_out always.  trans:
  * both buffers hold the transposed image; it has to be set if and only if
- * fp_ang is horizontal (|sin| > |cos|), and may be either without an FP.
+ * fp_ang is horizontal (|sin| > |cos|), and may be either without an FP.  turn:
+ * x_out (not x_in's buffer then) holds it the other way than x_in.
  * starts: uirk_fp_block_starts of the geometry with dir -1, or NULL; sin_h and
  * cos_h: the LUT in host memory; n_xcd: uirk_plan_num_xcd().
  * Bit-identical to uirk_fp_ref and uirk_bp_ref of one angle each. */
 int uirk_sart_ref_step(const float *x_in, float *x_out, const float *b, const float *ray_w, const float *starts,
                        const float *part_in, float *part_out, const float *sin_h, const float *cos_h, int n,
-                       int n_dets, float axis, float corr, float relax, int bp_ang, int fp_ang, int trans,
+                       int n_dets, float axis, float corr, float relax, int bp_ang, int fp_ang, int trans, int turn,
                        int n_xcd, void *stream);
 
 /* Reference-compatible BP (projector-parallel-joseph.cl:158-218) over a list of

@@ -1158,12 +1158,12 @@ typedef struct {
 static int sart_horizontal(const uir_task *p, uint32_t a) { return !(fabsf(p->h_sin[a]) <= fabsf(p->h_cos[a])); }
 
 static uir_status sart_step(mctx *c, const sart_prep *sp, const float *b, const float *x_in, float *x_out, int pi,
-                            int bp, int fp, int trans)
+                            int bp, int fp, int trans, int turn)
 {
     uir_task *p = c->p;
     return uir_check_hip(uirk_sart_ref_step(x_in, x_out, b, sp->ray_w, sp->starts, sp->part[pi], sp->part[!pi], p->h_sin,
                                             p->h_cos, (int)c->n, (int)c->D, sp->axis, p->correction_scale,
-                                            p->relaxation, bp, fp, trans, uirk_plan_num_xcd(), c->st),
+                                            p->relaxation, bp, fp, trans, turn, uirk_plan_num_xcd(), c->st),
                          "SART step launch");
 }
 
@@ -1184,8 +1184,9 @@ static uir_status sart_line_bp(mctx *c, float *x, const float *sino_tmp, uint32_
 
 /* One sweep (:208-220).  Joseph: step a applies the BP of angle a - 1 and sums
  * the FP of angle a, the image going back and forth between two buffers and
- * turned over where the angles' direction changes; a last step applies the BP
- * of the last angle into x. */
+ * turned over by the step before an angle of the other direction (by a launch
+ * of its own before the first BP); a last step applies the BP of the last angle
+ * into x. */
 static uir_status sart_sweep(mctx *c, const sart_prep *sp, const float *b, float *x)
 {
     uir_task *p = c->p;
@@ -1202,25 +1203,23 @@ static uir_status sart_sweep(mctx *c, const sart_prep *sp, const float *b, float
 #define OTHER (cur == sp->t[0] ? sp->t[1] : sp->t[0])
     for (uint32_t a = 0; a < c->A; ++a) {
         const int hor = sart_horizontal(p, a);
-        if (hor != trans) {
+        if (hor != trans) { /* a < 2 */
             float *turned = OTHER;
             HIPTRY(uirk_transpose(cur, turned, (int)c->n, c->st), "transpose");
             cur = turned;
             trans = hor;
         }
         float *next = OTHER;
-        TRY(sart_step(c, sp, b, cur, next, pi, (int)a - 1, (int)a, trans));
-        if (a)
+        const int turn = a > 0 && (a + 1 < c->A ? sart_horizontal(p, a + 1) : 0) != hor;
+        TRY(sart_step(c, sp, b, cur, next, pi, (int)a - 1, (int)a, trans, turn));
+        if (a) {
             cur = next;
+            trans ^= turn;
+        }
         pi = !pi;
     }
-    if (trans) {
-        float *turned = OTHER;
-        HIPTRY(uirk_transpose(cur, turned, (int)c->n, c->st), "transpose");
-        cur = turned;
-    }
 #undef OTHER
-    return sart_step(c, sp, b, cur, x, pi, (int)c->A - 1, -1, 0);
+    return sart_step(c, sp, b, cur, x, pi, (int)c->A - 1, -1, trans, trans);
 }
 
 /* Bytes of the FP block-start table of a geometry; tables above this bound
@@ -1727,11 +1726,11 @@ uir_status uir_task_time_kernels(uir_task *t, const uir_buffer *inputs, uir_buff
             s = uir_check_hip(hipEventRecord(ev[0], c.st), "hipEventRecord");
         if (s == UIR_OK)
             s = c.p->line ? sart_line_fp(&c, x, sp.sino_tmp, sp.ray_w, a)
-                          : sart_step(&c, &sp, b, hor ? sp.t[0] : x, NULL, 0, -1, (int)a, hor);
+                          : sart_step(&c, &sp, b, hor ? sp.t[0] : x, NULL, 0, -1, (int)a, hor, 0);
         if (s == UIR_OK && tm)
             s = uir_check_hip(hipEventRecord(ev[1], c.st), "hipEventRecord");
         if (s == UIR_OK)
-            s = c.p->line ? sart_line_bp(&c, x, sp.sino_tmp, a) : sart_step(&c, &sp, b, x, x, 1, (int)a, -1, 0);
+            s = c.p->line ? sart_line_bp(&c, x, sp.sino_tmp, a) : sart_step(&c, &sp, b, x, x, 1, (int)a, -1, 0, 0);
         if (s == UIR_OK && tm) {
             float f = 0, g = 0;
             s = uir_check_hip(hipEventRecord(ev[2], c.st), "hipEventRecord");
