@@ -427,10 +427,10 @@ def test_bp_shape_rule(monkeypatch, line, n, groups, want):
     size = C.c_size_t
     L.uirk_plan_bp_choose.restype = BpChoice
     L.uirk_plan_bp_choose.argtypes = [size, size, size, size, C.c_int]
-    L.uirk_plan_bp_count.argtypes = [C.c_uint32, C.c_int] + [C.POINTER(size)] * 3
+    L.uirk_plan_bp_count.argtypes = [C.c_uint32, C.c_int, C.c_int] + [C.POINTER(size)] * 3
     n32, p64, p32 = size(0), size(0), size(0)
     for g in groups:
         for i in range(g):
-            L.uirk_plan_bp_count(n, i % 2 == 0, C.byref(n32), C.byref(p64), C.byref(p32))
+            L.uirk_plan_bp_count(n, 64, i % 2 == 0, C.byref(n32), C.byref(p64), C.byref(p32))
     c = L.uirk_plan_bp_choose(sum(groups) * ((n + 63) // 64) ** 2, n32, p64, p32, line)
     assert (c.pairs, c.rows32, c.angles16) == want

@@ -1,4 +1,6 @@
 """Tile-shape cache of the autotuner (host side, no device needed)."""
+import ctypes as C
+
 import pytest
 
 import uir
@@ -29,3 +31,30 @@ def test_only_built_variants_are_accepted(tile):
     with pytest.raises(uir.UirError) as e:
         uir.tune_set(SPEC, "f16", *tile)
     assert e.value.status == 1
+
+
+class _Tile(C.Structure):
+    _fields_ = [(k, C.c_int32) for k in ("fp_angles", "bp_angles", "bp_rows", "fp_single", "bp_tuned")]
+
+
+class _Choice(C.Structure):
+    _fields_ = [(k, C.c_int) for k in ("pairs", "rows32", "angles16")]
+
+
+@pytest.mark.parametrize("tuned", [None, (16, 32, 64), (16, 16, 64), (16, 32, 32)])
+def test_tuned_bp_shape_keeps_its_angles(tuned):
+    """The rule on slice pairs sets the staged angles of an untuned geometry
+    only, also where tuning measured the default shape as the fastest."""
+    L = uir.load()
+    L.uir_tile_for.restype = L.uirk_plan_bp_tile.restype = _Tile
+    L.uirk_plan_bp_tile.argtypes = [_Tile, _Choice, C.c_int]
+    uir.tune_clear()
+    if tuned:
+        uir.tune_set(SPEC, "f16", *tuned)
+    spec = uir.slice_spec(SPEC)
+    tile = L.uir_tile_for(C.byref(spec), uir.DTYPE_F16)
+    got = L.uirk_plan_bp_tile(tile, _Choice(1, 0, 1), 0)
+    assert (got.bp_angles, got.bp_rows) == (tuned[1:] if tuned else (16, 64))
+    got = L.uirk_plan_bp_tile(tile, _Choice(1, 1, 0), 0)
+    assert (got.bp_angles, got.bp_rows) == (tuned[1] if tuned else 32, 32)
+    uir.tune_clear()

@@ -235,8 +235,9 @@ typedef struct {
      * 1 = single values (k_fp_tab, windows up to UIRK_FP_WMAX_SINGLE), for
      * geometries whose angle blocks the narrower window would cut short */
     int32_t fp_single;
+    int32_t bp_tuned; /* the BP's shape was measured: it keeps its staged angles */
 } uirk_tile;
-#define UIRK_TILE_DEFAULT {UIRK_FP_ANGLES, 32, UIRK_BP_TILE, 0}
+#define UIRK_TILE_DEFAULT {UIRK_FP_ANGLES, 32, UIRK_BP_TILE, 0, 0}
 /* Footprint width limit of a tile's FP. */
 #define UIRK_TILE_FP_WMAX(t) ((t).fp_single ? UIRK_FP_WMAX_SINGLE : UIRK_FP_WMAX)
 
@@ -313,18 +314,15 @@ typedef struct {
 } uirk_bp_choice;
 /* all: items of every slice of the launch at its tuned rows; n32: items of the
  * model's slices in tiles of 32 rows, unpaired; p64, p32: paired, in tiles of
- * 64 and 32 rows.  The environment variable UIR_PAIR_MIN_ITEMS, when set, is
+ * the tuned rows (64 if untuned) and of 32.  The environment variable UIR_PAIR_MIN_ITEMS, when set, is
  * the least paired table instead (0: pair whenever two slices of one geometry
  * are adjacent) and the largest one that takes 32 rows. */
 uirk_bp_choice uirk_plan_bp_choose(size_t all, size_t n32, size_t p64, size_t p32, int line);
-/* Adds the items of one n x n slice to *n32, and to *p64, *p32 if it leads a
- * pair or has no partner (counts_paired). */
-void uirk_plan_bp_count(uint32_t n, int counts_paired, size_t *n32, size_t *p64, size_t *p32);
+/* Adds the items of one n x n slice, tuned to `rows`, to *n32, and to *p64,
+ * *p32 if it leads a pair or has no partner (counts_paired). */
+void uirk_plan_bp_count(uint32_t n, int rows, int counts_paired, size_t *n32, size_t *p64, size_t *p32);
 /* A geometry's BP tile under the choice: a tuned tile keeps its angles. */
 uirk_tile uirk_plan_bp_tile(uirk_tile t, uirk_bp_choice c, int line);
-/* The least paired table the tuner probes with slice pairs (a full device, or
- * UIR_PAIR_MIN_ITEMS). */
-int uirk_plan_pair_min_items(void);
 /* FP32 <-> storage conversions */
 int uirk_convert(const void *src, int src_dtype, void *dst, int dst_dtype, size_t n, void *stream);
 

@@ -366,7 +366,7 @@ uir_status uir_batch_new(uir_resources *res, uir_dtype storage, const uir_slice_
             const int rows = G->model ? UIRK_BP_TILE : G->tile.bp_rows, second = i > 0 && lead[i - 1];
             all += (size_t)((G->n + UIRK_BP_TILE - 1) / UIRK_BP_TILE) * ((G->n + rows - 1) / rows);
             lead[i] = !second && i + 1 < n_slices && b->geom_of[i + 1] == b->geom_of[i];
-            uirk_plan_bp_count(G->n, !second, &n32[G->model != 0], &p64[G->model != 0], &p32[G->model != 0]);
+            uirk_plan_bp_count(G->n, rows, !second, &n32[G->model != 0], &p64[G->model != 0], &p32[G->model != 0]);
         }
         for (int m = 0; m < 2; ++m)
             bpc[m] = uirk_plan_bp_choose(all, n32[m], p64[m], p32[m], m);

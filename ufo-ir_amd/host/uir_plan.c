@@ -257,20 +257,12 @@ int uirk_plan_device_slots(void)
     return n;
 }
 
-int uirk_plan_pair_min_items(void)
-{
-    const char *env = getenv("UIR_PAIR_MIN_ITEMS"); /* override: 0 pairs always */
-    if (env && *env)
-        return atoi(env);
-    return uirk_plan_device_slots();
-}
-
-void uirk_plan_bp_count(uint32_t n, int counts_paired, size_t *n32, size_t *p64, size_t *p32)
+void uirk_plan_bp_count(uint32_t n, int rows, int counts_paired, size_t *n32, size_t *p64, size_t *p32)
 {
     const size_t w = (n + UIRK_BP_TILE - 1) / UIRK_BP_TILE, h32 = (n + 31) / 32;
     *n32 += w * h32;
     if (counts_paired) {
-        *p64 += w * w;
+        *p64 += w * ((n + (uint32_t)rows - 1) / (uint32_t)rows);
         *p32 += w * h32;
     }
 }
@@ -305,7 +297,7 @@ uirk_bp_choice uirk_plan_bp_choose(size_t all, size_t n32, size_t p64, size_t p3
 {
     const size_t cu = (size_t)uirk_plan_device_slots() / 4;
     uirk_bp_choice c = {0, all <= 4 * cu, 0};
-    const char *env = getenv("UIR_PAIR_MIN_ITEMS");
+    const char *env = getenv("UIR_PAIR_MIN_ITEMS"); /* override: 0 pairs always */
     if (env && *env) {
         const size_t least = (size_t)atoi(env);
         c.rows32 = all <= least;
@@ -326,7 +318,7 @@ uirk_tile uirk_plan_bp_tile(uirk_tile t, uirk_bp_choice c, int line)
     const uirk_tile def = UIRK_TILE_DEFAULT;
     if (line)
         t = def;
-    if (c.angles16 && t.bp_angles == def.bp_angles && t.bp_rows == def.bp_rows)
+    if (c.angles16 && !t.bp_tuned)
         t.bp_angles = 16;
     if (c.rows32)
         t.bp_rows = 32;

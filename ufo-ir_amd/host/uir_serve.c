@@ -624,7 +624,7 @@ static uir_status tables_build(uir_server *s)
             for (uint32_t j = 0; j < i; ++j)
                 second ^= s->active[j]->g == g;
             bp_items += g->n_bp;
-            uirk_plan_bp_count(g->n, !second, &n32[g->model != 0], &p64[g->model != 0], &p32[g->model != 0]);
+            uirk_plan_bp_count(g->n, g->tile.bp_rows, !second, &n32[g->model != 0], &p64[g->model != 0], &p32[g->model != 0]);
         }
         for (int m = 0; m < 2; ++m)
             bpc[m] = uirk_plan_bp_choose(bp_items, n32[m], p64[m], p32[m], m);

@@ -690,7 +690,7 @@ done:
 /* BP tiles of the task path's line mode: 64 x 32 pixels, twice as many
  * workgroups as 64 x 64 tiles (one slice per launch leaves few). */
 #define LINE_BP_ROWS 32
-static const uirk_tile g_line_tile = {UIRK_FP_ANGLES, 32, LINE_BP_ROWS, 0};
+static const uirk_tile g_line_tile = {UIRK_FP_ANGLES, 32, LINE_BP_ROWS, 0, 0};
 
 static uir_status line_plan(uir_task *p, uint32_t n)
 {

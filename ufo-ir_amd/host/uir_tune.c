@@ -61,7 +61,7 @@ uir_status uir_tune_set(const uir_slice_spec *spec, uir_dtype storage, const uir
 {
     if (!spec || !tile)
         return uir_set_error(UIR_ERR_INVALID_ARGUMENT, "NULL argument");
-    const uirk_tile t = {tile->fp_angles, tile->bp_angles, tile->bp_rows, 0};
+    const uir_tile t = *tile;
     if (!((t.fp_angles == 16 || t.fp_angles == 8 || t.fp_angles == 32) && (t.bp_angles == 32 || t.bp_angles == 16) &&
           (t.bp_rows == 64 || t.bp_rows == 32)))
         return uir_set_error(UIR_ERR_INVALID_ARGUMENT, "tile %d/%d/%d is not a variant", t.fp_angles, t.bp_angles,
@@ -115,8 +115,8 @@ int uir_fp_single_for(const uir_slice_spec *spec)
 uirk_tile uir_tile_for(const uir_slice_spec *spec, uir_dtype storage)
 {
     uir_tile t;
-    (void)uir_tune_get(spec, storage, &t);
-    const uirk_tile k = {t.fp_angles, t.bp_angles, t.bp_rows, uir_fp_single_for(spec)};
+    const int tuned = uir_tune_get(spec, storage, &t) == UIR_OK;
+    const uirk_tile k = {t.fp_angles, t.bp_angles, t.bp_rows, uir_fp_single_for(spec), tuned};
     return k;
 }
 
@@ -244,7 +244,7 @@ uir_status uir_tune_run(void *stream, const uir_slice_spec *spec, uir_dtype stor
     float best_fp = 3.0e38f, best_bp = 3.0e38f;
     out->best = (uir_tile){UIRK_FP_ANGLES, 32, UIRK_BP_TILE};
     for (int v = 0; v < 3 && s == UIR_OK; ++v) {
-        const uirk_tile tl = {k_fp_variants[v].fp_angles, 32, UIRK_BP_TILE, uir_fp_single_for(spec)};
+        const uirk_tile tl = {k_fp_variants[v].fp_angles, 32, UIRK_BP_TILE, uir_fp_single_for(spec), 0};
         uirk_fp_vec fv = {0};
         for (uint32_t i = 0; i < B && s == UIR_OK; ++i)
             if (uirk_plan_fp(&fv, (int)i, (int)n, (int)D, axis, h_sin, h_cos, runs, n_runs, tl.fp_angles,
@@ -274,13 +274,19 @@ uir_status uir_tune_run(void *stream, const uir_slice_spec *spec, uir_dtype stor
         }
         free(fv.v);
     }
+    /* every BP variant in slice pairs if a batch of the probe's slices, untuned,
+     * would pair them, else in none */
+    int pairs = 0;
+    {
+        size_t n32 = 0, p64 = 0, p32 = 0;
+        for (uint32_t i = 0; i < B; ++i)
+            uirk_plan_bp_count(n, UIRK_BP_TILE, i % 2 == 0, &n32, &p64, &p32);
+        const size_t w = (n + UIRK_BP_TILE - 1) / UIRK_BP_TILE;
+        pairs = B > 1 && uirk_plan_bp_choose(B * w * w, n32, p64, p32, 0).pairs;
+    }
     for (int v = 0; v < 4 && s == UIR_OK; ++v) {
-        const uirk_tile tl = {UIRK_FP_ANGLES, k_bp_variants[v].bp_angles, k_bp_variants[v].bp_rows, 0};
+        const uirk_tile tl = {UIRK_FP_ANGLES, k_bp_variants[v].bp_angles, k_bp_variants[v].bp_rows, 0, 0};
         uirk_bp_vec bv = {0};
-        /* slice pairs where a batch would use them: the paired table of the
-         * probe fills the device */
-        const size_t tiles = (size_t)((n + UIRK_BP_TILE - 1) / UIRK_BP_TILE) * ((n + tl.bp_rows - 1) / tl.bp_rows);
-        const int pairs = B > 1 && (B + 1) / 2 * tiles >= (size_t)uirk_plan_pair_min_items();
         for (uint32_t i = 0; i < B && s == UIR_OK; i += pairs ? 2 : 1) {
             const size_t b0 = bv.n;
             if (uirk_plan_bp(&bv, (int)i, (int)n, tl.bp_rows))
