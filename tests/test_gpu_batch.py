@@ -135,12 +135,12 @@ def test_batch_bp_shapes_equal_single_slices(res, monkeypatch, model, k, items):
 
 
 def test_batch_pairs_slices_by_default_only_at_scale(res, monkeypatch):
-    """With the default threshold (4 workgroups per CU), a BP table that
-    would hold no more items than that takes tiles of 32 rows instead of 64,
-    and BP slice pairs are used only while the paired table keeps at least
-    that many: ten 1024 x 1024 slices of one geometry pair up on 64-row tiles
-    (half the BP items), one or two take 32-row tiles unpaired.  The results
-    equal the single-slice ones bit for bit."""
+    """BP slice pairs are used from more than 4.25 unpaired items of 32 rows a CU
+    and 1.65 slices an item on, in tiles of 32 rows while the paired table holds
+    at most 4 items a CU; an unpaired table of at most 4 items of 64 rows a CU
+    takes 32 rows too.  Four, six and ten 1024 x 1024 slices of one geometry pair
+    up, on 32, 64 and 64 rows, three are too few an item, one or two take 32-row
+    tiles unpaired.  The results equal the single-slice ones bit for bit."""
     monkeypatch.delenv("UIR_PAIR_MIN_ITEMS", raising=False)
     n, d, a, iters = 1024, 1448, 90, 2
     spec = dict(n=n, n_dets=d, n_angles=a, step=float(np.float32(np.pi / a)), relaxation=0.5)
@@ -150,10 +150,11 @@ def test_batch_pairs_slices_by_default_only_at_scale(res, monkeypatch):
     fill = 4 * uir.probe_ceilings(res)["n_cu"]
     tiles = (n // 64) ** 2  # 64 x 64 tiles of one slice (the untuned BP tile)
 
-    def expected(k):  # BP items of k slices: the two rules
-        per = 2 * tiles if k * tiles <= fill else tiles
-        paired = (k // 2 + k % 2) * per
-        return paired if paired >= fill else k * per
+    def expected(k):  # BP items of k slices
+        items = (k + 1) // 2  # paired, in tiles
+        if 4 * k * 2 * tiles > 17 * (fill // 4) and 20 * k >= 33 * items:
+            return items * (2 * tiles if items * 2 * tiles <= fill else tiles)
+        return k * (2 * tiles if k * tiles <= fill else tiles)
 
     solo = uir.Batch(res, [spec], "f16-sino")
     big = uir.Batch(res, [spec] * 10, "f16-sino")
@@ -163,6 +164,10 @@ def test_batch_pairs_slices_by_default_only_at_scale(res, monkeypatch):
     assert big.info()["bp_items"] == expected(10) == 5 * tiles
     assert small.info()["bp_items"] == expected(2) == 4 * tiles
     small.close()
+    for k, items in ((3, 6 * tiles), (4, 4 * tiles), (6, 3 * tiles)):
+        mid = uir.Batch(res, [spec] * k, "f16-sino")
+        assert mid.info()["bp_items"] == expected(k) == items
+        mid.close()
     for i, b in enumerate(sinos):
         big.set_sinogram(i, b)
     big.reset()

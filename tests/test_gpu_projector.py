@@ -107,12 +107,13 @@ def test_bp_bit_exact(res, n, d, a, axis):
     assert np.array_equal(out.numpy(), O.bp(g, sino))
 
 
-@pytest.mark.parametrize("n", [96, 700])
-def test_forward_again_and_with_another_step(res, n):
+@pytest.mark.parametrize("n,a", [(96, 20), (700, 20), (300, 301)])
+def test_forward_again_and_with_another_step(res, n, a):
     """A forward projector keeps its tables between calls and takes a changed
-    step property at the next one, on both sides of the work table's line."""
-    print("case forward, changed step", n, flush=True)
-    d, a = n, 20
+    step property at the next one, on both sides of the work table's line
+    (90000 rays)."""
+    print("case forward, changed step", n, a, flush=True)
+    d = n
     x = ellipse_phantom(n, seed=n)
     steps = [np.float32(np.pi / a), np.float32(np.pi / a), np.float32(0.1)]
     p = _projector(n, d, a, steps[0], True).setup(res)
@@ -121,6 +122,25 @@ def test_forward_again_and_with_another_step(res, n):
         p["step"] = float(step)
         p.process(dx, ds)
         assert np.array_equal(ds.numpy(), O.fp(O.Geometry(n, d, a, step), x))
+
+
+@pytest.mark.parametrize("forward", [True, False])
+def test_lut_of_an_input_as_high_as_the_angle_count_stays(res, forward):
+    """The LUT is rebuilt when the angle count differs from the input's height
+    (ufo-ir-parallel-projector-task.c:305-347): a projector whose input is as
+    high as its angle count keeps the angles of its first call."""
+    n, a = 96, 96
+    print("case kept LUT", forward, flush=True)
+    first, later = np.float32(np.pi / a), np.float32(0.1)
+    g = O.Geometry(n, n, a, first)
+    x = np.random.default_rng(8).random((n, n)).astype(np.float32)
+    p = _projector(n, n, a, first, forward).setup(res)
+    dx, out = uir.DeviceArray.from_numpy(x), uir.DeviceArray((n, n))
+    for step in (first, later):
+        p["step"] = float(step)
+        assert p.requisition(dx) == (n, n)
+        p.process(dx, out)
+        assert np.array_equal(out.numpy(), O.fp(g, x) if forward else O.bp(g, x))
 
 
 def test_luts_and_runs_match_oracle(res):

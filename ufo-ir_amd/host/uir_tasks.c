@@ -554,8 +554,10 @@ static uir_status proj_requisition(uir_task *p, const uir_buffer *in, uir_requis
         return uir_set_error(UIR_ERR_INVALID_ARGUMENT, "empty input buffer");
     if (p->angles_num == 0)
         p->angles_num = in->dims[1];
-    /* a forward projector's input is the image, whose height is not the angle
-     * count: its LUT is rebuilt only for another count or step */
+    /* As in the reference, the LUT follows a changed step where the input's height
+     * is not the angle count (a forward projector's image, mostly) and stays as it
+     * is where it is.  The reference rebuilds it at every such call, here only for
+     * another count or step. */
     if (p->first_run || p->lut_n != p->angles_num || (p->angles_num != in->dims[1] && p->lut_step != p->step)) {
         p->first_run = 0;
         TRY(proj_build_luts(p, p->angles_num));
