@@ -95,6 +95,23 @@ def test_batch_slice_pairs_equal_single_slices(res, storage, monkeypatch):
         assert np.array_equal(bt.image(i), solo.image(0)), (i, c)
 
 
+@pytest.mark.parametrize("n,d,a,step", [(50, 71, 8, 1.94161104), (31, 44, 1, 0.5), (25, 45, 5, 0.0), (57, 85, 3, 1.6)])
+@pytest.mark.parametrize("model", ["joseph", "line"])
+def test_batch_small_slices_with_a_lone_angle_0(res, n, d, a, step, model):
+    """A direction run of angle 0 alone over an image smaller than a detector
+    block: the block's outer rays pass it on both sides, its inner ones do not."""
+    print("case lone angle 0", n, d, a, step, model, flush=True)
+    step = np.float32(step)
+    g = O.Geometry(n, d, a, step, model=model)
+    b = np.random.default_rng(n).random((a, d)).astype(np.float32)
+    bt = uir.Batch(res, [dict(n=n, n_dets=d, n_angles=a, step=float(step), relaxation=0.5, ray_weight_min=0.1,
+                              model=model)], "f32")
+    bt.set_sinogram(0, b)
+    bt.reset()
+    bt.iterate(3)
+    assert O.rel_l2(bt.image(0), O.sirt64(g, b.astype(np.float64), 3, 0.5, ray_weight_min=0.1)) <= 2e-5
+
+
 @pytest.mark.parametrize("model,k,items", [
     # items of 250 x 250 slices: 16 tiles of 64 rows, 32 of 32; per CU of 256
     ("joseph", 34, 1088),  # 4.25 items a CU: unpaired, 64 rows would be 544

@@ -96,6 +96,8 @@ GEOMS = [  # (n, n_dets, n_angles, step scale, axis property)
     (192, 272, 180, 1.0, 140.5),   # axis shifted right of the detector centre
     (192, 272, 180, 1.0, 128.0),   # and left
     (200, 283, 17, 0.37, -1.0),    # angles over part of [0, pi)
+    # a run of angle 0 alone, whose first detector block reaches past the image both ways
+    (50, 71, 8, 1.94161104 * 8 / np.pi, -1.0), (31, 44, 3, 0.0, -1.0), (57, 85, 1, 1.0, 40.75),
 ]
 
 

@@ -101,17 +101,19 @@ static void line_range(int n, int n_dets, double axis, const ray_step *ray, int 
     for (int a = 0; a < k; ++a) {
         const double det_step = ray[a].det, step = ray[a].line;
         const int ds[2] = {d0, d1};
+        double p0[2];
+        for (int i = 0; i < 2; ++i)
+            p0[i] = ((double)ds[i] + 0.5 - axis) * det_step - 0.5 * n * step + 0.5 * n + shift * step;
         for (int i = 0; i < 2; ++i) {
-            const double p0 = ((double)ds[i] + 0.5 - axis) * det_step - 0.5 * n * step + 0.5 * n + shift * step;
             double l_a, l_b;
-            if (fabs(step) < 1e-12) {
-                if (p0 < plo || p0 > phi)
+            if (fabs(step) < 1e-12) { /* the rays keep their positions: every line if one between the extremes is inside */
+                if (fmax(p0[0], p0[1]) < plo || fmin(p0[0], p0[1]) > phi)
                     continue;
                 l_a = 0;
                 l_b = n;
             } else {
-                l_a = (plo - p0) / step;
-                l_b = (phi - p0) / step;
+                l_a = (plo - p0[i]) / step;
+                l_b = (phi - p0[i]) / step;
                 if (l_a > l_b) {
                     const double t = l_a;
                     l_a = l_b;
