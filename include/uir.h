@@ -334,10 +334,12 @@ uir_status uir_batch_asdpocs_diagnostics(uir_batch *batch, uint32_t slice, float
 /* storage dtype; batches and the server then plan each geometry's work with */
 /* its tuned shape (the default 16 / 32 / 64 when untuned).  Variants apply  */
 /* the same arithmetic.  The BP's shape does not change any bit: a pixel's   */
-/* window and coordinates are those of its 64 x 64 tile, and a batch or      */
-/* server step whose BP table would not fill the device (4 work-groups per   */
-/* CU) takes tiles of 32 rows whatever the tuned rows.  The FP's ray         */
-/* coordinates are anchored per work item, so FP variants agree to FP32      */
+/* window and coordinates are those of its 64 x 64 tile.  A batch or server  */
+/* step takes tiles of 32 rows whatever the tuned rows where its BP table    */
+/* holds at most 4 work-groups per CU: at the tuned rows if its slices do    */
+/* not pair, in tiles of 32 rows if they do; and slice pairs of an untuned   */
+/* geometry stage 16 angles where their table exceeds 3 per CU.  The FP's    */
+/* ray coordinates are anchored per work item, so FP variants agree to FP32  */
 /* rounding.                                                                  */
 /* ------------------------------------------------------------------------ */
 typedef struct {

@@ -61,8 +61,8 @@ def test_sart(res, n, d, a, iters, relax):
     (64, 91, 24, -1.0, 4),
 ])
 def test_sart_bit_exact(res, n, d, a, axis, iters):
-    """The SART sweep's single-angle kernels (wave-per-ray FP from the block
-    start table, four-pixel BP) run the reference's operations in its order:
+    """The SART sweep's step (one angle's BP and the next one's FP, block sums
+    from the block start table) runs the reference's operations in its order:
     the task equals the oracle bit for bit."""
     print("case sart bit-exact", n, d, a, axis, flush=True)
     step = np.float32(np.pi / a)

@@ -175,7 +175,8 @@ __global__ __launch_bounds__(256) void k_fp_ref(FpRefArgs p)
 // replaying the reference's float additions (no memory traffic), so every
 // sample sees the coordinate the sequential walk would see.  The block sums
 // meet in LDS and are added in block order, as the reference adds them.
-// Used where few rays are projected at once (one angle per launch in SART).
+// Used where few rays are projected at once (kernel-level subsets of up to 4
+// angles).
 constexpr int kSplitRays = 16, kSplitSlots = 16, kMaxBlocks = 16384 / kBlockSamples;
 
 __global__ __launch_bounds__(256) void k_fp_ref_split(FpRefArgs p)
@@ -227,7 +228,7 @@ __global__ __launch_bounds__(256) void k_fp_ref_split(FpRefArgs p)
 // (FP_vert) or of the transposed image (FP_hor), so that the 64 rays' taps are
 // neighbours on one line and the line's ends read as zero.  The block sums
 // meet in LDS and are added in block order.  For images whose LDS-staged work
-// table (k_fp_tab) would leave most of the chip idle.
+// table (k_fp_ref_tab) would leave most of the chip idle.
 constexpr int kBlkWaves = 16;
 
 // kFpBatch samples (or n of them) of a block from line l on, added in order.
@@ -486,10 +487,11 @@ template <int R> void launch_bp_gather(const BpRefArgs &a, bool unit_lut, hipStr
 // it forms on the fly from x_in, and many short waves of little code do it.
 // Two kinds of workgroups share the launch and nothing else:
 //   FP: 64 detectors (lanes) x one 64-sample block, kSeg samples to each wave.
-//       A wave replays at most 60 additions of the step from the block's start, its taps are neighbours on a line, and every tap gets
-//       its BP update by the operations the BP workgroups use; the samples
-//       meet in LDS and one wave adds them in order (:82-90).  The block sum
-//       goes to part_out[block][detector].
+//       A wave replays at most 56 additions of the step from the block's start,
+//       its taps are neighbours on a line, and every tap gets its BP update by
+//       the operations the BP workgroups use; the samples meet in LDS and one
+//       wave adds them in order (:82-90).  The block sum goes to
+//       part_out[block][detector].
 //   BP: a tile of 64 x 64 pixels, kSeg per thread, x_out = x_in + relax BP (:196-216).
 // Both first form the residuals of the bins they need in LDS: the previous
 // launch's block sums added in block order, then (b + corr sum) R (:89-94).
@@ -517,7 +519,7 @@ struct SartStepArgs {
     const float *part_in;
     float *part_out;         // [block][detector]
     int n, n_dets;
-    int bp, trans;           // bp: apply the BP; trans: the buffers hold the transposed image
+    int bp;                  // apply the BP
     int n_fp, n_bp;          // FP and BP workgroups per band of 64 lines
     int n_xcd;
     float axis, corr, relax;
@@ -1162,7 +1164,6 @@ int uirk_sart_ref_step(const float *x_in, float *x_out, const float *b, const fl
     a.n = n;
     a.n_dets = n_dets;
     a.bp = bp_ang >= 0;
-    a.trans = trans;
     a.n_bp = bp_ang >= 0 ? nt : 0;
     a.n_xcd = n_xcd > 0 ? n_xcd : 1;
     a.axis = axis;
