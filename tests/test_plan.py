@@ -402,6 +402,26 @@ class BpChoice(C.Structure):
     _fields_ = [("pairs", C.c_int), ("rows32", C.c_int), ("angles16", C.c_int)]
 
 
+class BpCounts(C.Structure):
+    _fields_ = [("all", C.c_size_t)] + [(k, C.c_size_t * 2) for k in ("n32", "p64", "p32")] + \
+               [(k, C.c_uint64 * 2) for k in ("n32_angles", "p32_angles")] + \
+               [(k, C.c_uint32 * 2) for k in ("a_min", "a_max")]
+
+
+def _bp_choice(groups, line, half=0):
+    """The rule's choice for groups (edge, angles, slices) of one geometry each."""
+    L = uir.load()
+    if L.uirk_plan_device_slots() != 1024:
+        pytest.skip("items given for 256 CUs")
+    L.uirk_plan_bp_choose.restype = BpChoice
+    counts = BpCounts()
+    for n, a, k in groups:
+        for i in range(k):
+            L.uirk_plan_bp_count(C.byref(counts), n, a, 64, line, int(i % 2 == 0))
+    c = L.uirk_plan_bp_choose(C.byref(counts), line, half)
+    return c.pairs, c.rows32, c.angles16
+
+
 @pytest.mark.parametrize("line,n,groups,want", [
     # (slices of each group of one geometry), items a CU of 256: (pairs, rows32, angles16)
     (0, 1024, [1], (0, 1, 0)), (0, 1024, [2], (0, 1, 0)),
@@ -420,19 +440,27 @@ class BpChoice(C.Structure):
     (1, 1024, [1] * 20, (0, 0, 0)),       # no two slices share
 ])
 def test_bp_shape_rule(monkeypatch, line, n, groups, want):
-    """uirk_plan_bp_choose on both sides of its lines (256 CUs), with the
-    items counted by uirk_plan_bp_count; untuned tiles."""
+    """uirk_plan_bp_choose on both sides of its lines (256 CUs), for untuned
+    slices of one edge and angle count; counts past 32 bits change nothing."""
     monkeypatch.delenv("UIR_PAIR_MIN_ITEMS", raising=False)
-    L = uir.load()
-    if L.uirk_plan_device_slots() != 1024:
-        pytest.skip("items given for 256 CUs")
-    size = C.c_size_t
-    L.uirk_plan_bp_choose.restype = BpChoice
-    L.uirk_plan_bp_choose.argtypes = [size, size, size, size, C.c_int]
-    L.uirk_plan_bp_count.argtypes = [C.c_uint32, C.c_int, C.c_int] + [C.POINTER(size)] * 3
-    n32, p64, p32 = size(0), size(0), size(0)
-    for g in groups:
-        for i in range(g):
-            L.uirk_plan_bp_count(n, 64, i % 2 == 0, C.byref(n32), C.byref(p64), C.byref(p32))
-    c = L.uirk_plan_bp_choose(sum(groups) * ((n + 63) // 64) ** 2, n32, p64, p32, line)
-    assert (c.pairs, c.rows32, c.angles16) == want
+    for angles in (1, 400, 2 ** 31):
+        assert _bp_choice([(n, angles, k) for k in groups], line) == want, angles
+
+
+@pytest.mark.parametrize("line,half,groups,want", [
+    (0, 1, [(1024, 400, 3)] * 10, (1, 0, 1)), (0, 1, [(1024, 400, 2), (1024, 400, 1)] * 5, (1, 0, 1)),  # 16-bit images
+    (0, 1, [(1024, 400, 2), (1024, 400, 1), (1024, 400, 1)] * 5, (0, 0, 0)),
+    # angles that differ: items by their length, 5.1 of 720 angles a CU; 6.3 but 1.5 slices an item; 5.2; 5.7
+    (0, 0, [(256, 90, 1), (640, 720, 6), (128, 400, 5), (200, 720, 3)], (0, 1, 0)),
+    (0, 0, [(1024, 400, 3), (512, 90, 3)], (0, 1, 0)), (0, 0, [(1024, 180, 9), (200, 720, 6)], (0, 0, 0)),
+    (0, 0, [(1024, 180, 10), (200, 720, 6)], (1, 0, 1)),
+    (0, 0, [(1024, 400, 4), (512, 90, 4)], (1, 0, 0)), (0, 0, [(1024, 720, 8), (640, 90, 4)], (1, 0, 1)),
+    (0, 0, [(1024, 400, 8), (1024, 500, 2)], (1, 0, 1)),  # a quarter apart: as equal
+    (1, 0, [(512, 720, 5), (128, 400, 6)], (0, 1, 0)), (1, 0, [(512, 720, 6), (128, 90, 6)], (1, 1, 0)),
+    (1, 0, [(1024, 180, 3), (512, 90, 3)], (1, 1, 0)),
+    (0, 0, [], (0, 1, 0)), (1, 0, [], (0, 1, 0)),
+])
+def test_bp_shape_rule_of_mixed_slices(monkeypatch, line, half, groups, want):
+    """The same for 16-bit images and for slices of unequal angle counts."""
+    monkeypatch.delenv("UIR_PAIR_MIN_ITEMS", raising=False)
+    assert _bp_choice(groups, line, half) == want

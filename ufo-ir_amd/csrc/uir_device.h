@@ -312,15 +312,23 @@ typedef struct {
     int rows32;   /* tiles of 32 rows */
     int angles16; /* 16 angles a staged batch */
 } uirk_bp_choice;
-/* all: items of every slice of the launch at its tuned rows; n32: items of the
- * model's slices in tiles of 32 rows, unpaired; p64, p32: paired, in tiles of
- * the tuned rows (64 if untuned) and of 32.  The environment variable UIR_PAIR_MIN_ITEMS, when set, is
- * the least paired table instead (0: pair whenever two slices of one geometry
- * are adjacent) and the largest one that takes 32 rows. */
-uirk_bp_choice uirk_plan_bp_choose(size_t all, size_t n32, size_t p64, size_t p32, int line);
-/* Adds the items of one n x n slice, tuned to `rows`, to *n32, and to *p64,
- * *p32 if it leads a pair or has no partner (counts_paired). */
-void uirk_plan_bp_count(uint32_t n, int rows, int counts_paired, size_t *n32, size_t *p64, size_t *p32);
+/* What the choice goes by; zero before the first slice.  all: items of every
+ * slice of the launch at its tuned rows.  Per model (1: line): n32: items of its
+ * slices in tiles of 32 rows, unpaired; p64, p32: paired, in tiles of the tuned
+ * rows (64 if untuned) and of 32; n32_angles, p32_angles: the same items times
+ * their angles; a_min, a_max: the fewest and the most angles of a slice. */
+typedef struct {
+    size_t all, n32[2], p64[2], p32[2];
+    uint64_t n32_angles[2], p32_angles[2];
+    uint32_t a_min[2], a_max[2];
+} uirk_bp_counts;
+/* Adds an n x n slice, tuned to `rows`; it adds to the paired counts if it leads
+ * a pair or has no partner (counts_paired). */
+void uirk_plan_bp_count(uirk_bp_counts *c, uint32_t n, uint32_t angles, int rows, int line, int counts_paired);
+/* half_images: images of 16 bits.  The environment variable UIR_PAIR_MIN_ITEMS,
+ * when set, is the least paired table instead (0: pair whenever two slices of
+ * one geometry are adjacent) and the largest one that takes 32 rows. */
+uirk_bp_choice uirk_plan_bp_choose(const uirk_bp_counts *c, int line, int half_images);
 /* A geometry's BP tile under the choice: a tuned tile keeps its angles. */
 uirk_tile uirk_plan_bp_tile(uirk_tile t, uirk_bp_choice c, int line);
 /* FP32 <-> storage conversions */

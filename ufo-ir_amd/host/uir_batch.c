@@ -360,16 +360,16 @@ uir_status uir_batch_new(uir_resources *res, uir_dtype storage, const uir_slice_
      * up in it (modes 3 and 4), per model */
     uirk_bp_choice bpc[2];
     {
-        size_t all = 0, n32[2] = {0, 0}, p64[2] = {0, 0}, p32[2] = {0, 0};
+        uirk_bp_counts counts;
+        memset(&counts, 0, sizeof counts);
         for (uint32_t i = 0; i < n_slices; ++i) {
             const geom_t *G = &b->geoms[b->geom_of[i]];
-            const int rows = G->model ? UIRK_BP_TILE : G->tile.bp_rows, second = i > 0 && lead[i - 1];
-            all += (size_t)((G->n + UIRK_BP_TILE - 1) / UIRK_BP_TILE) * ((G->n + rows - 1) / rows);
+            const int second = i > 0 && lead[i - 1];
             lead[i] = !second && i + 1 < n_slices && b->geom_of[i + 1] == b->geom_of[i];
-            uirk_plan_bp_count(G->n, rows, !second, &n32[G->model != 0], &p64[G->model != 0], &p32[G->model != 0]);
+            uirk_plan_bp_count(&counts, G->n, G->A, G->tile.bp_rows, G->model, !second);
         }
         for (int m = 0; m < 2; ++m)
-            bpc[m] = uirk_plan_bp_choose(all, n32[m], p64[m], p32[m], m);
+            bpc[m] = uirk_plan_bp_choose(&counts, m, b->esi == 2);
         for (uint32_t i = 0; i < n_slices; ++i)
             lead[i] = lead[i] && bpc[b->geoms[b->geom_of[i]].model != 0].pairs;
     }

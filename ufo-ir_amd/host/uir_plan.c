@@ -259,14 +259,21 @@ int uirk_plan_device_slots(void)
     return n;
 }
 
-void uirk_plan_bp_count(uint32_t n, int rows, int counts_paired, size_t *n32, size_t *p64, size_t *p32)
+void uirk_plan_bp_count(uirk_bp_counts *c, uint32_t n, uint32_t angles, int rows, int line, int counts_paired)
 {
+    const int m = line != 0;
     const size_t w = (n + UIRK_BP_TILE - 1) / UIRK_BP_TILE, h32 = (n + 31) / 32;
-    *n32 += w * h32;
+    const size_t tuned = w * ((n + (uint32_t)rows - 1) / (uint32_t)rows);
+    c->all += tuned;
+    c->n32[m] += w * h32;
+    c->n32_angles[m] += (uint64_t)(w * h32) * angles;
     if (counts_paired) {
-        *p64 += w * ((n + (uint32_t)rows - 1) / (uint32_t)rows);
-        *p32 += w * h32;
+        c->p64[m] += tuned;
+        c->p32[m] += w * h32;
+        c->p32_angles[m] += (uint64_t)(w * h32) * angles;
     }
+    c->a_min[m] = c->a_max[m] == 0 || angles < c->a_min[m] ? angles : c->a_min[m];
+    c->a_max[m] = angles > c->a_max[m] ? angles : c->a_max[m];
 }
 
 /* A pair's item takes 1.4 times the time of one slice's (line model: 1.25), so
@@ -275,15 +282,18 @@ void uirk_plan_bp_count(uint32_t n, int rows, int counts_paired, size_t *n32, si
  * model: 4).  The tiles are of 32 rows while the paired table is resident at
  * once that way, else of 64; 32 angles are staged while the table is resident at
  * once with them (fewer barriers), else 16.  A slice without a partner runs the
- * pair kernel at a pair's cost, so the slices an item holds count as well.
+ * pair kernel at a pair's cost, so the slices an item holds count as well.  Items
+ * count by their angles, relative to the longest.
  *   Joseph: from more than 4.25 unpaired items of 32 rows a CU on, with at least
  * 1.65 slices an item.  BP in us (f16 sinograms, 200 to 700 angles), unpaired
  * against pairs: 9 x 512 (4.5 a CU) 91 / 83, 4 x 800 229 / 186, 12 x 512 273 /
  * 221, 4 x 1024 259 / 209, 12 x 1024 904 / 738; 7 x 640 (1.75 slices an item)
  * 217 / 211, 5 x 1024 (1.67) 447 / 407, 16 groups of 5 x 512 892 / 840; with 1.5
  * they come out even (10 groups of 3 x 1024 1288 / 1329, 6 of 3 x 417 157 / 165,
- * 6 of 3 x 512 144 / 126).  Below the line they lose to about 3 a CU (8 x 300
- * 76 / 80, 4 x 512 134 / 142, 6 x 512 199 / 202); from 3 to 4 they would mostly
+ * 6 of 3 x 512 144 / 126).  Images of 16 bits: from 1.5 (3 x 1448 with 90 angles
+ * 126 / 109, 4 groups of 3 x 768 127 / 102, 8 of 3 x 512 102 / 75; with 400 angles
+ * 390 / 403, 387 / 399, 325 / 294).  Below the line they lose to about 3 a CU (8 x
+ * 300 76 / 80, 4 x 512 134 / 142, 6 x 512 199 / 202); from 3 to 4 they would mostly
  * gain (8 x 417 220 / 200, 2 x 1024 163 / 145, 5 x 640 234 / 245), but one or two
  * slices of 1024 are documented to run unpaired in tiles of 32 rows.
  *   Line model: from 2 unpaired items a CU on (5 x 417, 1.9: 137 / 155; 16 x 256
@@ -294,22 +304,36 @@ void uirk_plan_bp_count(uint32_t n, int rows, int counts_paired, size_t *n32, si
  * x 512 597 / 543, 2 x 4 x 1024 697 / 650; 1.25: 5 x 5 x 512 973 / 964, 3 x 5 x 640
  * 507 / 536; with fewer 1.33 is even or loses: 3 x 4 x 417 170 / 175).  Up to 5 paired
  * items of 32 rows a CU they keep the 32 rows that the unpaired table would take
- * (3 groups of 3 x 640, 4.7: 191 against 200 with 64; 2 of 3 x 800, 5.1: 376 / 345). */
-uirk_bp_choice uirk_plan_bp_choose(size_t all, size_t n32, size_t p64, size_t p32, int line)
+ * (3 groups of 3 x 640, 4.7: 191 against 200 with 64; 2 of 3 x 800, 5.1: 376 / 345).
+ *   Slices whose angle counts differ by more than a quarter leave the CUs unevenly
+ * loaded, where fewer and longer items cost more: pairs from 5.5 items a CU on
+ * (line model: 3), 32 rows as in the line model.  Over 365 mixed batches that was
+ * 8 % faster than the build that paired from 4 paired items a CU on, and 1 % than
+ * 4.25 items of whatever length; one in 25 is slower than the better of both by
+ * 5 to 35 % (2 x 1024 of 400 angles beside small slices of 90 to 180: 192 / 131),
+ * as the rule does not look at how the items fall on the CUs.  Line model, 200
+ * batches: 5 and 3 %. */
+uirk_bp_choice uirk_plan_bp_choose(const uirk_bp_counts *n, int line, int half_images)
 {
-    const size_t cu = (size_t)uirk_plan_device_slots() / 4;
-    uirk_bp_choice c = {0, all <= 4 * cu, 0};
+    const int m = line != 0;
+    const size_t cu = (size_t)uirk_plan_device_slots() / 4, p64 = n->p64[m], p32 = n->p32[m];
+    const uint64_t w = n->n32_angles[m], wp = n->p32_angles[m]; /* w / wp: slices an item */
+    const uint64_t full = (uint64_t)cu * n->a_max[m];           /* one of the longest items a CU */
+    const int uneven = 4 * (uint64_t)n->a_max[m] > 5 * (uint64_t)n->a_min[m];
+    uirk_bp_choice c = {0, n->all <= 4 * cu, 0};
     const char *env = getenv("UIR_PAIR_MIN_ITEMS"); /* override: 0 pairs always */
     if (env && *env) {
         const size_t least = (size_t)atoi(env);
-        c.rows32 = all <= least;
+        c.rows32 = n->all <= least;
         c.pairs = (c.rows32 ? p32 : p64) >= least;
         return c;
     }
-    if (line ? n32 >= 2 * cu && (2 * n32 >= 3 * p32 || (4 * n32 >= 5 * p32 && p64 >= 4 * cu))
-             : 4 * n32 > 17 * cu && 20 * n32 >= 33 * p32) {
+    const int enough = line ? w >= (uneven ? 3 : 2) * full : 4 * w > (uneven ? 22 : 17) * full;
+    const int shared = line ? 2 * w >= 3 * wp || (4 * w >= 5 * wp && p64 >= 4 * cu)
+                            : (half_images && !uneven ? 2 * w >= 3 * wp : 20 * w >= 33 * wp);
+    if (n->n32[m] && enough && shared) {
         c.pairs = 1;
-        c.rows32 = p32 <= 4 * cu || (line && all <= 4 * cu && p32 <= 5 * cu);
+        c.rows32 = p32 <= 4 * cu || ((line || uneven) && n->all <= 4 * cu && p32 <= 5 * cu);
         c.angles16 = !line && (c.rows32 ? p32 : p64) > 3 * cu;
     }
     return c;

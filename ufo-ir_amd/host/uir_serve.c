@@ -612,22 +612,22 @@ static int geom_bp_shape(const sgeom *g, const uirk_bp_choice *bpc)
 static uir_status tables_build(uir_server *s)
 {
     const uint32_t na = s->n_active;
-    size_t nf[SRV_FP_SHAPES] = {0}, nb[SRV_BP_SHAPES] = {0}, ncost = 1, bp_items = 0;
+    size_t nf[SRV_FP_SHAPES] = {0}, nb[SRV_BP_SHAPES] = {0}, ncost = 1;
     /* the BP's shapes and pairs per model, from the slices and the pairs that
      * the active requests make when ordered by geometry */
     uirk_bp_choice bpc[2];
     {
-        size_t n32[2] = {0, 0}, p64[2] = {0, 0}, p32[2] = {0, 0};
+        uirk_bp_counts counts;
+        memset(&counts, 0, sizeof counts);
         for (uint32_t i = 0; i < na; ++i) {
             const sgeom *g = s->active[i]->g;
             int second = 0;
             for (uint32_t j = 0; j < i; ++j)
                 second ^= s->active[j]->g == g;
-            bp_items += g->n_bp;
-            uirk_plan_bp_count(g->n, g->tile.bp_rows, !second, &n32[g->model != 0], &p64[g->model != 0], &p32[g->model != 0]);
+            uirk_plan_bp_count(&counts, g->n, g->A, g->tile.bp_rows, g->model, !second);
         }
         for (int m = 0; m < 2; ++m)
-            bpc[m] = uirk_plan_bp_choose(bp_items, n32[m], p64[m], p32[m], m);
+            bpc[m] = uirk_plan_bp_choose(&counts, m, s->esi == 2);
     }
     s->bpg[SRV_BP_LINE].tile.bp_rows = bpc[1].rows32 ? 32 : UIRK_BP_TILE;
     for (uint32_t i = 0; i < na; ++i) {

@@ -278,11 +278,11 @@ uir_status uir_tune_run(void *stream, const uir_slice_spec *spec, uir_dtype stor
      * would pair them, else in none */
     int pairs = 0;
     {
-        size_t n32 = 0, p64 = 0, p32 = 0;
+        uirk_bp_counts counts;
+        memset(&counts, 0, sizeof counts);
         for (uint32_t i = 0; i < B; ++i)
-            uirk_plan_bp_count(n, UIRK_BP_TILE, i % 2 == 0, &n32, &p64, &p32);
-        const size_t w = (n + UIRK_BP_TILE - 1) / UIRK_BP_TILE;
-        pairs = B > 1 && uirk_plan_bp_choose(B * w * w, n32, p64, p32, 0).pairs;
+            uirk_plan_bp_count(&counts, n, A, UIRK_BP_TILE, 0, i % 2 == 0);
+        pairs = B > 1 && uirk_plan_bp_choose(&counts, 0, esi == 2).pairs;
     }
     for (int v = 0; v < 4 && s == UIR_OK; ++v) {
         const uirk_tile tl = {UIRK_FP_ANGLES, k_bp_variants[v].bp_angles, k_bp_variants[v].bp_rows, 0, 0};
