@@ -39,13 +39,14 @@ def test_fp_bp_joseph_per_subset(res, n, a):
 
 
 @pytest.mark.parametrize("n", [200, 513])  # one and two pixels a thread
-@pytest.mark.parametrize("scale", [0.5, 1.0, 1.75, float("nan")])
-def test_bp_joseph_takes_any_lut(res, n, scale):
+@pytest.mark.parametrize("scale", [0.5, 1.0, 1.75, float("nan"), float("inf")])
+@pytest.mark.parametrize("axis", [-1.0, 97.25, 0.2])  # centred; a smaller window; no active detector
+def test_bp_joseph_takes_any_lut(res, n, scale, axis):
     """The caller's LUT need not hold sines and cosines: pairs scaled by a pixel
-    size, and a NaN, give the oracle's image bit for bit."""
-    print("case bp any lut", n, scale, flush=True)
+    size, infinities and NaN give the oracle's image bit for bit."""
+    print("case bp any lut", n, scale, axis, flush=True)
     d, a = int(np.ceil(n * 2 ** 0.5)) + 2, 9
-    g = O.Geometry(n, d, a, np.float32(np.pi / a))
+    g = O.Geometry(n, d, a, np.float32(np.pi / a), axis)
     g.sin[2:] *= np.float32(scale)
     g.cos[2:] *= np.float32(scale)
     rng = np.random.default_rng(n)

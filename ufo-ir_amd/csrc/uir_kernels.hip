@@ -356,7 +356,8 @@ __device__ __forceinline__ int cvt_flr(float x)
 
 // CLAMP 2: any axis and any LUT.  1: 0.5 <= edge0 <= edge1 <= n_dets - 0.5 (an
 // axis with active detectors), so that the clamp is one median and every lower
-// tap lies in the row.  0: no pixel reaches an edge either, no clamp.
+// tap lies in the row.  0: no pixel reaches an edge either, no clamp.  3: as 1
+// for any LUT: a NaN coordinate stays one, which the median would drop.
 template <int R, int CLAMP> __global__ __launch_bounds__(256) void k_bp_gather(BpRefArgs p)
 {
     const int N = p.n, D = p.n_dets;
@@ -404,6 +405,8 @@ template <int R, int CLAMP> __global__ __launch_bounds__(256) void k_bp_gather(B
                     float u = fXc - fY[q] * st + shift;
                     if (CLAMP == 1) {
                         u = __builtin_amdgcn_fmed3f(u, edge0, edge1);
+                    } else if (CLAMP == 3) {
+                        u = u != u ? u : __builtin_amdgcn_fmed3f(u, edge0, edge1);
                     } else if (CLAMP == 2) {
                         if (u > edge1)
                             u = edge1;
@@ -412,9 +415,9 @@ template <int R, int CLAMP> __global__ __launch_bounds__(256) void k_bp_gather(B
                     }
                     const float w = u - 0.5f;
                     const int i0 = cvt_flr(w);
-                    a[e][q] = CLAMP < 2 ? __builtin_amdgcn_fractf(w) : w - floorf(w); // the same for w >= 0
+                    a[e][q] = CLAMP != 2 ? __builtin_amdgcn_fractf(w) : w - floorf(w); // the same for w >= 0
                     t0[e][q] = row_load(r0, i0);
-                    t1[e][q] = CLAMP < 2 ? row_load(r1, i0) : row_load(r0, opaque(i0 + 1));
+                    t1[e][q] = CLAMP != 2 ? row_load(r1, i0) : row_load(r0, opaque(i0 + 1));
                 }
             }
 #pragma unroll
@@ -462,10 +465,10 @@ template <int R> void launch_bp_gather(const BpRefArgs &a, bool unit_lut, hipStr
     const double reach = 0.7071067811865476 * (a.n - 1) * (1.0 + 1e-5) + 1e-3;
     const bool inside = window && shift - reach > edge0 && shift + reach < edge1;
     const dim3 grid((a.n + 63) / 64, (a.n + 4 * R - 1) / (4 * R));
-    // a caller's LUT may hold anything: a pair longer than 1 reaches past the
-    // corners' distance, and a NaN has to stay one (the median drops it)
-    if (!unit_lut)
-        hipLaunchKernelGGL((k_bp_gather<R, 2>), grid, dim3(256), 0, st, a);
+    // a caller's LUT may hold anything, as pairs longer than 1, which reach past
+    // the corners' distance
+    if (!unit_lut && window)
+        hipLaunchKernelGGL((k_bp_gather<R, 3>), grid, dim3(256), 0, st, a);
     else if (inside)
         hipLaunchKernelGGL((k_bp_gather<R, 0>), grid, dim3(256), 0, st, a);
     else if (window)
